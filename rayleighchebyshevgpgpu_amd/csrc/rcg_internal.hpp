@@ -165,6 +165,38 @@ void launch_mixed_combine(int64_t n, double* V, int ld, int nc, const double* um
                           const float* E, hipStream_t st);
 void launch_to_f32(int64_t n, const double* x, float* y, hipStream_t st);
 
+// The whole filter of a small CSR operator in one launch (rcg_small.hip).
+// T = double: x <- P_m x.  T = float: the correction steps 2..m from e0, e1
+// and r with the coefficient rows kap + j*ld, and the recombination
+// v <- vs_end (um[c] v + E_m); e0 and e1 are not written.
+constexpr int64_t kSmallFilterRows = 4096;
+template <typename T>
+struct SmallFilter {
+  int n = 0;
+  const int* rowptr = nullptr;
+  const int* col = nullptr;
+  const T* val = nullptr;  // interleaved (re, im) for complex operators
+  T* x = nullptr;
+  const T* e0 = nullptr;
+  const T* e1 = nullptr;
+  const T* r = nullptr;
+  const T* kap = nullptr;
+  double* v = nullptr;
+  const double* um = nullptr;
+  double vs_end = 0.0;
+  int ld = 0;  // real elements per row
+  int m = 0;
+  T g1 = T(0), g2 = T(0), s_end = T(0);
+};
+// Whether the one-launch filter takes an operator of this size, with cols
+// columns (complex ones count once; c128: the FP64 filter of a complex one)
+// and degree m.
+bool small_filter_fits(int64_t n, int64_t nnz, int64_t max_row, int64_t cols, int64_t m,
+                       bool c128);
+template <typename T>
+void launch_small_filter(const SmallFilter<T>& a, int cols, int64_t max_row, bool cx,
+                         hipStream_t st);
+
 // Dense symmetric operator A (n x n, lda; row-major = column-major): one
 // step on a row-interleaved block, mode as the CSR kernels:
 //   0 apply: out = p0 A X; 1: out = p0 A X + p1 out;

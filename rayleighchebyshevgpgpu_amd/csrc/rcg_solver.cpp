@@ -318,6 +318,7 @@ struct rcg_operator_s {
   const int* col = nullptr;
   const double* val = nullptr;
   DevBuf own_rowptr, own_col, own_val;
+  int64_t max_row = -1;            // nonzeros of the longest row (-1: not looked up yet)
   int64_t gx = 0, gy = 0, gz = 0;  // structured-grid hint (rows x + gx(y + gy z))
   std::vector<std::unique_ptr<SchedCand>> scheds;
   struct Tuned {
@@ -965,6 +966,25 @@ class Engine {
     return &op_->scheds[tuned_for(b).sched]->sc;
   }
 
+  // Whether the filter of b columns runs in one launch (rcg_small.hip).  The
+  // longest row of an operator that lives in the caller's device memory is
+  // looked up once; it steers the choice only, any row length is computed.
+  bool small_filter(int64_t b, long m, bool fp64) {
+    if (batcher_ || !op_->is_csr() || n_ > rcg::kSmallFilterRows) return false;
+    // a forced panel or order asks for the general kernel
+    if (std::getenv("RCG_FILTER_PANEL") || std::getenv("RCG_FILTER_SCHED")) return false;
+    std::lock_guard<std::mutex> lk(op_->lazy_mu);
+    if (op_->max_row < 0) {
+      std::vector<int> rp((size_t)n_ + 1);
+      RCG_HIP(hipMemcpyAsync(rp.data(), op_->rowptr, sizeof(int) * rp.size(),
+                             hipMemcpyDeviceToHost, st_));
+      sync();
+      for (int64_t i = 0; i < n_; ++i)
+        op_->max_row = std::max<int64_t>(op_->max_row, rp[i + 1] - rp[i]);
+    }
+    return rcg::small_filter_fits(n_, op_->nnz, op_->max_row, b, m, cx_ && fp64);
+  }
+
   // V <- P_m(A')^rep V over b columns (LanczosCpolyOperatorLM.h:192-304):
   // X1 = g2(g1 A X0 + X0), Xj = g2(g1 A X_{j-1} + X_{j-1}) - X_{j-2}, out = Xm/(m+1).
   void filter(int64_t b, long m, long rep, double lmax, double shift) {
@@ -973,12 +993,32 @@ class Engine {
     if (batcher_) return filter_batched(b, m, rep, lmax, shift);
     const auto c = rcg::cpoly::coefficients(m, lmax, shift);
     const int64_t rb = cw_ * b;  // real columns
+    const double csr = double(op_->nnz) * (4.0 + 8.0 * cw_) + 4.0 * double(n_ + 1);
+    const double blk = 8.0 * double(n_) * double(rb);
+    if (b > 0 && small_filter(b, m, true)) {
+      last_panel_ = (int)rb;
+      last_sched_ = "one-launch";
+      step_begin(rep, double(rep) * (csr + 2.0 * blk + double(m - 1) * (csr + 3.0 * blk)));
+      rcg::SmallFilter<double> f;
+      f.n = (int)n_;
+      f.rowptr = op_->rowptr;
+      f.col = op_->col;
+      f.val = op_->val;
+      f.x = V();
+      f.ld = (int)ld_;
+      f.m = (int)m;
+      f.g1 = c.g1;
+      f.g2 = c.g2;
+      f.s_end = 1.0 / double(m + 1);
+      for (long r = 0; r < rep; ++r)
+        rcg::launch_small_filter<double>(f, (int)b, op_->max_row, cx_, st_);
+      step_end();
+      return;
+    }
     const auto tn = tuned_for(rb);
     const rcg::CsrSched* sc = &op_->scheds[tn.sched]->sc;
     last_panel_ = tn.panel;
     last_sched_ = op_->scheds[tn.sched]->name;
-    const double csr = double(op_->nnz) * (4.0 + 8.0 * cw_) + 4.0 * double(n_ + 1);
-    const double blk = 8.0 * double(n_) * double(rb);
     step_begin(rep * m * ((rb + tn.panel - 1) / tn.panel),
                double(rep) * (csr + 2.0 * blk + double(m - 1) * (csr + 3.0 * blk)));
     for (long r = 0; r < rep; ++r) {
@@ -1210,6 +1250,8 @@ class Engine {
     // (bit-identical results).
     const char* unf = std::getenv("RCG_MIXED_UNFUSED");
     const bool fused = !dn && !(unf && unf[0] == '1');
+    const bool small = fused && b > 0 && small_filter(b, m, false);
+    if (small) last_sched_ = "one-launch";
     for (long r = 0; r < rep; ++r) {
       if (fused) {
         rcg::MixedArgs ms;
@@ -1245,6 +1287,28 @@ class Engine {
         d.kap = dk;
         batch_submit(d, true, cx_, 2);
         rcg::launch_mixed_combine(n_, V(), (int)ld_, (int)rb, dum, end.s_end, E_[m % 2], st_);
+        continue;
+      }
+      if (small) {
+        rcg::SmallFilter<float> f;
+        f.n = (int)n_;
+        f.rowptr = op_->rowptr;
+        f.col = op_->col;
+        f.val = val32;
+        f.e0 = E_[0];
+        f.e1 = E_[1];
+        f.r = R32_;
+        f.kap = dk;
+        f.v = V();
+        f.um = dum;
+        f.vs_end = end.s_end;
+        f.ld = (int)ld_;
+        f.m = (int)m;
+        f.g1 = g1f;
+        f.g2 = g2f;
+        step_begin(1, double(m - 1) * (csr + 4.0 * blk));
+        rcg::launch_small_filter<float>(f, (int)b, op_->max_row, cx_, st_);
+        step_end();
         continue;
       }
       float* X0 = E_[0];
@@ -1291,7 +1355,10 @@ class Engine {
   // Device time of the Chebyshev step launches (hipEvents around each run
   // of steps), their count and algorithmic bytes; read once the stream has
   // passed the end event.
+  // Solves read them; the piecewise entry points do not and skip the events.
+  void time_steps() { timed_ = true; }
   void step_begin(long launches, double bytes) {
+    if (!timed_) return;
     if (!fev_[0]) {
       RCG_HIP(hipEventCreate(&fev_[0]));
       RCG_HIP(hipEventCreate(&fev_[1]));
@@ -1302,6 +1369,7 @@ class Engine {
     pend_bytes_ = bytes;
   }
   void step_end() {
+    if (!timed_) return;
     RCG_HIP(hipEventRecord(fev_[1], st_));
     step_pending_ = true;
   }
@@ -1861,6 +1929,7 @@ class Engine {
   hipEvent_t fev_[2] = {nullptr, nullptr};
   FilterBatcher* batcher_ = nullptr;
   hipEvent_t ev_done_ = nullptr;  // the batcher has run this engine's steps
+  bool timed_ = false;
   bool step_pending_ = false;
   long pend_launches_ = 0, step_launches_ = 0;
   double pend_bytes_ = 0.0, step_bytes_ = 0.0, step_seconds_ = 0.0;
@@ -1941,6 +2010,7 @@ class Solver {
          FilterBatcher* batcher = nullptr)
       : op_(op), p_(p), eng_(ctx ? ctx : op->ctx, op, op->n), clock_(eng_.stream()) {
     eng_.set_batcher(batcher);
+    eng_.time_steps();
     for (DevBuf* b : {&Vb_, &Tb_, &Wb_, &Yb_, &Mb_}) b->use_stream(eng_.stream());
   }
   Solver(const Solver&) = delete;
@@ -2765,6 +2835,8 @@ int rcg_operator_csr_create(rcg_context ctx, int64_t n, int64_t nnz, const int32
       // validated on the host before anything reaches a kernel
       need(rowptr[0] == 0 && rowptr[n] == nnz, "rowptr must start at 0 and end at nnz");
       for (int64_t i = 0; i < n; ++i) need(rowptr[i] <= rowptr[i + 1], "rowptr must be non-decreasing");
+      for (int64_t i = 0; i < n; ++i)
+        o->max_row = std::max<int64_t>(o->max_row, rowptr[i + 1] - rowptr[i]);
       for (int64_t p = 0; p < nnz; ++p) need(col[p] >= 0 && col[p] < n, "column index out of range");
       o->own_rowptr.ensure(sizeof(int) * (size_t)(n + 1));
       o->own_col.ensure(sizeof(int) * (size_t)std::max<int64_t>(nnz, 1));
@@ -2794,6 +2866,10 @@ int rcg_operator_csr_share(rcg_operator base, const void* val, int mem, rcg_oper
     o->dtype = base->dtype;
     o->rowptr = base->rowptr;
     o->col = base->col;
+    {
+      std::lock_guard<std::mutex> lk(base->lazy_mu);
+      o->max_row = base->max_row;
+    }
     o->gx = base->gx;
     o->gy = base->gy;
     o->gz = base->gz;

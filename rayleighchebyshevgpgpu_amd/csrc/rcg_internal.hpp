@@ -48,6 +48,28 @@ void set_last_error(const std::string& msg);
 // -------------------------------------------------------------- launchers
 // All pointers are device pointers; every launch goes on `st`.
 
+// Tiles of a structured grid for the step that gathers from LDS (rcg_tile.hip):
+// per tile the rows it copies (its own first), where its own rows' nonzeros
+// start in the CSR arrays, and each nonzero's place among the copied rows.
+struct TilePlan {
+  const int* srow = nullptr;
+  const int* pstart = nullptr;
+  const unsigned char* lidx = nullptr;
+  int smax = 0;  // rows copied per tile
+  int64_t ntile = 0;
+};
+struct TileShape {
+  int ex = 0, ey = 0, ez = 0;  // rows of a tile along x, y, z
+  int sy = 0, sz = 0;          // tiles of a bundle along y, z
+  int smax = 0;
+  int64_t ntile = 0;
+  size_t srow = 0, pstart = 0, lidx = 0;  // entries of the plan's arrays
+};
+TileShape tile_shape(int64_t gx, int64_t gy, int64_t gz);
+// *bad (zero before) is set if the operator does not fit the tiles.
+void launch_tile_plan(const TileShape& t, int64_t n, const int* rowptr, const int* col, int64_t gx,
+                      int64_t gy, int64_t gz, int* srow, int* pstart, unsigned char* lidx, int* bad,
+                      hipStream_t st);
 // Order in which the CSR kernels visit row blocks.  The rows computed and
 // their arithmetic do not depend on it; it only changes which rows are in
 // flight together (cache locality).  order == nullptr: contiguous blocks.
@@ -56,6 +78,7 @@ struct CsrSched {
   int64_t rows_per_blk = 0;    // rows per block when `order` is set
   int64_t nblk = 0;            // number of row blocks when `order` is set
   int remap = 1;               // 1: each XCD takes a contiguous range of logical blocks
+  const TilePlan* tile = nullptr;  // steps over tiles gathered from LDS
 };
 
 // ---- batched filter steps over many CSR operators (the serving engine)
@@ -129,6 +152,12 @@ struct MixedArgs {
   const double* um = nullptr;    // u_m(theta_c) per column
   double s_end = 0.0;            // 1 / (m + 1)
 };
+
+// One step (mode: CsrMode) on ncols real columns; false: a mode it does not have.
+template <typename T>
+bool launch_tile_step(const TilePlan& t, int mode, const T* val, const T* X, const T* Z, T* out,
+                      int ld, int ncols, T p0, T p1, T p2, const T* R, const T* kap, bool cx,
+                      const MixedArgs& ms, hipStream_t st);
 
 // Mixed-precision filter.  The FP64 filter output s*X_m of X_0 = v is split
 // per column as X_j = u_j(theta_c) v + E_j, u_j the scalar recurrence of the

@@ -137,6 +137,10 @@ void csr_launch(int64_t n, const int* rp, const int* ci, const T* va, const T* X
                 T* out, int ld, int ncols, T p0, T p1, T p2, hipStream_t st, const CsrSched* sc,
                 const T* R = nullptr, const T* kap = nullptr, bool cx = false,
                 const MixedArgs& ms = MixedArgs{}) {
+  if (sc && sc->tile &&
+      launch_tile_step<T>(*sc->tile, MODE, va, X, Z, out, ld, ncols, p0, p1, p2, R, kap, cx, ms,
+                          st))
+    return;
   if (cx) {
     if (ncols % 2 != 0) throw Error(1, "complex blocks have an even number of real columns");
     csr_launch_cx<T, MODE, true>(n, rp, ci, va, X, Z, out, ld, ncols, p0, p1, p2, st, sc, R, kap, ms);
@@ -1713,7 +1717,7 @@ void launch_cheb_step(int64_t n, const int* rowptr, const int* col, const T* val
   // Column panels: each launch streams the CSR arrays once and touches only
   // `panel` columns of every row, which shrinks the per-plane footprint of
   // the gathered block so that neighbour rows stay in L2 between uses.
-  if (panel <= 0 || panel >= ncols) panel = ncols;
+  if (panel <= 0 || panel >= ncols || (sc && sc->tile)) panel = ncols;
   if (panel % 4 != 0) panel = round_up(panel, 4);
   for (int c0 = 0; c0 < ncols; c0 += panel) {
     const int pc = std::min(panel, ncols - c0);
@@ -1731,7 +1735,7 @@ void launch_cheb_step_src(int64_t n, const int* rowptr, const int* col, const fl
                           const float* kap, int ld, int ncols, float g1, float g2, float s,
                           hipStream_t st, int panel, const CsrSched* sc, bool cx) {
   if (n <= 0 || ncols <= 0) return;
-  if (panel <= 0 || panel >= ncols) panel = ncols;
+  if (panel <= 0 || panel >= ncols || (sc && sc->tile)) panel = ncols;
   if (panel % 4 != 0) panel = round_up(panel, 4);
   for (int c0 = 0; c0 < ncols; c0 += panel) {
     const int pc = std::min(panel, ncols - c0);
@@ -1746,7 +1750,7 @@ void launch_cheb_step_src_end(int64_t n, const int* rowptr, const int* col, cons
                               hipStream_t st, int panel, const CsrSched* sc, bool cx) {
   if (n <= 0 || ncols <= 0) return;
   if (!end.v_end || !end.um) throw Error(1, "fused recombination: V and um are required");
-  if (panel <= 0 || panel >= ncols) panel = ncols;
+  if (panel <= 0 || panel >= ncols || (sc && sc->tile)) panel = ncols;
   if (panel % 4 != 0) panel = round_up(panel, 4);
   for (int c0 = 0; c0 < ncols; c0 += panel) {
     const int pc = std::min(panel, ncols - c0);

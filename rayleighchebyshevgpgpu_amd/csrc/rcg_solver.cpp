@@ -308,6 +308,8 @@ struct SchedCand {
   std::string name;
   DevBuf order;
   rcg::CsrSched sc;
+  DevBuf srow, pstart, lidx;  // of the tile plan
+  rcg::TilePlan plan;
 };
 
 struct rcg_operator_s {
@@ -320,7 +322,13 @@ struct rcg_operator_s {
   DevBuf own_rowptr, own_col, own_val;
   int64_t max_row = -1;            // nonzeros of the longest row (-1: not looked up yet)
   int64_t gx = 0, gy = 0, gz = 0;  // structured-grid hint (rows x + gx(y + gy z))
+  int64_t dx = 0, dy = 0, dz = 0;  // the grid its rows show (detect_grid), without a hint
+  // row pointers and columns are the library's copy, which nobody changes: a
+  // plan made from them stays true.  Arrays in the caller's memory may change.
+  bool own_pattern = false;
   std::vector<std::unique_ptr<SchedCand>> scheds;
+  std::unique_ptr<SchedCand> tiles;  // the step over LDS tiles (made when first wanted)
+  bool tiles_tried = false;
   struct Tuned {
     int panel;
     int sched;
@@ -861,12 +869,68 @@ class Engine {
     }
   }
 
-  // Filter shape for b columns: the fastest row-block order, then the fastest
-  // column-panel width {b, 32, 16} under it, timed with hipEvents on this
-  // operator (3 Chebyshev steps after a warm-up step) and cached on it per
-  // step kind (0: FP64 step, 1: FP32 correction step).  `launch(panel, sched)`
-  // runs one step on scratch buffers.  RCG_FILTER_PANEL / RCG_FILTER_SCHED
-  // override the choice.
+  // Index of the tile schedule beside those of `scheds`.
+  static constexpr int kTileSched = -2;
+  const SchedCand& sched_at(int k) const {
+    return k == kTileSched ? *op_->tiles : *op_->scheds[k];
+  }
+  // Whether the operator has tiles; made on the first call (lazy_mu held).
+  bool have_tiles() {
+    if (!op_->tiles_tried) {
+      build_tiles();
+      op_->tiles_tried = true;
+    }
+    return op_->tiles != nullptr;
+  }
+  // FP64 steps of b real columns go over LDS tiles from 3 * 2^20 block entries
+  // (24 MB: past L2) and 16 columns.  Measured on periodic 3-D and 2-D grids (us
+  // per step, row blocks / tiles): 64^3 x 16 34 / 32, x 64 120 / 87; 96^3 x 24
+  // 220 / 117; 128^3 x 32 534 / 349, x 64 825 / 676; 1024^2 x 64 377 / 317; equal
+  // at 12 columns.  Below, the blocks stay in L2 and there are too few tiles to
+  // fill the chip: 32^3 x 64 15.4 / 17.4, 44^3 x 32 17.1 / 18.0, x 45 31.6 / 26.5.
+  bool tiles_fp64(int64_t b) const { return n_ * b >= (int64_t)3 << 20 && b >= 16; }
+
+  // The tile plan of an operator on a grid, as a schedule of its own.
+  void build_tiles() {
+    const bool hint = op_->gx > 0;
+    const int64_t gx = hint ? op_->gx : op_->dx, gy = hint ? op_->gy : op_->dy,
+                  gz = hint ? op_->gz : op_->dz;
+    if (!op_->own_pattern || gx < 4 || gy < 4 || gx * gy * gz != n_) return;
+    const rcg::TileShape sh = rcg::tile_shape(gx, gy, gz);
+    auto c = std::make_unique<SchedCand>();
+    c->name = "lds-tiles";
+    try {
+      c->srow.ensure(sizeof(int) * sh.srow);
+      c->pstart.ensure(sizeof(int) * sh.pstart);
+      c->lidx.ensure(sh.lidx);
+    } catch (const Error& e) {
+      if (e.code != RCG_ERR_ALLOC) throw;
+      return;  // no memory for a plan: the general step needs none
+    }
+    DevBuf bad(st_);
+    bad.ensure(sizeof(int));
+    int hbad = 0;
+    RCG_HIP(hipMemcpyAsync(bad.p, &hbad, sizeof(int), hipMemcpyHostToDevice, st_));
+    rcg::launch_tile_plan(sh, n_, op_->rowptr, op_->col, gx, gy, gz, c->srow.as<int>(),
+                          c->pstart.as<int>(), c->lidx.as<unsigned char>(), bad.as<int>(), st_);
+    RCG_HIP(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st_));
+    sync();
+    if (hbad) return;
+    c->plan.srow = c->srow.as<int>();
+    c->plan.pstart = c->pstart.as<int>();
+    c->plan.lidx = c->lidx.as<unsigned char>();
+    c->plan.smax = sh.smax;
+    c->plan.ntile = sh.ntile;
+    c->sc.tile = &c->plan;
+    op_->tiles = std::move(c);
+  }
+
+  // Filter shape for b columns: LDS tiles where they are known to win, else the
+  // fastest of the row-block orders (and tiles), then the fastest column-panel
+  // width {b, 32, 16} under it, timed with hipEvents on this operator (3
+  // Chebyshev steps after a warm-up step) and cached on it per step kind (0: FP64
+  // step, 1: FP32 correction step).  `launch(panel, sched)` runs one step on
+  // scratch buffers.  RCG_FILTER_PANEL / RCG_FILTER_SCHED override the choice.
   template <class Launch>
   rcg_operator_s::Tuned tuned_for(int64_t b, int kind, Launch&& launch) {
     std::lock_guard<std::mutex> lk(op_->lazy_mu);
@@ -874,14 +938,17 @@ class Engine {
     const int64_t key = (int64_t)kind * 1000000000000LL + ld_ * 100000 + b;
     auto it = op_->tuned.find(key);
     rcg_operator_s::Tuned t{(int)b, 0};
+    const bool fp32 = kind == 1 || kind == 3;
     if (it != op_->tuned.end()) {
       t = it->second;
+    } else if (!fp32 && tiles_fp64(b) && have_tiles()) {
+      t.sched = kTileSched;
     } else if (n_ * b >= (int64_t)1 << 22) {  // only large blocks are worth timing
       hipEvent_t e0, e1;
       RCG_HIP(hipEventCreate(&e0));
       RCG_HIP(hipEventCreate(&e1));
       auto time_it = [&](int panel, int sched) {
-        const rcg::CsrSched* sc = &op_->scheds[sched]->sc;
+        const rcg::CsrSched* sc = &sched_at(sched).sc;
         launch(panel, sc);
         RCG_HIP(hipEventRecord(e0, st_));
         for (int r = 0; r < 3; ++r) launch(panel, sc);
@@ -892,7 +959,17 @@ class Engine {
         return ms;
       };
       float best = 1e30f;
-      for (int sidx = 0; sidx < (int)op_->scheds.size(); ++sidx) {
+      // FP32 steps over tiles win from about 45 columns and lose below 32 (64^3 x
+      // 48 81 / 48 us, x 64 83 / 56; 128^3 x 64 488 / 445, x 24 268 / 294; 1024^2 x
+      // 96 345 / 387), where the best order of row blocks is seldom far from
+      // "rows" and "tile16x16": those three are timed, else every order
+      const bool tiles = fp32 && b >= 24 && have_tiles();
+      std::vector<int> cands;
+      for (int k = 0; k < (int)op_->scheds.size(); ++k)
+        if (!tiles || op_->scheds[k]->name == "rows" || op_->scheds[k]->name == "tile16x16")
+          cands.push_back(k);
+      if (tiles) cands.push_back(kTileSched);
+      for (int sidx : cands) {
         const float ms = time_it((int)b, sidx);
         if (ms < best) {
           best = ms;
@@ -900,7 +977,7 @@ class Engine {
         }
       }
       for (int cand : {32, 16}) {
-        if (cand >= b) continue;
+        if (cand >= b || tiles) continue;
         const float ms = time_it(cand, t.sched);
         if (ms < best) {
           best = ms;
@@ -919,7 +996,8 @@ class Engine {
       int pick = -1;
       for (int sidx = 0; sidx < (int)op_->scheds.size(); ++sidx)
         if (op_->scheds[sidx]->name == env) pick = sidx;
-      if (pick < 0)
+      if (std::string("lds-tiles") == env && have_tiles()) pick = kTileSched;
+      if (pick == -1)
         throw Error(RCG_ERR_INVALID, std::string("RCG_FILTER_SCHED names no schedule of this "
                                                  "operator: ") + env);
       t.sched = pick;
@@ -933,6 +1011,7 @@ class Engine {
     if (!T() || !V()) {
       std::lock_guard<std::mutex> lk(op_->lazy_mu);
       build_schedules();
+      if (tiles_fp64(b) && have_tiles()) return rcg_operator_s::Tuned{(int)b, kTileSched};
       auto it = op_->tuned.find((int64_t)(cx_ ? 2 : 0) * 1000000000000LL + ld_ * 100000 + b);
       return it != op_->tuned.end() ? it->second : rcg_operator_s::Tuned{(int)b, 0};
     }
@@ -962,8 +1041,8 @@ class Engine {
                                   (int)(cw_ * d0), (int)(cw_ * cnt), st_);
   }
   const rcg::CsrSched* sched_for(int64_t b) {
-    if (!op_ || batcher_ || n_ * b < (int64_t)1 << 22) return nullptr;
-    return &op_->scheds[tuned_for(b).sched]->sc;
+    if (!op_ || batcher_ || n_ * b < (int64_t)3 << 20) return nullptr;
+    return &sched_at(tuned_for(b).sched).sc;
   }
 
   // Whether the filter of b columns runs in one launch (rcg_small.hip).  The
@@ -1016,9 +1095,9 @@ class Engine {
       return;
     }
     const auto tn = tuned_for(rb);
-    const rcg::CsrSched* sc = &op_->scheds[tn.sched]->sc;
+    const rcg::CsrSched* sc = &sched_at(tn.sched).sc;
     last_panel_ = tn.panel;
-    last_sched_ = op_->scheds[tn.sched]->name;
+    last_sched_ = sched_at(tn.sched).name;
     step_begin(rep * m * ((rb + tn.panel - 1) / tn.panel),
                double(rep) * (csr + 2.0 * blk + double(m - 1) * (csr + 3.0 * blk)));
     for (long r = 0; r < rep; ++r) {
@@ -1239,9 +1318,9 @@ class Engine {
                                   dk + 2 * ld_, (int)ld_, (int)rb, g1f, g2f, 1.0f, st_, panel, sc,
                                   cx_);
       });
-    const rcg::CsrSched* sc = (dn || batcher_) ? nullptr : &op_->scheds[tn.sched]->sc;
+    const rcg::CsrSched* sc = (dn || batcher_) ? nullptr : &sched_at(tn.sched).sc;
     last_panel_ = tn.panel;
-    last_sched_ = dn ? "dense" : (batcher_ ? "batched" : op_->scheds[tn.sched]->name);
+    last_sched_ = dn ? "dense" : (batcher_ ? "batched" : sched_at(tn.sched).name);
     const double csr = dn ? 4.0 * double(n_) * double(n_)
                           : double(op_->nnz) * (4.0 + 4.0 * cw_) + 4.0 * double(n_ + 1);
     const double blk = 4.0 * double(n_) * double(rb);
@@ -2602,6 +2681,27 @@ void check_pair(rcg_operator op, rcg_block a, rcg_block b, int64_t cols, bool al
   need(a->ctx == op->ctx && b->ctx == op->ctx, "handles belong to different contexts");
 }
 
+// The grid a CSR operator's rows are numbered over, read off 256 rows in the
+// middle: the column offsets that at least half of them have are 1, nx and, in
+// 3-D, nx ny.  Only a hint (it chooses which rows are computed together).
+void detect_grid(int64_t n, const int32_t* rowptr, const int32_t* col, int64_t* dx, int64_t* dy,
+                 int64_t* dz) {
+  const int64_t r0 = std::max<int64_t>(0, n / 2 - 128), r1 = std::min<int64_t>(n, r0 + 256);
+  if (rowptr[r1] - rowptr[r0] > 16 * (r1 - r0)) return;
+  std::map<int64_t, int64_t> seen;
+  for (int64_t i = r0; i < r1; ++i)
+    for (int64_t p = rowptr[i]; p < rowptr[i + 1]; ++p)
+      if (col[p] > i) ++seen[col[p] - i];
+  std::vector<int64_t> d;
+  for (const auto& s : seen)
+    if (2 * s.second >= r1 - r0) d.push_back(s.first);
+  if (d.size() < 2 || d.size() > 3 || d[0] != 1 || n % d[1] != 0) return;
+  if (d.size() == 3 && (d[2] % d[1] != 0 || n % d[2] != 0)) return;
+  *dx = d[1];
+  *dy = d.size() == 3 ? d[2] / d[1] : n / d[1];
+  *dz = d.size() == 3 ? n / d[2] : 1;
+}
+
 // leading dimension of a block in real elements
 int64_t real_ld(const rcg_block_s* b) { return (b->dtype == RCG_C128 ? 2 : 1) * b->ld; }
 
@@ -2837,6 +2937,8 @@ int rcg_operator_csr_create(rcg_context ctx, int64_t n, int64_t nnz, const int32
       for (int64_t i = 0; i < n; ++i) need(rowptr[i] <= rowptr[i + 1], "rowptr must be non-decreasing");
       for (int64_t i = 0; i < n; ++i)
         o->max_row = std::max<int64_t>(o->max_row, rowptr[i + 1] - rowptr[i]);
+      o->own_pattern = true;
+      detect_grid(n, rowptr, col, &o->dx, &o->dy, &o->dz);
       for (int64_t p = 0; p < nnz; ++p) need(col[p] >= 0 && col[p] < n, "column index out of range");
       o->own_rowptr.ensure(sizeof(int) * (size_t)(n + 1));
       o->own_col.ensure(sizeof(int) * (size_t)std::max<int64_t>(nnz, 1));
@@ -2873,6 +2975,10 @@ int rcg_operator_csr_share(rcg_operator base, const void* val, int mem, rcg_oper
     o->gx = base->gx;
     o->gy = base->gy;
     o->gz = base->gz;
+    o->dx = base->dx;
+    o->dy = base->dy;
+    o->dz = base->dz;
+    o->own_pattern = base->own_pattern;
     if (mem == RCG_MEM_DEVICE) {
       o->val = static_cast<const double*>(val);
     } else {
@@ -2941,6 +3047,8 @@ int rcg_operator_set_grid(rcg_operator op, int64_t nx, int64_t ny, int64_t nz) {
     op->gy = ny;
     op->gz = nz;
     op->scheds.clear();
+    op->tiles.reset();
+    op->tiles_tried = false;
     op->tuned.clear();
   });
 }
@@ -2972,11 +3080,14 @@ int rcg_operator_apply(rcg_operator op, rcg_block in, rcg_block out, double alph
                                      (int)cols, alpha, beta, 0.0,
                                      beta == 0.0 ? rcg::kStepApply : rcg::kStepApplyBeta, nullptr,
                                      nullptr, op->ctx->stream);
-    else
+    else {
+      Engine e(op->ctx, op, op->n);
+      e.attach(nullptr, nullptr, nullptr, real_ld(in), nullptr, 0);
       rcg::launch_csr_apply<double>(op->n, op->rowptr, op->col, op->val,
                                     static_cast<const double*>(in->d()), static_cast<double*>(out->d()),
                                     (int)real_ld(in), (int)((cx ? 2 : 1) * cols), alpha, beta,
-                                    op->ctx->stream, nullptr, cx);
+                                    op->ctx->stream, e.sched_for((cx ? 2 : 1) * cols), cx);
+    }
     RCG_HIP(hipStreamSynchronize(op->ctx->stream));
   });
 }

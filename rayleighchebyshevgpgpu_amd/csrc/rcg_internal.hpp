@@ -295,6 +295,9 @@ void launch_resid_norm_sumsq_args(int64_t n, const double* V, const double* W, i
 // ldc entries per column.  to_cols: rows -> column-major, else the reverse.
 void launch_layout(int64_t n, int cols, int cw, double* rows, int64_t ldr_real, double* colmaj,
                    int64_t ldc, bool to_cols, hipStream_t st);
+// The same for entries of es = 4, 8 or 16 bytes, leading dimensions in entries.
+void launch_block_layout(int64_t n, int cols, int es, void* rows, int64_t ldr, void* colmaj,
+                         int64_t ldc, bool to_cols, hipStream_t st);
 // out = p2 (p1 (p0 AX + X) - Z) (rows layout; AX column-major, Z optional
 // and may alias out): a Chebyshev step around a caller operator's product.
 void launch_cheb_combine(int64_t n, int cols, int cw, const double* AX, int64_t ldc,

@@ -2307,31 +2307,31 @@ __global__ __launch_bounds__(kThreads) void cheb_combine_kernel(int64_t n, int c
   }
 }
 
+void launch_block_layout(int64_t n, int cols, int es, void* rows, int64_t ldr, void* colmaj,
+                         int64_t ldc, bool to_cols, hipStream_t st) {
+  if (n <= 0 || cols <= 0) return;
+  const dim3 grid((unsigned)((n + kLt - 1) / kLt), (unsigned)((cols + kLt - 1) / kLt));
+  auto go = [&](auto entry) {
+    using E = decltype(entry);
+    if (to_cols)
+      hipLaunchKernelGGL((layout_kernel<E, true>), grid, dim3(kThreads), 0, st, n, cols,
+                         static_cast<E*>(rows), ldr, static_cast<E*>(colmaj), ldc);
+    else
+      hipLaunchKernelGGL((layout_kernel<E, false>), grid, dim3(kThreads), 0, st, n, cols,
+                         static_cast<E*>(rows), ldr, static_cast<E*>(colmaj), ldc);
+  };
+  if (es == 4) go(float());
+  else if (es == 8) go(double());
+  else if (es == 16) go(double2());
+  else throw Error(1, "block entries are 4, 8 or 16 bytes");
+  RCG_HIP(hipGetLastError());
+}
+
 void launch_layout(int64_t n, int cols, int cw, double* rows, int64_t ldr_real, double* colmaj,
                    int64_t ldc, bool to_cols, hipStream_t st) {
-  if (n <= 0 || cols <= 0) return;
   if (cw != 1 && cw != 2) throw Error(1, "entries are real or complex");
   if (ldr_real % cw != 0) throw Error(1, "row stride is not a whole number of entries");
-  const dim3 grid((unsigned)((n + kLt - 1) / kLt), (unsigned)((cols + kLt - 1) / kLt));
-  const int64_t ldr = ldr_real / cw;
-  if (cw == 1) {
-    if (to_cols)
-      hipLaunchKernelGGL((layout_kernel<double, true>), grid, dim3(kThreads), 0, st, n, cols, rows,
-                         ldr, colmaj, ldc);
-    else
-      hipLaunchKernelGGL((layout_kernel<double, false>), grid, dim3(kThreads), 0, st, n, cols, rows,
-                         ldr, colmaj, ldc);
-  } else {
-    double2* r2 = reinterpret_cast<double2*>(rows);
-    double2* c2 = reinterpret_cast<double2*>(colmaj);
-    if (to_cols)
-      hipLaunchKernelGGL((layout_kernel<double2, true>), grid, dim3(kThreads), 0, st, n, cols, r2,
-                         ldr, c2, ldc);
-    else
-      hipLaunchKernelGGL((layout_kernel<double2, false>), grid, dim3(kThreads), 0, st, n, cols, r2,
-                         ldr, c2, ldc);
-  }
-  RCG_HIP(hipGetLastError());
+  launch_block_layout(n, cols, 8 * cw, rows, ldr_real / cw, colmaj, ldc, to_cols, st);
 }
 
 void launch_cheb_combine(int64_t n, int cols, int cw, const double* AX, int64_t ldc,

@@ -260,6 +260,20 @@ template <typename T>
 void launch_tall_gemm(int64_t n, const T* X, int ldx, int bx, const T* C, int ldc, int by,
                       T alpha, T beta, const T* Z, T* out, int ldo, hipStream_t st);
 
+// The same (FP64) with a by-product formed from out's rows while they are in
+// registers: its column sums of squares; out^T out (by x by); X^T out (bx x by,
+// beta = 1).  The latter two take at most 64 columns.  ws holds partials, within
+// gram_ws_bound.
+void launch_tall_gemm_sums(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc,
+                           int by, double alpha, double beta, const double* Z, double* out, int ldo,
+                           double* sums, double* ws, size_t ws_elems, hipStream_t st);
+void launch_tall_gemm_gram(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc,
+                           int by, double* out, int ldo, double* G, double* ws, size_t ws_elems,
+                           hipStream_t st);
+void launch_tall_gemm_cross(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc,
+                            int by, double alpha, const double* Z, double* out, int ldo, double* G,
+                            double* ws, size_t ws_elems, hipStream_t st);
+
 // sums[c] = sum_i |X[i,c]|^2, c < nc.
 template <typename T>
 void launch_col_sumsq(int64_t n, const T* X, int ld, int nc, double* sums, double* ws,
@@ -311,6 +325,9 @@ void launch_lz_dot_c(int64_t n, const double* w, const double* v, double* alpha_
 // residual norm of each (complex, cw = 2) column from its real columns' sums.
 void launch_group_sqrt(const double* sums, int cw, int count, double* out, hipStream_t st);
 
+// out[i,c] = X[i,c] / sqrt(|sums[c]|), c < nc (out may be X).
+void launch_scale_cols(int64_t n, const double* X, int ld, int nc, const double* sums, double* out,
+                       hipStream_t st);
 // X[i,c] *= 1/sqrt(sums[c]), c < nc.
 template <typename T>
 void launch_normalize_cols(int64_t n, T* X, int ld, int nc, const double* sums, hipStream_t st);

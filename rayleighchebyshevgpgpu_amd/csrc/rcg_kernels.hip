@@ -675,6 +675,8 @@ __global__ __launch_bounds__(kThreads, 2) void gram_lds_kernel(
     }
 }
 
+enum TallAfter { kTallNone = 0, kTallSums = 1, kTallGram = 2, kTallCross = 3 };
+
 // out = alpha X C + beta Z (X: n x bx, C: bx x by column-major).  A wave owns
 // 16 rows of a 64-row tile; lane (kk = l/16, r = l%16) loads the 16
 // consecutive entries [16kk, 16kk+16) of row r of a 64-wide k chunk with
@@ -683,11 +685,19 @@ __global__ __launch_bounds__(kThreads, 2) void gram_lds_kernel(
 // j, so 16 lanes store 16 consecutive columns of one row.  Workgroups loop
 // over row tiles; C is staged once when bx <= 64.  blockIdx.y selects 64
 // output columns.
-template <bool BETA, int NTC>
+//
+// AFTER: what is also formed from the rows while they are in registers, so that
+// no pass over the block follows for it (one partial per workgroup in P):
+//   kTallSums: out's column sums of squares (by values);
+//   kTallGram: out^T out (by x by, bx and by <= 64): a register of D is the A and
+//     the B fragment of the rows' Gram product as it stands (lane (kk, r) holds
+//     row 4j+kk of column 16t+r), so it costs MFMAs only;
+//   kTallCross: X^T out (bx x by, both <= 64), X read again in D's layout.
+template <bool BETA, int NTC, int AFTER, int NTX>
 __global__ __launch_bounds__(kThreads) void tall_gemm_mfma_kernel(
     int64_t n, const double* __restrict__ X, int ldx, int bx, const double* __restrict__ C,
     int ldc, int by, double alpha, double beta, const double* Z, double* out, int ldo,
-    int64_t ntiles, int ct, int64_t nstripe) {
+    int64_t ntiles, int ct, int64_t nstripe, double* __restrict__ P) {
   __shared__ double cs[kTile][kTile + 1];  // [k][c]
   // 1-D grid of nstripe x ct workgroups: the ct column tiles of a row stripe are
   // consecutive logical workgroups on one XCD, so X rows are read from HBM once
@@ -711,6 +721,18 @@ __global__ __launch_bounds__(kThreads) void tall_gemm_mfma_kernel(
   if (nk == 1) {
     stage(0);
     __syncthreads();
+  }
+  double sum[AFTER == kTallSums ? NTC : 1];
+  d4v gram[AFTER >= kTallGram ? NTX : 1][AFTER >= kTallGram ? NTC : 1];
+  if constexpr (AFTER == kTallSums) {
+#pragma unroll
+    for (int t = 0; t < NTC; ++t) sum[t] = 0.0;
+  }
+  if constexpr (AFTER >= kTallGram) {
+#pragma unroll
+    for (int p = 0; p < NTX; ++p)
+#pragma unroll
+      for (int t = 0; t < NTC; ++t) gram[p][t] = d4v{0.0, 0.0, 0.0, 0.0};
   }
   for (int64_t tile = stripe; tile < ntiles; tile += nstripe) {
     const int64_t row = tile * kTile + wave * 16 + r;
@@ -763,18 +785,91 @@ __global__ __launch_bounds__(kThreads) void tall_gemm_mfma_kernel(
         }
       }
     }
+    // X in D's layout: rows 4j+kk, columns 16p+r (read before the stores)
+    double ya[AFTER == kTallCross ? 4 : 1][NTX];
+    if constexpr (AFTER == kTallCross) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t ro = tile * kTile + wave * 16 + 4 * j + kk;
+#pragma unroll
+        for (int p = 0; p < NTX; ++p)
+          ya[j][p] = (ro < n && 16 * p + r < bx) ? X[ro * ldx + 16 * p + r] : 0.0;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int64_t ro = tile * kTile + wave * 16 + 4 * j + kk;
-      if (ro >= n) continue;
 #pragma unroll
       for (int t = 0; t < NTC; ++t) {
         const int c = c0 + 16 * t + r;
-        if (c >= by) continue;
         double v = alpha * acc[t][j];
         if constexpr (BETA) v = fma(beta, zv[j][t], v);
-        out[ro * ldo + c] = v;
+        if (ro < n && c < by) out[ro * ldo + c] = v;
+        // rows past n and columns past by are zero here
+        if constexpr (AFTER == kTallSums) sum[t] = fma(v, v, sum[t]);
+        if constexpr (AFTER >= kTallGram) acc[t][j] = v;
       }
+    }
+    if constexpr (AFTER >= kTallGram) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int p = 0; p < NTX; ++p)
+#pragma unroll
+          for (int t = 0; t < NTC; ++t) {
+            if (AFTER == kTallGram && p > t) continue;
+            gram[p][t] =
+                mfma16x16x4(AFTER == kTallGram ? acc[p][j] : ya[j][p], acc[t][j], gram[p][t]);
+          }
+    }
+  }
+  if constexpr (AFTER == kTallSums) {
+    // over the 4 row groups of a wave, then the waves in order
+#pragma unroll
+    for (int t = 0; t < NTC; ++t) {
+      sum[t] += __shfl_xor(sum[t], 16);
+      sum[t] += __shfl_xor(sum[t], 32);
+    }
+    __syncthreads();  // C is no longer read
+    double* red = &cs[0][0];
+    if (kk == 0) {
+#pragma unroll
+      for (int t = 0; t < NTC; ++t) red[wave * kTile + 16 * t + r] = sum[t];
+    }
+    __syncthreads();
+    const int c = (int)threadIdx.x;
+    if (c < 16 * NTC && c0 + c < by)
+      P[stripe * by + c0 + c] =
+          ((red[c] + red[kTile + c]) + red[2 * kTile + c]) + red[3 * kTile + c];
+  }
+  if constexpr (AFTER >= kTallGram) {
+    __syncthreads();
+    double* red = &cs[0][0];
+    for (int w = 0; w < 4; ++w) {
+      if (wave == w) {
+#pragma unroll
+        for (int p = 0; p < NTX; ++p)
+#pragma unroll
+          for (int t = 0; t < NTC; ++t) {
+            if (AFTER == kTallGram && p > t) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const int e = (16 * p + 4 * j + kk) + kTile * (16 * t + r);
+              red[e] = (w == 0) ? gram[p][t][j] : red[e] + gram[p][t][j];
+            }
+          }
+      }
+      __syncthreads();
+    }
+    const int rows = AFTER == kTallGram ? by : bx;
+    double* Pb = P + stripe * (int64_t)rows * by;
+    for (int e = threadIdx.x; e < kTile * kTile; e += kThreads) {
+      const int a = e % kTile, b = e / kTile;
+      if (a >= rows || b >= by) continue;
+      // out^T out: the subtiles above the diagonal, and their mirror
+      Pb[a + (int64_t)b * rows] = (AFTER == kTallGram && (a >> 4) > (b >> 4))
+                                      ? red[b + kTile * a]
+                                      : red[a + kTile * b];
     }
   }
 }
@@ -789,11 +884,12 @@ __global__ __launch_bounds__(kThreads) void tall_gemm_mfma_kernel(
 // wave's chunk exists is decided once per wave (a scalar branch): loads that
 // lanes take or skip on their own would make the wave wait for the loads in
 // flight where the paths join, which takes the prefetch's overlap away.
-template <int KCH>
+// SUMS: also out's column sums of squares, a partial per workgroup in P.
+template <int KCH, bool SUMS>
 __global__ __launch_bounds__(kThreads) void tall_gemm_wide_kernel(
     int64_t n, const double* __restrict__ X, int ldx, int bx, const double* __restrict__ C,
     int ldc, int by, double alpha, double beta, const double* Z, double* out, int ldo,
-    int64_t ntiles, int ct, int64_t nstripe) {
+    int64_t ntiles, int ct, int64_t nstripe, double* __restrict__ P) {
   constexpr int KP = KCH * kTile;
   __shared__ double cs[KP][kTile + 1];  // [k][c]
   const int64_t L = xcd_remap(blockIdx.x, gridDim.x);
@@ -842,6 +938,7 @@ __global__ __launch_bounds__(kThreads) void tall_gemm_wide_kernel(
   // register that entered the loops with a load in flight would make every
   // chunk wait for the loads issued ahead of its MFMAs
   double xa[2][16], xn[2][16];
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
   if (stripe < ntiles) load(stripe * (2 * kTile) + wave * 32, 0, xn);
   for (int64_t tile = stripe; tile < ntiles; tile += nstripe) {
     const int64_t r0 = tile * (2 * kTile) + wave * 32;
@@ -921,6 +1018,7 @@ __global__ __launch_bounds__(kThreads) void tall_gemm_wide_kernel(
             double v = alpha * acc[g][t][j];
             if (beta != 0.0) v = fma(beta, zv[g][j][t], v);
             out[(r0 + 16 * g + 4 * j + kk) * ldo + c0 + 16 * t + r] = v;
+            if constexpr (SUMS) sum[t] = fma(v, v, sum[t]);
           }
     } else {
 #pragma unroll
@@ -936,9 +1034,28 @@ __global__ __launch_bounds__(kThreads) void tall_gemm_wide_kernel(
             double v = alpha * acc[g][t][j];
             if (beta != 0.0) v = fma(beta, zv[g][j][t], v);
             out[ro * ldo + c] = v;
+            if constexpr (SUMS) sum[t] = fma(v, v, sum[t]);
           }
         }
     }
+  }
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      sum[t] += __shfl_xor(sum[t], 16);
+      sum[t] += __shfl_xor(sum[t], 32);
+    }
+    __syncthreads();  // C is no longer read
+    double* red = &cs[0][0];
+    if (kk == 0) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) red[wave * kTile + 16 * t + r] = sum[t];
+    }
+    __syncthreads();
+    const int c = (int)threadIdx.x;
+    if (c < kTile && c0 + c < by)
+      P[stripe * by + c0 + c] =
+          ((red[c] + red[kTile + c]) + red[2 * kTile + c]) + red[3 * kTile + c];
   }
 }
 
@@ -1326,6 +1443,19 @@ __global__ __launch_bounds__(kThreads) void normalize_cols_kernel(int64_t n, T* 
   if (i >= n) return;
   const double s = 1.0 / sqrt(fabs(sums[c]));
   X[i * ld + c] = T(double(X[i * ld + c]) * s);
+}
+
+// out[i,c] = X[i,c] / sqrt(|sums[c]|) (out may be X)
+__global__ __launch_bounds__(kThreads) void scale_cols_kernel(int64_t n, const double* X, int ld,
+                                                              int nc,
+                                                              const double* __restrict__ sums,
+                                                              double* out) {
+  const int64_t e = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  const int64_t i = e / nc;
+  const int c = (int)(e % nc);
+  if (i >= n) return;
+  const double s = 1.0 / sqrt(fabs(sums[c]));
+  out[i * ld + c] = X[i * ld + c] * s;
 }
 
 template <typename T>
@@ -1938,61 +2068,153 @@ void launch_gram_pair(int64_t n, const double* X, int ldx, const double* Y, int 
   RCG_HIP(hipGetLastError());
 }
 
+namespace {
+// Workgroups of the wide tall product: C slice resident in LDS (66.5, 100 or
+// 133 KB) and about 300 registers per lane, one workgroup per CU, persistent
+// over 128-row tiles.
+int64_t wide_stripes(int64_t n, int ct) {
+  const int64_t nrt = (n + 2 * kTile - 1) / (2 * kTile);
+  return std::max<int64_t>(1, std::min<int64_t>(nrt, 256 / (int64_t)ct));
+}
+// Workgroups of the narrow one, persistent over 64-row tiles: as many as fit at
+// once on a 256-CU part (four per CU, three with the registers that hold beta Z
+// or column sums, two with a Gram matrix's).
+int64_t tall_stripes(int64_t n, int ct, bool beta, int after) {
+  const int64_t wgs = after >= kTallGram ? 512 : (beta || after == kTallSums ? 768 : 1024);
+  return std::max<int64_t>(1, std::min<int64_t>((n + kTile - 1) / kTile, wgs / (int64_t)ct));
+}
+template <bool SUMS>
+void tall_wide(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc, int by,
+               double alpha, double beta, const double* Z, double* out, int ldo, double* P,
+               hipStream_t st) {
+  const int ct = (by + kTile - 1) / kTile;
+  const int kch = (bx + kTile - 1) / kTile;
+  const int64_t nrt = (n + 2 * kTile - 1) / (2 * kTile);
+  const int64_t nstripe = wide_stripes(n, ct);
+  const dim3 grid((unsigned)round_up(nstripe * ct, kXcds));
+#define RCG_WIDE(K)                                                                               \
+  hipLaunchKernelGGL((tall_gemm_wide_kernel<K, SUMS>), grid, dim3(kThreads), 0, st, n, X, ldx, bx, \
+                     C, ldc, by, alpha, beta, Z, out, ldo, nrt, ct, nstripe, P)
+  if (kch == 2) RCG_WIDE(2);
+  else if (kch == 3) RCG_WIDE(3);
+  else RCG_WIDE(4);
+#undef RCG_WIDE
+  RCG_HIP(hipGetLastError());
+}
+template <int AFTER, int NTC, int NTX>
+void tall_one(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc, int by,
+              double alpha, double beta, const double* Z, double* out, int ldo, double* P,
+              hipStream_t st) {
+  const int ct = (by + kTile - 1) / kTile;
+  const int64_t nrb = (n + kTile - 1) / kTile;
+  const int64_t nstripe = tall_stripes(n, ct, beta != 0.0, AFTER);
+  const dim3 grid((unsigned)round_up(nstripe * ct, kXcds));
+  // out^T out follows products without Z, X^T out the deflation's only
+  if constexpr (AFTER != kTallGram)
+    if (beta != 0.0)
+      hipLaunchKernelGGL((tall_gemm_mfma_kernel<true, NTC, AFTER, NTX>), grid, dim3(kThreads), 0,
+                         st, n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, nrb, ct, nstripe,
+                         P);
+  if constexpr (AFTER != kTallCross)
+    if (beta == 0.0 || AFTER == kTallGram)
+      hipLaunchKernelGGL((tall_gemm_mfma_kernel<false, NTC, AFTER, NTX>), grid, dim3(kThreads), 0,
+                         st, n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, nrb, ct, nstripe,
+                         P);
+  RCG_HIP(hipGetLastError());
+}
+template <int AFTER>
+void tall_narrow(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc, int by,
+                 double alpha, double beta, const double* Z, double* out, int ldo, double* P,
+                 hipStream_t st) {
+  const int ntc = by >= kTile ? 4 : (by + 15) / 16;
+#define RCG_TALL(NTC, NTX) \
+  tall_one<AFTER, NTC, NTX>(n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, P, st)
+  if constexpr (AFTER == kTallCross) {
+    const int ntx = bx <= 16 ? 1 : (bx <= 32 ? 2 : 4);
+#define RCG_TALL_X(NTC)               \
+  if (ntx == 1) RCG_TALL(NTC, 1);     \
+  else if (ntx == 2) RCG_TALL(NTC, 2); \
+  else RCG_TALL(NTC, 4);              \
+  break;
+    switch (ntc) {
+      case 1: RCG_TALL_X(1)
+      case 2: RCG_TALL_X(2)
+      case 3: RCG_TALL_X(3)
+      default: RCG_TALL_X(4)
+    }
+#undef RCG_TALL_X
+  } else {
+    switch (ntc) {
+      case 1: RCG_TALL(1, 1); break;
+      case 2: RCG_TALL(2, 2); break;
+      case 3: RCG_TALL(3, 3); break;
+      default: RCG_TALL(4, 4); break;
+    }
+  }
+#undef RCG_TALL
+}
+}  // namespace
+
 template <typename T>
 void launch_tall_gemm(int64_t n, const T* X, int ldx, int bx, const T* C, int ldc, int by,
                       T alpha, T beta, const T* Z, T* out, int ldo, hipStream_t st) {
   if (n <= 0 || by <= 0) return;
-  const int64_t nrb = (n + kTile - 1) / kTile;
-  const int64_t grid = round_up(nrb, kXcds);
-  const unsigned ct = (unsigned)((by + kTile - 1) / kTile);
   if constexpr (std::is_same<T, double>::value) {
-    if (bx > kTile && bx <= 4 * kTile) {
-      // C slice resident in LDS (66.5, 100 or 133 KB) and about 300 registers
-      // per lane: one workgroup per CU, persistent over 128-row tiles
-      const int kch = (bx + kTile - 1) / kTile;
-      const int64_t nrt = (n + 2 * kTile - 1) / (2 * kTile);
-      const int64_t nstripe = std::max<int64_t>(1, std::min<int64_t>(nrt, 256 / (int64_t)ct));
-      const dim3 grid((unsigned)round_up(nstripe * ct, kXcds));
-      if (kch == 2)
-        hipLaunchKernelGGL(tall_gemm_wide_kernel<2>, grid, dim3(kThreads), 0, st, n, X, ldx, bx, C,
-                           ldc, by, alpha, beta, Z, out, ldo, nrt, (int)ct, nstripe);
-      else if (kch == 3)
-        hipLaunchKernelGGL(tall_gemm_wide_kernel<3>, grid, dim3(kThreads), 0, st, n, X, ldx, bx, C,
-                           ldc, by, alpha, beta, Z, out, ldo, nrt, (int)ct, nstripe);
-      else
-        hipLaunchKernelGGL(tall_gemm_wide_kernel<4>, grid, dim3(kThreads), 0, st, n, X, ldx, bx, C,
-                           ldc, by, alpha, beta, Z, out, ldo, nrt, (int)ct, nstripe);
-      RCG_HIP(hipGetLastError());
-      return;
-    }
-    // persistent over row tiles: as many workgroups as fit at once on a
-    // 256-CU part (four per CU, three with the registers that hold beta Z)
-    const int64_t wgs = beta != 0.0 ? 768 : 1024;
-    const int64_t nstripe = std::max<int64_t>(1, std::min<int64_t>(nrb, wgs / (int64_t)ct));
-    const dim3 grid((unsigned)round_up(nstripe * ct, kXcds));
-    const int ntc = by >= kTile ? 4 : (by + 15) / 16;
-#define RCG_TALL_NTC(NTC)                                                                           \
-  case NTC:                                                                                         \
-    if (beta != 0.0)                                                                                \
-      hipLaunchKernelGGL((tall_gemm_mfma_kernel<true, NTC>), grid, dim3(kThreads), 0, st, n, X, ldx, \
-                         bx, C, ldc, by, alpha, beta, Z, out, ldo, nrb, (int)ct, nstripe);          \
-    else                                                                                            \
-      hipLaunchKernelGGL((tall_gemm_mfma_kernel<false, NTC>), grid, dim3(kThreads), 0, st, n, X,    \
-                         ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, nrb, (int)ct, nstripe);     \
-    break;
-    switch (ntc) {
-      RCG_TALL_NTC(1)
-      RCG_TALL_NTC(2)
-      RCG_TALL_NTC(3)
-      RCG_TALL_NTC(4)
-      default: throw Error(1, "bad tall product width");
-    }
-#undef RCG_TALL_NTC
+    if (bx > kTile && bx <= 4 * kTile)
+      tall_wide<false>(n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, nullptr, st);
+    else
+      tall_narrow<kTallNone>(n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, nullptr, st);
   } else {
-    hipLaunchKernelGGL(tall_gemm_kernel<T>, dim3((unsigned)grid, ct), dim3(kThreads), 0, st, n, X,
-                       ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, nrb);
+    const int64_t nrb = (n + kTile - 1) / kTile;
+    const unsigned ct = (unsigned)((by + kTile - 1) / kTile);
+    hipLaunchKernelGGL(tall_gemm_kernel<T>, dim3((unsigned)round_up(nrb, kXcds), ct),
+                       dim3(kThreads), 0, st, n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo,
+                       nrb);
+    RCG_HIP(hipGetLastError());
   }
+}
+
+namespace {
+void reduce_to(const double* P, int64_t nblk, int64_t m, double* out, hipStream_t st) {
+  hipLaunchKernelGGL((reduce_partials_kernel<double, double>), dim3(reduce_grid(m)),
+                     dim3(kThreads), 0, st, P, nblk, m, out);
   RCG_HIP(hipGetLastError());
+}
+}  // namespace
+
+void launch_tall_gemm_sums(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc,
+                           int by, double alpha, double beta, const double* Z, double* out, int ldo,
+                           double* sums, double* ws, size_t ws_elems, hipStream_t st) {
+  if (n <= 0 || by <= 0) return;
+  const bool wide = bx > kTile && bx <= 4 * kTile;
+  const int ct = (by + kTile - 1) / kTile;
+  const int64_t nblk = wide ? wide_stripes(n, ct) : tall_stripes(n, ct, beta != 0.0, kTallSums);
+  if ((size_t)(nblk * by) > ws_elems) throw Error(3, "column-sum workspace too small");
+  if (wide) tall_wide<true>(n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, ws, st);
+  else tall_narrow<kTallSums>(n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, ws, st);
+  reduce_to(ws, nblk, by, sums, st);
+}
+
+void launch_tall_gemm_gram(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc,
+                           int by, double* out, int ldo, double* G, double* ws, size_t ws_elems,
+                           hipStream_t st) {
+  if (n <= 0 || by <= 0) return;
+  if (bx > kTile || by > kTile) throw Error(1, "fused Gram products take at most 64 columns");
+  const int64_t nblk = tall_stripes(n, 1, false, kTallGram), m = (int64_t)by * by;
+  if ((size_t)(nblk * m) > ws_elems) throw Error(3, "gram workspace too small");
+  tall_narrow<kTallGram>(n, X, ldx, bx, C, ldc, by, 1.0, 0.0, nullptr, out, ldo, ws, st);
+  reduce_to(ws, nblk, m, G, st);
+}
+
+void launch_tall_gemm_cross(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc,
+                            int by, double alpha, const double* Z, double* out, int ldo, double* G,
+                            double* ws, size_t ws_elems, hipStream_t st) {
+  if (n <= 0 || by <= 0) return;
+  if (bx > kTile || by > kTile) throw Error(1, "fused Gram products take at most 64 columns");
+  const int64_t nblk = tall_stripes(n, 1, true, kTallCross), m = (int64_t)bx * by;
+  if ((size_t)(nblk * m) > ws_elems) throw Error(3, "gram workspace too small");
+  tall_narrow<kTallCross>(n, X, ldx, bx, C, ldc, by, alpha, 1.0, Z, out, ldo, ws, st);
+  reduce_to(ws, nblk, m, G, st);
 }
 
 size_t colred_ws_elems(int64_t n, int nc) {
@@ -2079,6 +2301,14 @@ void launch_normalize_cols(int64_t n, T* X, int ld, int nc, const double* sums, 
   if (n <= 0 || nc <= 0) return;
   hipLaunchKernelGGL(normalize_cols_kernel<T>, dim3(grid_for(n * nc)), dim3(kThreads), 0, st, n, X,
                      ld, nc, sums);
+  RCG_HIP(hipGetLastError());
+}
+
+void launch_scale_cols(int64_t n, const double* X, int ld, int nc, const double* sums, double* out,
+                       hipStream_t st) {
+  if (n <= 0 || nc <= 0) return;
+  hipLaunchKernelGGL(scale_cols_kernel, dim3(grid_for(n * nc)), dim3(kThreads), 0, st, n, X, ld, nc,
+                     sums, out);
   RCG_HIP(hipGetLastError());
 }
 

@@ -1482,8 +1482,11 @@ class Engine {
                     int64_t by, S* host, bool lower_only = false) {
     constexpr int w = std::is_same<S, cplx>::value ? 2 : 1;
     const int64_t rx = w * bx, ry = w * by;
-    rcg::launch_gram<double>(n_, X, (int)ldx, (int)rx, Yp, (int)ldy, (int)ry, dres(), ws(),
-                             ws_elems_, st_, lower_only);
+    // V^H V may have been formed by the product that wrote V
+    if (!(gram_ready_ && X == V() && Yp == V()))
+      rcg::launch_gram<double>(n_, X, (int)ldx, (int)rx, Yp, (int)ldy, (int)ry, dres(), ws(),
+                               ws_elems_, st_, lower_only);
+    gram_ready_ = false;
     sync();
     const double* g = hres();
     if constexpr (w == 1) {
@@ -1498,10 +1501,10 @@ class Engine {
     }
   }
 
-  // V <- V C, C host b x b column-major; the result lands in T, then swaps.
-  // Complex C enters the real product through its 2b x 2b real embedding.
+  // C (host, b x b column-major) into dmatA(); complex C as its 2b x 2b real
+  // embedding.
   template <class S>
-  void right_multiply(int64_t b, const S* C) {
+  void upload_factor(int64_t b, const S* C) {
     if constexpr (std::is_same<S, double>::value) {
       std::memcpy(hmatB(), C, sizeof(double) * b * b);
     } else {
@@ -1518,16 +1521,41 @@ class Engine {
     }
     const int64_t rb = cw_ * b;
     RCG_HIP(hipMemcpyAsync(dmatA(), hmatB(), sizeof(double) * rb * rb, hipMemcpyHostToDevice, st_));
-    rcg::launch_tall_gemm<double>(n_, V(), (int)ld_, (int)rb, dmatA(), (int)rb, (int)rb, 1.0, 0.0,
-                                  nullptr, T(), (int)ld_, st_);
+  }
+  // V <- V C; the result lands in T, then swaps.  gram: the real Gram matrix of
+  // the new V's (real) columns goes to dres() as well (at most 64 columns).
+  template <class S>
+  void right_multiply(int64_t b, const S* C, bool gram = false) {
+    upload_factor<S>(b, C);
+    const int64_t rb = cw_ * b;
+    if (gram && rb <= 64)
+      rcg::launch_tall_gemm_gram(n_, V(), (int)ld_, (int)rb, dmatA(), (int)rb, (int)rb, T(),
+                                 (int)ld_, dres(), ws(), ws_elems_, st_);
+    else
+      rcg::launch_tall_gemm<double>(n_, V(), (int)ld_, (int)rb, dmatA(), (int)rb, (int)rb, 1.0,
+                                    0.0, nullptr, T(), (int)ld_, st_);
     swapVT();
+    gram_ready_ = gram && rb <= 64;
+  }
+  // V <- normalize(V C) (rcg_rotate): the columns' norms come with the product
+  // and the scaling pass brings it back from T, against a pass each for norms,
+  // scaling and the copy back (128^3 x 64: 1.45 -> 0.87 ms).
+  template <class S>
+  void rotate_normalized(int64_t b, const S* C) {
+    upload_factor<S>(b, C);
+    const int64_t rb = cw_ * b;
+    rcg::launch_tall_gemm_sums(n_, V(), (int)ld_, (int)rb, dmatA(), (int)rb, (int)rb, 1.0, 0.0,
+                               nullptr, T(), (int)ld_, dsums(), ws(), ws_elems_, st_);
+    if (cx_) rcg::launch_pair_sums(dsums(), (int)b, st_);
+    rcg::launch_scale_cols(n_, T(), (int)ld_, (int)rb, dsums(), V(), st_);
   }
 
   // One CholQR pass on V[:, :b]: G = V^H V scaled to unit diagonal,
   // G = R^H R, V <- V D R^{-1}.  A failed factorisation retries with the
   // shift 11(nb + b(b+1)) u ||G|| (shifted CholeskyQR); returns false then.
+  // gram: the next pass's Gram matrix is formed with the product.
   template <class S>
-  bool cholqr_pass(int64_t b, bool allow_shift) {
+  bool cholqr_pass(int64_t b, bool allow_shift, bool gram = false) {
     std::vector<S> G(b * b);
     gram_to_host<S>(V(), ld_, b, V(), ld_, b, G.data());
     std::vector<double> d(b);
@@ -1551,7 +1579,7 @@ class Engine {
     rcg::dense::upper_inverse(R, b, Ri);
     for (int64_t j = 0; j < b; ++j)
       for (int64_t i = 0; i < b; ++i) Ri[i + j * b] *= d[i];
-    right_multiply<S>(b, Ri.data());
+    right_multiply<S>(b, Ri.data(), gram);
     return clean;
   }
 
@@ -1565,8 +1593,8 @@ class Engine {
   }
   template <class S>
   void orthonormalize_t(int64_t b) {
-    const bool clean = cholqr_pass<S>(b, true);
-    cholqr_pass<S>(b, true);
+    const bool clean = cholqr_pass<S>(b, true, true);
+    cholqr_pass<S>(b, true, !clean);
     if (!clean) cholqr_pass<S>(b, false);
   }
 
@@ -1574,23 +1602,38 @@ class Engine {
   // OrthogonalizeAtoB (RayleighChebyshevLM.h:1844-1917) against Y[:, :found]:
   // V -= Y (Y^H V), twice.  The normalisation of the reference is implied by
   // the CholQR that follows in the solve.
-  void deflate(int64_t b, int64_t found) {
+  // Up to 64 real columns each, the second pass's Y^H V is formed by the product
+  // of the first (no read of Y and V of its own); with `norms` the second
+  // product also leaves the columns' squared norms in dsums().
+  void deflate(int64_t b, int64_t found, bool norms = false) {
     if (found <= 0 || b <= 0) return;
+    gram_ready_ = false;
     const int64_t rf = cw_ * found, rb = cw_ * b;
+    const bool cross = rf <= 64 && rb <= 64;
     for (int pass = 0; pass < 2; ++pass) {
-      rcg::launch_gram<double>(n_, Y_, (int)ldy_, (int)rf, V(), (int)ld_, (int)rb, dmatA(), ws(),
-                               ws_elems_, st_);
+      if (pass == 0 || !cross)
+        rcg::launch_gram<double>(n_, Y_, (int)ldy_, (int)rf, V(), (int)ld_, (int)rb, dmatA(), ws(),
+                                 ws_elems_, st_);
       if (cx_) rcg::launch_herm_embed(dmatA(), (int)found, (int)b, st_);
-      rcg::launch_tall_gemm<double>(n_, Y_, (int)ldy_, (int)rf, dmatA(), (int)rf, (int)rb, -1.0,
-                                    1.0, V(), V(), (int)ld_, st_);
+      if (pass == 0 && cross)
+        rcg::launch_tall_gemm_cross(n_, Y_, (int)ldy_, (int)rf, dmatA(), (int)rf, (int)rb, -1.0,
+                                    V(), V(), (int)ld_, dmatA(), ws(), ws_elems_, st_);
+      else if (pass == 1 && norms)
+        rcg::launch_tall_gemm_sums(n_, Y_, (int)ldy_, (int)rf, dmatA(), (int)rf, (int)rb, -1.0, 1.0,
+                                   V(), V(), (int)ld_, dsums(), ws(), ws_elems_, st_);
+      else
+        rcg::launch_tall_gemm<double>(n_, Y_, (int)ldy_, (int)rf, dmatA(), (int)rf, (int)rb, -1.0,
+                                      1.0, V(), V(), (int)ld_, st_);
     }
   }
 
-  void normalize(int64_t b) {
+  // Columns to unit norm; have_norms: dsums() holds their squared norms.
+  void normalize(int64_t b, bool have_norms = false) {
     const int64_t rb = cw_ * b;
-    rcg::launch_col_sumsq<double>(n_, V(), (int)ld_, (int)rb, dsums(), ws(), ws_elems_, st_);
+    if (!have_norms)
+      rcg::launch_col_sumsq<double>(n_, V(), (int)ld_, (int)rb, dsums(), ws(), ws_elems_, st_);
     if (cx_) rcg::launch_pair_sums(dsums(), (int)b, st_);
-    rcg::launch_normalize_cols<double>(n_, V(), (int)ld_, (int)rb, dsums(), st_);
+    rcg::launch_scale_cols(n_, V(), (int)ld_, (int)rb, dsums(), V(), st_);
   }
 
   // formVtAV (RayleighChebyshevLM.h:1928-1969): W = A V, H(j,i) = V_j^H W_i
@@ -1643,29 +1686,33 @@ class Engine {
       project<S>(b, H);
       return;
     }
-    if (!cholqr_pass<S>(b, true)) {
+    const int64_t rb = cw_ * b;
+    const char* unp = std::getenv("RCG_GRAM_UNPAIRED");
+    const bool apart = unp && unp[0] == '1';
+    const bool large = n_ * rb >= (int64_t(1) << 22);
+    if (!cholqr_pass<S>(b, true, large && !apart)) {
       cholqr_pass<S>(b, true);
       cholqr_pass<S>(b, false);
       project<S>(b, H);
       return;
     }
     apply(V(), W_, b);
-    const int64_t rb = cw_ * b;
-    // G = V^H V and H1 = V^H W right after it, so that one copy brings both
+    // G = V^H V and H1 = V^H W right after it, so that one wait brings both
     // back.  Below 2^22 block entries both products go in one paired launch
     // (the same values; plain solves of served-size requests 568 -> 586
-    // eigenpairs/s); above, the paired kernel's one wave per SIMD costs more
-    // than the launch it saves (128^3 x 64 solve 1987 -> 2003 ms).
-    // RCG_GRAM_UNPAIRED=1 always runs them separately.
-    const char* unp = std::getenv("RCG_GRAM_UNPAIRED");
-    if ((unp && unp[0] == '1') || n_ * rb >= (int64_t(1) << 22)) {
-      rcg::launch_gram<double>(n_, V(), (int)ld_, (int)rb, V(), (int)ld_, (int)rb, dres(), ws(),
-                               ws_elems_, st_);
-      rcg::launch_gram<double>(n_, V(), (int)ld_, (int)rb, W_, (int)ld_, (int)rb,
-                               dres() + rb * rb, ws(), ws_elems_, st_, true);
-    } else {
+    // eigenpairs/s); above, G comes with the product that wrote V (128^3 x 64: no
+    // pass of 0.27 ms of its own).  RCG_GRAM_UNPAIRED=1 runs the two products
+    // separately, with the paired launch's values.
+    if (!large && !apart) {
       rcg::launch_gram_pair(n_, V(), (int)ld_, W_, (int)ld_, (int)rb, dres(), ws(), ws_elems_,
                             st_);
+    } else {
+      if (!gram_ready_)
+        rcg::launch_gram<double>(n_, V(), (int)ld_, (int)rb, V(), (int)ld_, (int)rb, dres(), ws(),
+                                 ws_elems_, st_);
+      gram_ready_ = false;
+      rcg::launch_gram<double>(n_, V(), (int)ld_, (int)rb, W_, (int)ld_, (int)rb,
+                               dres() + rb * rb, ws(), ws_elems_, st_, true);
     }
     sync();
     std::vector<S> G(b * b), H1(b * b);
@@ -2008,6 +2055,7 @@ class Engine {
   hipEvent_t fev_[2] = {nullptr, nullptr};
   FilterBatcher* batcher_ = nullptr;
   hipEvent_t ev_done_ = nullptr;  // the batcher has run this engine's steps
+  bool gram_ready_ = false;  // dres() holds (or will) the real Gram matrix of V's columns
   bool timed_ = false;
   bool step_pending_ = false;
   long pend_launches_ = 0, step_launches_ = 0;
@@ -3339,8 +3387,8 @@ int rcg_deflate(rcg_block X, int64_t cols, rcg_block Y, int64_t found) {
     e.reserve(std::max(real_ld(X), real_ld(Y)), std::max(real_ld(X), real_ld(Y)));
     e.attach(static_cast<double*>(X->d()), nullptr, nullptr, real_ld(X),
              static_cast<double*>(Y->d()), real_ld(Y));
-    e.deflate(cols, found);
-    e.normalize(cols);
+    e.deflate(cols, found, true);
+    e.normalize(cols, found > 0);
     e.sync();
   });
 }
@@ -3372,9 +3420,8 @@ int rcg_rotate(rcg_block V, rcg_block tmp, int64_t cols, const double* Y_host) {
     check_block_pair(V, tmp, cols);
     DeviceGuard g(V->ctx->device);
     Piece pc(V, tmp, nullptr);
-    if (pc.eng.cx()) pc.eng.right_multiply(cols, reinterpret_cast<const cplx*>(Y_host));
-    else pc.eng.right_multiply(cols, Y_host);
-    pc.eng.normalize(cols);
+    if (pc.eng.cx()) pc.eng.rotate_normalized(cols, reinterpret_cast<const cplx*>(Y_host));
+    else pc.eng.rotate_normalized(cols, Y_host);
     pc.settle(V, cols);
   });
 }

@@ -251,6 +251,105 @@ __global__ __launch_bounds__(kThreads) void reduce_partials_kernel(const T* __re
   if (sl == 0 && o < m) out[o] = TO((red[0][ol] + red[1][ol]) + (red[2][ol] + red[3][ol]));
 }
 
+// The partial sums of a b x b Gram matrix (b <= B) and its Cholesky factor, in one
+// workgroup: G = R^T R of the matrix scaled to unit diagonal, C = D R^{-1} (b x b
+// column-major; V C is orthonormal), so that a CholQR pass needs no trip to the
+// host.  *clean = 1, or 0 where a pivot is not positive; C is then the identity.
+//
+// One wave factors, without a barrier: lane c < 32 holds column c of the trailing
+// matrix, lane 32 + c column c of M = R^{-T} (the same eliminations applied to the
+// identity), and row j reaches every lane by lane reads.  A version with the
+// matrix in LDS and three barriers per column took 13 us at 16 columns and 23 at
+// 24, more than the host's factor with its wait and copies (21).
+constexpr int kCholMax = 32;
+constexpr int kCholThreads = 1024;
+__device__ __forceinline__ double lane_of(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(b & 0xffffffffll), l);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
+// 1/sqrt(d), d > 0 and normal: the hardware's estimate and three Newton steps
+// (it sits in the factor's serial chain; sqrt and divide take four times as long)
+__device__ __forceinline__ double rsqrt_newton(double d) {
+  double r = __builtin_amdgcn_rsq(d);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) r = fma(r * 0.5, fma(-d * r, r, 1.0), r);
+  return r;
+}
+template <int B>
+__global__ __launch_bounds__(kCholThreads) void reduce_chol_kernel(const double* __restrict__ P,
+                                                                   int64_t nblk, int b,
+                                                                   double* __restrict__ C,
+                                                                   double* clean) {
+  constexpr int NO = (B * B + 255) / 256;  // outputs per thread
+  constexpr int NU = B <= 24 ? 8 : 4;      // partials of each in flight
+  __shared__ double part[4][NO * 256];
+  const int m = b * b;
+  {
+    const int t = threadIdx.x % 256;
+    const int sl = threadIdx.x / 256;
+    double s[NO];
+#pragma unroll
+    for (int k = 0; k < NO; ++k) s[k] = 0.0;
+    for (int64_t q = sl; q < nblk; q += 4 * NU) {
+      double x[NO][NU];
+#pragma unroll
+      for (int k = 0; k < NO; ++k)
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+          const int64_t blk = q + 4 * u;
+          x[k][u] = (blk < nblk && t + 256 * k < m) ? P[blk * m + t + 256 * k] : 0.0;
+        }
+#pragma unroll
+      for (int k = 0; k < NO; ++k)
+#pragma unroll
+        for (int u = 0; u < NU; ++u) s[k] += x[k][u];
+    }
+#pragma unroll
+    for (int k = 0; k < NO; ++k) part[sl][t + 256 * k] = s[k];
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x;
+  const bool right = lane >= 32;  // a column of M
+  const int c = lane & 31;
+  auto g = [&](int i, int k) {
+    const int e = i + k * b;
+    return (part[0][e] + part[1][e]) + (part[2][e] + part[3][e]);
+  };
+  double dg = 1.0;
+  if (c < b) {
+    const double d = g(c, c);
+    dg = (d > 0.0 && isfinite(d)) ? 1.0 / sqrt(d) : 1.0;
+  }
+  double a[B];
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    const double di = lane_of(dg, i);
+    a[i] = i == c ? 1.0 : 0.0;
+    if (!right && i < b && c < b) a[i] = g(i, c) * (di * dg);
+  }
+  bool ok = true;
+#pragma unroll
+  for (int j = 0; j < B; ++j) {
+    const double d = lane_of(a[j], j);
+    // unit diagonal before elimination: a pivot below 1e-200 is no pivot
+    const bool fine = d > 1e-200 && isfinite(d);
+    ok = ok && fine;
+    a[j] *= rsqrt_newton(fine ? d : 1.0);
+#pragma unroll
+    for (int i = j + 1; i < B; ++i) a[i] = fma(-lane_of(a[j], i), a[j], a[i]);
+  }
+  if (right && c < b) {
+    // R^{-1}[c][k] = M[k][c], zero below the diagonal
+#pragma unroll
+    for (int k = 0; k < B; ++k)
+      if (k < b) C[c + k * b] = ok ? (c <= k ? a[k] * dg : 0.0) : (c == k ? 1.0 : 0.0);
+  }
+  if (lane == 0) *clean = ok ? 1.0 : 0.0;
+}
+
 inline unsigned reduce_grid(int64_t m) { return (unsigned)((m + 63) / 64); }
 
 template <typename T>
@@ -2043,6 +2142,32 @@ void launch_gram(int64_t n, const T* X, int ldx, int bx, const T* Y, int ldy, in
   const int64_t m = (int64_t)bx * by;
   hipLaunchKernelGGL((reduce_partials_kernel<T, T>), dim3(reduce_grid(m)), dim3(kThreads), 0, st, ws,
                      nblk, m, G);
+  RCG_HIP(hipGetLastError());
+}
+
+// One workgroup reads all partials: up to 2^16 (0.5 MB) that is no slower than
+// the workgroups of a reduction of its own.
+bool chol_fits(int64_t n, int b) {
+  int64_t rpb;
+  return n > 0 && b >= 1 && b <= kCholMax && gram_blocks<double>(n, b, b, &rpb) * b * b <= 65536;
+}
+
+void launch_gram_chol(int64_t n, const double* X, int ldx, int b, double* C, double* clean,
+                      double* ws, size_t ws_elems, hipStream_t st) {
+  if (!chol_fits(n, b)) throw Error(1, "block too large for the device factor");
+  int64_t rpb;
+  const int64_t nblk = gram_blocks<double>(n, b, b, &rpb);
+  if ((size_t)nblk * b * b > ws_elems) throw Error(3, "gram workspace too small");
+  gram_one_tile<kGramDiag>(gram_nt(b, b), dim3((unsigned)round_up(nblk, kXcds)), st, n, X, ldx, b,
+                           X, ldx, b, ws, rpb, 1, 1, nblk);
+  RCG_HIP(hipGetLastError());
+#define RCG_CHOL(B)                                                                              \
+  hipLaunchKernelGGL(reduce_chol_kernel<B>, dim3(1), dim3(kCholThreads), 0, st, ws, nblk, b, C, \
+                     clean)
+  if (b <= 16) RCG_CHOL(16);
+  else if (b <= 24) RCG_CHOL(24);
+  else RCG_CHOL(32);
+#undef RCG_CHOL
   RCG_HIP(hipGetLastError());
 }
 

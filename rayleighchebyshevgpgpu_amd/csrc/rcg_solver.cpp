@@ -828,6 +828,9 @@ class Engine {
   double* hvecUp() { return ctx_->pinned.as<double>() + 2 * bb_ * bb_ + bb_; }
   double* hlz() { return ctx_->pinned.as<double>() + 2 * bb_ * bb_ + 3 * bb_; }
 
+  // where reduce_chol_kernel says whether its factor is sound (past the Grams)
+  size_t clean_at() const { return 2 * (size_t)(cw_ * bb_) * (size_t)(cw_ * bb_) + 4 * (size_t)(cw_ * bb_); }
+
   double* ws() { return ctx_->ws.as<double>(); }
 
   // Candidate row-block orders: contiguous blocks with and without the XCD
@@ -1677,6 +1680,27 @@ class Engine {
   // rotation (rotate_residuals), so the block is rotated once.  Wider blocks,
   // a first pass that needed a shift, or a G that does not factor take the
   // plain passes.
+  // W = A V1, then
+  // G = V^H V and H1 = V^H W right after it, so that one wait brings both
+  // back.  Below 2^22 block entries both products go in one paired launch
+  // (the same values; plain solves of served-size requests 568 -> 586
+  // eigenpairs/s); above, G comes with the product that wrote V (128^3 x 64: no
+  // pass of 0.27 ms of its own).  RCG_GRAM_UNPAIRED=1 runs the two products
+  // separately, with the paired launch's values.
+  void first_projection(int64_t b, int64_t rb, bool apart, bool large) {
+    apply(V(), W_, b);
+    if (!large && !apart) {
+      rcg::launch_gram_pair(n_, V(), (int)ld_, W_, (int)ld_, (int)rb, dres(), ws(), ws_elems_,
+                            st_);
+    } else {
+      if (!gram_ready_)
+        rcg::launch_gram<double>(n_, V(), (int)ld_, (int)rb, V(), (int)ld_, (int)rb, dres(), ws(),
+                                 ws_elems_, st_);
+      gram_ready_ = false;
+      rcg::launch_gram<double>(n_, V(), (int)ld_, (int)rb, W_, (int)ld_, (int)rb,
+                               dres() + rb * rb, ws(), ws_elems_, st_, true);
+    }
+  }
   template <class S>
   void ortho_project(int64_t b, std::vector<S>& H) {
     fold_b_ = 0;
@@ -1690,31 +1714,33 @@ class Engine {
     const char* unp = std::getenv("RCG_GRAM_UNPAIRED");
     const bool apart = unp && unp[0] == '1';
     const bool large = n_ * rb >= (int64_t(1) << 22);
-    if (!cholqr_pass<S>(b, true, large && !apart)) {
-      cholqr_pass<S>(b, true);
-      cholqr_pass<S>(b, false);
-      project<S>(b, H);
-      return;
-    }
-    apply(V(), W_, b);
-    // G = V^H V and H1 = V^H W right after it, so that one wait brings both
-    // back.  Below 2^22 block entries both products go in one paired launch
-    // (the same values; plain solves of served-size requests 568 -> 586
-    // eigenpairs/s); above, G comes with the product that wrote V (128^3 x 64: no
-    // pass of 0.27 ms of its own).  RCG_GRAM_UNPAIRED=1 runs the two products
-    // separately, with the paired launch's values.
-    if (!large && !apart) {
-      rcg::launch_gram_pair(n_, V(), (int)ld_, W_, (int)ld_, (int)rb, dres(), ws(), ws_elems_,
-                            st_);
-    } else {
-      if (!gram_ready_)
-        rcg::launch_gram<double>(n_, V(), (int)ld_, (int)rb, V(), (int)ld_, (int)rb, dres(), ws(),
-                                 ws_elems_, st_);
+    // the first pass's factor on the device, without a trip to the host; taken
+    // back (the old block is in T) if the Gram matrix turns out not to factor
+    bool on_device = !cx_ && !large && rcg::chol_fits(n_, (int)b);
+    if (on_device) {
       gram_ready_ = false;
-      rcg::launch_gram<double>(n_, V(), (int)ld_, (int)rb, W_, (int)ld_, (int)rb,
-                               dres() + rb * rb, ws(), ws_elems_, st_, true);
+      rcg::launch_gram_chol(n_, V(), (int)ld_, (int)b, dmatA(), dres() + clean_at(), ws(),
+                            ws_elems_, st_);
+      rcg::launch_tall_gemm<double>(n_, V(), (int)ld_, (int)b, dmatA(), (int)b, (int)b, 1.0, 0.0,
+                                    nullptr, T(), (int)ld_, st_);
+      swapVT();
+      first_projection(b, rb, apart, large);
+      sync();
+      if (hres()[clean_at()] == 0.0) {
+        swapVT();
+        on_device = false;
+      }
     }
-    sync();
+    if (!on_device) {
+      if (!cholqr_pass<S>(b, true, large && !apart)) {
+        cholqr_pass<S>(b, true);
+        cholqr_pass<S>(b, false);
+        project<S>(b, H);
+        return;
+      }
+      first_projection(b, rb, apart, large);
+      sync();
+    }
     std::vector<S> G(b * b), H1(b * b);
     combine_gram<S>(hres(), b, b, G.data());
     combine_gram<S>(hres() + rb * rb, b, b, H1.data());

@@ -250,7 +250,8 @@ void launch_gram(int64_t n, const T* X, int ldx, int bx, const T* Y, int ldy, in
 void launch_gram_pair(int64_t n, const double* X, int ldx, const double* Y, int ldy, int b,
                       double* G, double* ws, size_t ws_elems, hipStream_t st);
 // The CholQR factor C = D R^{-1} (b x b) of X's columns on the device (see
-// reduce_chol_kernel); *clean = 0 where the Gram matrix is not positive definite.
+// reduce_chol_kernel); *clean = the smallest pivot of the Gram matrix scaled to
+// unit diagonal, 0 where it is not positive definite.
 bool chol_fits(int64_t n, int b);
 void launch_gram_chol(int64_t n, const double* X, int ldx, int b, double* C, double* clean,
                       double* ws, size_t ws_elems, hipStream_t st);
@@ -304,6 +305,11 @@ struct ThetaArgs {
 #endif
   double operator[](int c) const { return v[c]; }
 };
+// out = V C (b <= 64 columns, all with ld) and sums as below for its first nc
+// columns with W C in the place of A out (W = A V).
+void launch_tall_resid(int64_t n, const double* V, const double* W, int ld, int b, const double* C,
+                       double* out, const ThetaArgs& theta, int nc, double* sums, double* ws,
+                       size_t ws_elems, hipStream_t st);
 void launch_resid_norm_sumsq_args(int64_t n, const double* V, const double* W, int ld, int nc,
                                   const ThetaArgs& theta, double* sums, double* ws,
                                   size_t ws_elems, hipStream_t st);

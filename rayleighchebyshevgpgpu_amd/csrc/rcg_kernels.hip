@@ -254,7 +254,8 @@ __global__ __launch_bounds__(kThreads) void reduce_partials_kernel(const T* __re
 // The partial sums of a b x b Gram matrix (b <= B) and its Cholesky factor, in one
 // workgroup: G = R^T R of the matrix scaled to unit diagonal, C = D R^{-1} (b x b
 // column-major; V C is orthonormal), so that a CholQR pass needs no trip to the
-// host.  *clean = 1, or 0 where a pivot is not positive; C is then the identity.
+// host.  *clean = the smallest pivot, or 0 where one is not positive; C is then
+// the identity.
 //
 // One wave factors, without a barrier: lane c < 32 holds column c of the trailing
 // matrix, lane 32 + c column c of M = R^{-T} (the same eliminations applied to the
@@ -331,12 +332,14 @@ __global__ __launch_bounds__(kCholThreads) void reduce_chol_kernel(const double*
     if (!right && i < b && c < b) a[i] = g(i, c) * (di * dg);
   }
   bool ok = true;
+  double least = 1.0;
 #pragma unroll
   for (int j = 0; j < B; ++j) {
     const double d = lane_of(a[j], j);
     // unit diagonal before elimination: a pivot below 1e-200 is no pivot
     const bool fine = d > 1e-200 && isfinite(d);
     ok = ok && fine;
+    least = fmin(least, d);
     a[j] *= rsqrt_newton(fine ? d : 1.0);
 #pragma unroll
     for (int i = j + 1; i < B; ++i) a[i] = fma(-lane_of(a[j], i), a[j], a[i]);
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(kCholThreads) void reduce_chol_kernel(const double*
     for (int k = 0; k < B; ++k)
       if (k < b) C[c + k * b] = ok ? (c <= k ? a[k] * dg : 0.0) : (c == k ? 1.0 : 0.0);
   }
-  if (lane == 0) *clean = ok ? 1.0 : 0.0;
+  if (lane == 0) *clean = ok ? least : 0.0;
 }
 
 inline unsigned reduce_grid(int64_t m) { return (unsigned)((m + 63) / 64); }
@@ -835,6 +838,7 @@ __global__ __launch_bounds__(kThreads) void tall_gemm_mfma_kernel(
   }
   for (int64_t tile = stripe; tile < ntiles; tile += nstripe) {
     const int64_t row = tile * kTile + wave * 16 + r;
+    int zero = 0;
     d4v acc[NTC];
 #pragma unroll
     for (int t = 0; t < NTC; ++t) acc[t] = d4v{0.0, 0.0, 0.0, 0.0};
@@ -861,12 +865,14 @@ __global__ __launch_bounds__(kThreads) void tall_gemm_mfma_kernel(
       }
 #pragma unroll
       for (int sidx = 0; sidx < 16; ++sidx) {
+        // as in tall_resid_kernel, where a Gram matrix needs the registers
+        if (AFTER >= kTallGram && sidx % 4 == 0) asm volatile("" : "+s"(zero));
         // step sidx contracts k0 + sidx + {0, 16, 32, 48}: none is a column of X
         // once k0 + sidx >= bx (uniform)
         if (NTC == 4 || k0 + sidx < bx) {
           const int k = 16 * kk + sidx;
 #pragma unroll
-          for (int t = 0; t < NTC; ++t) acc[t] = mfma16x16x4(xa[sidx], cs[k][16 * t + r], acc[t]);
+          for (int t = 0; t < NTC; ++t) acc[t] = mfma16x16x4(xa[sidx], cs[k][16 * t + r + zero], acc[t]);
         }
       }
     }
@@ -970,6 +976,127 @@ __global__ __launch_bounds__(kThreads) void tall_gemm_mfma_kernel(
                                       ? red[b + kTile * a]
                                       : red[a + kTile * b];
     }
+  }
+}
+
+// out = V C and, for its first nc columns, the sums of |theta_c out_c - (W C)_c|^2
+// and |out_c|^2 (V, W: n x b, C: b x b column-major, b <= 64): the Ritz rotation
+// and its residuals in one pass.  With W = A V, W C is A out, so the operator is
+// not applied again: reads V and W and writes out, against a product, an apply and
+// a pass over both results (128^3 x 64, 32 residuals: 0.42 + 0.46 + 0.18 ms -> 0.61;
+// n = 17576, 24 columns: 10 + 6 + 6 us -> 14).  Lanes and
+// fragments as in tall_gemm_mfma_kernel, C feeding both products.  NTC, NTR: 16-column
+// subtiles of out and of its residual columns (constants: a branch on nc between
+// the MFMAs made the accumulators spill, 1.43 ms).
+template <int NTC, int NTR>
+__global__ __launch_bounds__(kThreads, 2) void tall_resid_kernel(
+    int64_t n, const double* __restrict__ V, const double* __restrict__ W, int ld, int b,
+    const double* __restrict__ C, double* __restrict__ out, const ThetaArgs theta, int nc,
+    int64_t ntiles, int64_t nstripe, double* __restrict__ P) {
+  __shared__ double cs[kTile][kTile + 1];  // [k][c]
+  const int64_t stripe = xcd_remap(blockIdx.x, gridDim.x);
+  if (stripe >= nstripe) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int kk = lane >> 4;
+  const int r = lane & 15;
+  const bool vec_ok = ld % 2 == 0 && ((reinterpret_cast<uintptr_t>(V) & 15) == 0) &&
+                      ((reinterpret_cast<uintptr_t>(W) & 15) == 0);
+  for (int e = threadIdx.x; e < kTile * kTile; e += kThreads) {
+    const int k = e % kTile;
+    const int c = e / kTile;
+    cs[k][c] = (k < b && c < b) ? C[k + (int64_t)c * b] : 0.0;
+  }
+  double th[NTR], res[NTR], nrm[NTR];
+#pragma unroll
+  for (int t = 0; t < NTR; ++t) {
+    th[t] = 16 * t + r < nc ? theta.v[16 * t + r] : 0.0;
+    res[t] = nrm[t] = 0.0;
+  }
+  __syncthreads();
+  for (int64_t tile = stripe; tile < ntiles; tile += nstripe) {
+    const int64_t row = tile * kTile + wave * 16 + r;
+    double xa[16], wa[16];
+    const int kb = 16 * kk;
+    if (row < n && kb + 16 <= b && vec_ok) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const dvec2 x = *reinterpret_cast<const dvec2*>(V + row * ld + kb + 2 * q);
+        const dvec2 w = *reinterpret_cast<const dvec2*>(W + row * ld + kb + 2 * q);
+        xa[2 * q] = x.x;
+        xa[2 * q + 1] = x.y;
+        wa[2 * q] = w.x;
+        wa[2 * q + 1] = w.y;
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const bool in = row < n && kb + q < b;
+        xa[q] = in ? V[row * ld + kb + q] : 0.0;
+        wa[q] = in ? W[row * ld + kb + q] : 0.0;
+      }
+    }
+    int zero = 0;
+    d4v av[NTC], aw[NTR];
+#pragma unroll
+    for (int t = 0; t < NTC; ++t) av[t] = d4v{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < NTR; ++t) aw[t] = d4v{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int sidx = 0; sidx < 16; ++sidx) {
+      // C's fragments are read from LDS four steps at a time (an offset of zero
+      // that the compiler cannot see through): held in registers for all steps, or
+      // over the tiles, as it would, they spill
+      if (sidx % 4 == 0) asm volatile("" : "+s"(zero));
+      // step sidx contracts sidx + {0, 16, 32, 48}: none below b once sidx >= b
+      if (NTC == 4 || sidx < b) {
+#pragma unroll
+        for (int t = 0; t < NTC; ++t) {
+          const double f = cs[16 * kk + sidx][16 * t + r + zero];
+          av[t] = mfma16x16x4(xa[sidx], f, av[t]);
+          if (t < NTR) aw[t < NTR ? t : 0] = mfma16x16x4(wa[sidx], f, aw[t < NTR ? t : 0]);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t ro = tile * kTile + wave * 16 + 4 * j + kk;
+#pragma unroll
+      for (int t = 0; t < NTC; ++t) {
+        const double v = av[t][j];
+        if (ro < n && 16 * t + r < b) out[ro * ld + 16 * t + r] = v;
+        if (t < NTR) {  // zero in rows past n
+          constexpr int last = NTR - 1;
+          const int u = t < NTR ? t : last;
+          const double d = th[u] * v - aw[u][j];
+          res[u] = fma(d, d, res[u]);
+          nrm[u] = fma(v, v, nrm[u]);
+        }
+      }
+    }
+  }
+  // over the 4 row groups of a wave, then the waves in order
+#pragma unroll
+  for (int t = 0; t < NTR; ++t) {
+    res[t] += __shfl_xor(res[t], 16);
+    res[t] += __shfl_xor(res[t], 32);
+    nrm[t] += __shfl_xor(nrm[t], 16);
+    nrm[t] += __shfl_xor(nrm[t], 32);
+  }
+  __syncthreads();  // C is no longer read
+  double* red = &cs[0][0];
+  if (kk == 0) {
+#pragma unroll
+    for (int t = 0; t < NTR; ++t) {
+      red[(2 * wave) * kTile + 16 * t + r] = res[t];
+      red[(2 * wave + 1) * kTile + 16 * t + r] = nrm[t];
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < 2 * nc; e += kThreads) {
+    const int c = e % nc, h = e / nc;  // h: 0 residuals, 1 norms
+    P[stripe * 2 * nc + e] = ((red[h * kTile + c] + red[(2 + h) * kTile + c]) +
+                              red[(4 + h) * kTile + c]) + red[(6 + h) * kTile + c];
   }
 }
 
@@ -2318,6 +2445,38 @@ void launch_tall_gemm_sums(int64_t n, const double* X, int ldx, int bx, const do
   if (wide) tall_wide<true>(n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, ws, st);
   else tall_narrow<kTallSums>(n, X, ldx, bx, C, ldc, by, alpha, beta, Z, out, ldo, ws, st);
   reduce_to(ws, nblk, by, sums, st);
+}
+
+void launch_tall_resid(int64_t n, const double* V, const double* W, int ld, int b, const double* C,
+                       double* out, const ThetaArgs& theta, int nc, double* sums, double* ws,
+                       size_t ws_elems, hipStream_t st) {
+  if (n <= 0 || b <= 0 || nc <= 0) throw Error(1, "residuals of an empty block");
+  if (b > kTile || nc > b) throw Error(1, "fused residuals take at most 64 columns");
+  const int64_t nrb = (n + kTile - 1) / kTile;
+  const int64_t nblk = std::min<int64_t>(nrb, 512);  // two workgroups per CU
+  if ((size_t)(nblk * 2 * nc) > ws_elems) throw Error(3, "column-sum workspace too small");
+  const dim3 grid((unsigned)round_up(nblk, kXcds));
+  // 16-column subtiles of the block and of its residual columns
+#define RCG_RESID(N, R)                                                                            \
+  case 10 * N + R:                                                                                 \
+    hipLaunchKernelGGL((tall_resid_kernel<N, R>), grid, dim3(kThreads), 0, st, n, V, W, ld, b, C,  \
+                       out, theta, nc, nrb, nblk, ws);                                             \
+    break;
+  switch (10 * ((b + 15) / 16) + (nc + 15) / 16) {
+    RCG_RESID(1, 1)
+    RCG_RESID(2, 1)
+    RCG_RESID(2, 2)
+    RCG_RESID(3, 1)
+    RCG_RESID(3, 2)
+    RCG_RESID(3, 3)
+    RCG_RESID(4, 1)
+    RCG_RESID(4, 2)
+    RCG_RESID(4, 3)
+    RCG_RESID(4, 4)
+  }
+#undef RCG_RESID
+  RCG_HIP(hipGetLastError());
+  reduce_to(ws, nblk, 2 * nc, sums, st);
 }
 
 void launch_tall_gemm_gram(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc,

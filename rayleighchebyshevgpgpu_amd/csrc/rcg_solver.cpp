@@ -1553,6 +1553,24 @@ class Engine {
     rcg::launch_scale_cols(n_, T(), (int)ld_, (int)rb, dsums(), V(), st_);
   }
 
+  // G <- D G D with a unit diagonal, D in d
+  template <class S>
+  static void unit_diagonal(int64_t b, std::vector<S>& G, std::vector<double>& d) {
+    for (int64_t j = 0; j < b; ++j) {
+      const double g = std::real(G[j + j * b]);
+      d[j] = (g > 0.0 && std::isfinite(g)) ? 1.0 / std::sqrt(g) : 1.0;
+    }
+    for (int64_t j = 0; j < b; ++j)
+      for (int64_t i = 0; i < b; ++i) G[i + j * b] *= d[i] * d[j];
+  }
+  // the smallest pivot of the factorisation that gave R
+  template <class S>
+  static double least_pivot(int64_t b, const std::vector<S>& R) {
+    double p = 1.0;
+    for (int64_t j = 0; j < b; ++j) p = std::min(p, std::norm(R[j + j * b]));
+    return p;
+  }
+
   // One CholQR pass on V[:, :b]: G = V^H V scaled to unit diagonal,
   // G = R^H R, V <- V D R^{-1}.  A failed factorisation retries with the
   // shift 11(nb + b(b+1)) u ||G|| (shifted CholeskyQR); returns false then.
@@ -1562,14 +1580,10 @@ class Engine {
     std::vector<S> G(b * b);
     gram_to_host<S>(V(), ld_, b, V(), ld_, b, G.data());
     std::vector<double> d(b);
-    for (int64_t j = 0; j < b; ++j) {
-      const double g = std::real(G[j + j * b]);
-      d[j] = (g > 0.0 && std::isfinite(g)) ? 1.0 / std::sqrt(g) : 1.0;
-    }
-    for (int64_t j = 0; j < b; ++j)
-      for (int64_t i = 0; i < b; ++i) G[i + j * b] *= d[i] * d[j];
+    unit_diagonal(b, G, d);
     std::vector<S> R, Ri;
     bool clean = rcg::dense::cholesky_upper(G.data(), b, R);
+    one_pass_ = clean && least_pivot(b, R) >= kOnePass;
     if (!clean) {
       if (!allow_shift) throw Error(RCG_ERR_NUMERIC, "CholQR breakdown after a shifted pass");
       double gn = 0.0;
@@ -1590,9 +1604,11 @@ class Engine {
   // pass when the first needed a shift.
   void orthonormalize(int64_t b) {
     fold_b_ = 0;
+
     if (b <= 0) return;
-    if (cx_) return orthonormalize_t<cplx>(b);
-    orthonormalize_t<double>(b);
+    if (cx_) orthonormalize_t<cplx>(b);
+    else orthonormalize_t<double>(b);
+    one_pass_ = false;
   }
   template <class S>
   void orthonormalize_t(int64_t b) {
@@ -1680,7 +1696,15 @@ class Engine {
   // rotation (rotate_residuals), so the block is rotated once.  Wider blocks,
   // a first pass that needed a shift, or a G that does not factor take the
   // plain passes.
-  // W = A V1, then
+  //
+  // Once the filter acts on Ritz vectors its output is nearly orthogonal, and
+  // the first pass does nothing that the second cannot: where the last Gram
+  // matrix, scaled to unit diagonal, had no pivot below 1/2 (R's condition is then
+  // a small number and one pass loses a few ulps), the projection starts from
+  // the block as it is and the first pass is skipped.  The Gram matrix that comes
+  // with it must meet the same bound; if not, the first pass runs after all.
+  static constexpr double kOnePass = 0.5;
+  // W = A V, then
   // G = V^H V and H1 = V^H W right after it, so that one wait brings both
   // back.  Below 2^22 block entries both products go in one paired launch
   // (the same values; plain solves of served-size requests 568 -> 586
@@ -1714,9 +1738,22 @@ class Engine {
     const char* unp = std::getenv("RCG_GRAM_UNPAIRED");
     const bool apart = unp && unp[0] == '1';
     const bool large = n_ * rb >= (int64_t(1) << 22);
+    std::vector<S> G(b * b), H1(b * b), R, Ri;
+    std::vector<double> scale(b, 1.0);
+    bool one_pass = one_pass_;
+    if (one_pass) {
+      gram_ready_ = false;
+      first_projection(b, rb, apart, large);
+      sync();
+      combine_gram<S>(hres(), b, b, G.data());
+      unit_diagonal(b, G, scale);
+      one_pass = rcg::dense::cholesky_upper(G.data(), b, R) && least_pivot(b, R) >= kOnePass;
+      if (!one_pass) std::fill(scale.begin(), scale.end(), 1.0);
+      one_pass_ = one_pass;
+    }
     // the first pass's factor on the device, without a trip to the host; taken
     // back (the old block is in T) if the Gram matrix turns out not to factor
-    bool on_device = !cx_ && !large && rcg::chol_fits(n_, (int)b);
+    bool on_device = !one_pass && !cx_ && !large && rcg::chol_fits(n_, (int)b);
     if (on_device) {
       gram_ready_ = false;
       rcg::launch_gram_chol(n_, V(), (int)ld_, (int)b, dmatA(), dres() + clean_at(), ws(),
@@ -1726,12 +1763,13 @@ class Engine {
       swapVT();
       first_projection(b, rb, apart, large);
       sync();
+      one_pass_ = hres()[clean_at()] >= kOnePass;
       if (hres()[clean_at()] == 0.0) {
         swapVT();
         on_device = false;
       }
     }
-    if (!on_device) {
+    if (!one_pass && !on_device) {
       if (!cholqr_pass<S>(b, true, large && !apart)) {
         cholqr_pass<S>(b, true);
         cholqr_pass<S>(b, false);
@@ -1741,17 +1779,17 @@ class Engine {
       first_projection(b, rb, apart, large);
       sync();
     }
-    std::vector<S> G(b * b), H1(b * b);
-    combine_gram<S>(hres(), b, b, G.data());
     combine_gram<S>(hres() + rb * rb, b, b, H1.data());
-    std::vector<S> R, Ri;
-    if (!rcg::dense::cholesky_upper(G.data(), b, R)) {
+    if (!one_pass) combine_gram<S>(hres(), b, b, G.data());
+    if (!one_pass && !rcg::dense::cholesky_upper(G.data(), b, R)) {
       // V1 is left as it is: the plain second (and third) pass, then project
       if (!cholqr_pass<S>(b, true)) cholqr_pass<S>(b, false);
       project<S>(b, H);
       return;
     }
     rcg::dense::upper_inverse(R, b, Ri);
+    for (int64_t j = 0; j < b; ++j)
+      for (int64_t i = 0; i <= j; ++i) Ri[i + j * b] *= scale[i];
     for (int64_t i = 0; i < b; ++i) {
       H1[i + i * b] = std::real(H1[i + i * b]);
       for (int64_t j = i + 1; j < b; ++j) H1[i + j * b] = conj_s(H1[j + i * b]);
@@ -1788,7 +1826,9 @@ class Engine {
   // round-off; the residuals are divided by the computed norms instead of
   // rescaling the block (the filter is linear and CholQR normalises), and the
   // columns handed out as eigenvectors are scaled at lock time.
-  // After ortho_project the block is V1 and the rotation is R^{-1} Y.
+  // After ortho_project the block is V1, W = A V1 and the rotation is C = R^{-1} Y:
+  // A (V1 C) is W C, so one pass over V1 and W gives the rotated block and its
+  // residuals without another product with A.
   template <class S>
   void rotate_residuals(int64_t b, const std::vector<S>& Yh, const std::vector<double>& th,
                         int64_t count, std::vector<double>& res) {
@@ -1801,6 +1841,18 @@ class Engine {
           for (int64_t i = 0; i <= k; ++i) C[i + j * b] += Ri[i + k * b] * y;
         }
       fold_b_ = 0;
+      if (count > 0) {
+        const int64_t rc = cw_ * count;
+        upload_factor<S>(b, C.data());
+        rcg::ThetaArgs ta{};
+        for (int64_t c = 0; c < rc; ++c) ta.v[c] = th[c / cw_];
+        rcg::launch_tall_resid(n_, V(), W_, (int)ld_, (int)(cw_ * b), dmatA(), T(), ta, (int)rc,
+                               dres(), ws(), ws_elems_, st_);
+        swapVT();
+        gram_ready_ = false;
+        take_residuals(count, res);
+        return;
+      }
       right_multiply<S>(b, C.data());
     } else {
       fold_b_ = 0;
@@ -1828,8 +1880,14 @@ class Engine {
       rcg::launch_resid_norm_sumsq<double>(n_, V(), W_, (int)ld_, (int)rc, dtheta(), dres(), ws(),
                                            ws_elems_, st_);
     }
+    take_residuals(count, res);
+  }
+  // The residual norms and column norms from the sums in dres().
+  void take_residuals(int64_t count, std::vector<double>& res) {
+    const int64_t rc = cw_ * count;
     sync();
     const double* sums = hres();
+    res.assign(count, 0.0);
     last_norms_.assign(count, 1.0);
     for (int64_t c = 0; c < count; ++c) {
       double t = 0.0, q = 0.0;
@@ -2081,6 +2139,7 @@ class Engine {
   hipEvent_t fev_[2] = {nullptr, nullptr};
   FilterBatcher* batcher_ = nullptr;
   hipEvent_t ev_done_ = nullptr;  // the batcher has run this engine's steps
+  bool one_pass_ = false;    // the last scaled Gram matrix had no pivot below kOnePass
   bool gram_ready_ = false;  // dres() holds (or will) the real Gram matrix of V's columns
   bool timed_ = false;
   bool step_pending_ = false;

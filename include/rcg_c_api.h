@@ -294,13 +294,14 @@ typedef struct rcg_solve_result {
   int64_t filter_degree_sum; /* Chebyshev step launches (sum of starDegree * rep) */
   double t_total;            /* host wall seconds of the solve */
   double t_lanczos, t_filter, t_ortho, t_rr; /* seconds of the solve's stream per phase,
-                                from hipEvents recorded where each phase begins (so a
+                                from hipEvents recorded where each phase begins, or the
+                                host's clock where the stream is empty there (so a
                                 phase includes the stream's idle time while the host
                                 works inside it); t_ortho: start vectors, CholQR and
                                 deflation; t_rr: the projection with its CholQR passes,
                                 the small eigensolve, rotation, residuals and the final
                                 refinement */
-  double t_filter_device;    /* seconds between hipEvents around the Chebyshev step
+  double t_filter_device;    /* seconds between such marks around the Chebyshev step
                                 launches (FP64 steps, or the FP32 correction steps) */
   double filter_bytes;       /* algorithmic bytes of those steps: CSR + 3 block passes
                                 (FP64) or CSR(FP32 values) + 4 FP32 block passes */

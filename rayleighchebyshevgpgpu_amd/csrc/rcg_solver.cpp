@@ -741,6 +741,93 @@ class FilterBatcher {
   int64_t launches_ = 0, timed_ = 0;
 };
 
+// Stream time per phase of a solve: a phase's time runs from the mark where it
+// begins to the next mark, so it includes the stream's idle time while the host
+// works inside it (the small eigensolve counts to Rayleigh-Ritz, a served solve's
+// wait for its shared filter batch to the filter).  Where the stream is known to
+// be empty, after a wait, a mark is the host's time; elsewhere it is an event,
+// put on the host's time axis by an event recorded when the clock was made.  An
+// event costs the stream 3-5 us, a tenth of a small solve's iteration when every
+// phase and every run of steps took one.  Finished intervals are folded whenever
+// a new phase begins; the solve's host waits keep the list of pending marks short.
+class PhaseClock {
+ public:
+  // kSteps: the Chebyshev step launches inside the filter
+  enum { kLanczos = 0, kFilter, kSteps, kOrtho, kRR, kOther, kCount };
+  explicit PhaseClock(hipStream_t st) : st_(st) {
+    RCG_HIP(hipEventCreate(&zero_));
+    RCG_HIP(hipEventRecord(zero_, st_));
+    RCG_HIP(hipEventSynchronize(zero_));
+    zero_at_ = wall();
+  }
+  PhaseClock(const PhaseClock&) = delete;
+  PhaseClock& operator=(const PhaseClock&) = delete;
+  ~PhaseClock() {
+    for (const Mark& m : marks_)
+      if (m.ev) (void)hipEventDestroy(m.ev);
+    for (hipEvent_t e : pool_) (void)hipEventDestroy(e);
+    (void)hipEventDestroy(zero_);
+  }
+  void mark(int phase, bool idle = false) {
+    fold(false);
+    hipEvent_t e = nullptr;
+    if (!idle) {
+      if (!pool_.empty()) {
+        e = pool_.back();
+        pool_.pop_back();
+      } else {
+        RCG_HIP(hipEventCreate(&e));
+      }
+      RCG_HIP(hipEventRecord(e, st_));
+    }
+    marks_.push_back({e, phase, wall()});
+  }
+  // closes the last phase and folds every interval (waits for the stream)
+  void finish() {
+    mark(kOther);
+    wait_event(marks_.back().ev, true);
+    fold(true);
+  }
+  double seconds(int phase) const { return sec_[phase]; }
+
+ private:
+  struct Mark {
+    hipEvent_t ev;  // null: `at` is the mark's time
+    int phase;
+    double at;
+  };
+  // the mark's time, taken from its event once that has passed
+  bool known(Mark& m, bool done) {
+    if (!m.ev) return true;
+    if (!done) {
+      const hipError_t r = hipEventQuery(m.ev);
+      if (r != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
+    }
+    float ms = 0.f;
+    RCG_HIP(hipEventElapsedTime(&ms, zero_, m.ev));
+    m.at = zero_at_ + 1.0e-3 * ms;
+    pool_.push_back(m.ev);
+    m.ev = nullptr;
+    return true;
+  }
+  void fold(bool done) {
+    while (marks_.size() >= 2) {
+      if (!known(marks_[0], done) || !known(marks_[1], done)) break;
+      sec_[marks_[0].phase] += std::max(0.0, marks_[1].at - marks_[0].at);
+      marks_.pop_front();
+    }
+  }
+  hipStream_t st_;
+  hipEvent_t zero_ = nullptr;
+  double zero_at_ = 0.0;
+  std::deque<Mark> marks_;
+  std::vector<hipEvent_t> pool_;
+  double sec_[kCount] = {};
+};
+
 // ------------------------------------------------------------------ engine
 // Device operations of the solve over attached row-interleaved buffers:
 // V (the subspace, ld), T (second recurrence / rotation buffer, ld),
@@ -809,6 +896,7 @@ class Engine {
     } else {
       RCG_HIP(hipStreamSynchronize(st_));
     }
+    coef_busy_ = false;
   }
 
   // Scratch layout (device `small` and host `pinned` alike):
@@ -1284,8 +1372,8 @@ class Engine {
     const size_t nd = 2 * (size_t)rb + (size_t)ld_;
     const size_t bytes = sizeof(double) * nd + sizeof(float) * (size_t)(m + 1) * (size_t)ld_;
     // the pinned table of the previous call is no longer in flight
-    if (coef_ev_) wait_event(coef_ev_, ctx_->blocking_ev != nullptr);
-    else RCG_HIP(hipEventCreateWithFlags(&coef_ev_, hipEventDisableTiming));
+    if (coef_busy_) sync();
+    idle_ = false;
     coef_.ensure(bytes);
     hcoef_.ensure(bytes);
     double* hd = hcoef_.as<double>();
@@ -1307,7 +1395,7 @@ class Engine {
       hd[2 * rb + col] = u1;  // u_m
     }
     RCG_HIP(hipMemcpyAsync(coef_.p, hcoef_.p, bytes, hipMemcpyHostToDevice, st_));
-    RCG_HIP(hipEventRecord(coef_ev_, st_));
+    coef_busy_ = true;
     const double* dcp = coef_.as<double>();
     const double* dum = dcp + 2 * rb;
     const float* dk = reinterpret_cast<const float*>(dcp + nd);
@@ -1411,7 +1499,7 @@ class Engine {
         }
         std::swap(X0, X1);
       }
-      step_end();
+      step_end(dn || !fused);
       if (dn || !fused)
         rcg::launch_mixed_combine(n_, V(), (int)ld_, (int)rb, dum, end.s_end, X1, st_);
     }
@@ -1434,45 +1522,27 @@ class Engine {
     return op_->val32.as<float>();
   }
 
-  // Device time of the Chebyshev step launches (hipEvents around each run
-  // of steps), their count and algorithmic bytes; read once the stream has
-  // passed the end event.
-  // Solves read them; the piecewise entry points do not and skip the events.
-  void time_steps() { timed_ = true; }
+  // Each run of Chebyshev step launches is a phase of the solve's clock, their
+  // count and algorithmic bytes are added up.  The piecewise entry points have no
+  // clock.  more: the filter goes on after the steps (else the solve's next
+  // phase ends them).
+  void set_clock(PhaseClock* c) { clock_ = c; }
+  // the stream is empty (the host has waited for it): the next step_begin needs
+  // no event if nothing was launched before it
+  void set_idle() { idle_ = true; }
   void step_begin(long launches, double bytes) {
-    if (!timed_) return;
-    if (!fev_[0]) {
-      RCG_HIP(hipEventCreate(&fev_[0]));
-      RCG_HIP(hipEventCreate(&fev_[1]));
-    }
-    collect_step_time();
-    RCG_HIP(hipEventRecord(fev_[0], st_));
-    pend_launches_ = launches;
-    pend_bytes_ = bytes;
+    if (clock_) clock_->mark(PhaseClock::kSteps, idle_);
+    idle_ = false;
+    step_launches_ += launches;
+    step_bytes_ += bytes;
   }
-  void step_end() {
-    if (!timed_) return;
-    RCG_HIP(hipEventRecord(fev_[1], st_));
-    step_pending_ = true;
+  void step_end(bool more = false) {
+    if (clock_ && more) clock_->mark(PhaseClock::kFilter);
   }
-  void collect_step_time() {
-    if (!step_pending_) return;
-    RCG_HIP(hipEventSynchronize(fev_[1]));
-    float ms = 0.f;
-    RCG_HIP(hipEventElapsedTime(&ms, fev_[0], fev_[1]));
-    step_seconds_ += 1.0e-3 * ms;
-    step_launches_ += pend_launches_;
-    step_bytes_ += pend_bytes_;
-    step_pending_ = false;
-  }
-  double step_seconds() { collect_step_time(); return step_seconds_; }
-  double step_bytes() { collect_step_time(); return step_bytes_; }
-  long step_launches() { collect_step_time(); return step_launches_; }
+  double step_bytes() const { return step_bytes_; }
+  long step_launches() const { return step_launches_; }
   ~Engine() {
-    for (auto& e : fev_)
-      if (e) (void)hipEventDestroy(e);
     if (ev_done_) (void)hipEventDestroy(ev_done_);
-    if (coef_ev_) (void)hipEventDestroy(coef_ev_);
   }
   int last_panel() const { return last_panel_; }
   const std::string& last_sched() const { return last_sched_; }
@@ -2134,86 +2204,21 @@ class Engine {
   }
   DevBuf coef_;                       // mixed filter coefficient table
   DevBuf cb_in_, cb_out_;             // column-major blocks of a caller's operator
-  hipEvent_t coef_ev_ = nullptr;      // its upload from hcoef_ has finished
+  bool coef_busy_ = false;            // its upload from hcoef_ may be in flight
   HostBuf hcoef_;
-  hipEvent_t fev_[2] = {nullptr, nullptr};
   FilterBatcher* batcher_ = nullptr;
   hipEvent_t ev_done_ = nullptr;  // the batcher has run this engine's steps
   bool one_pass_ = false;    // the last scaled Gram matrix had no pivot below kOnePass
   bool gram_ready_ = false;  // dres() holds (or will) the real Gram matrix of V's columns
-  bool timed_ = false;
-  bool step_pending_ = false;
-  long pend_launches_ = 0, step_launches_ = 0;
-  double pend_bytes_ = 0.0, step_bytes_ = 0.0, step_seconds_ = 0.0;
+  PhaseClock* clock_ = nullptr;
+  bool idle_ = false;
+  long step_launches_ = 0;
+  double step_bytes_ = 0.0;
 };
 
 // ------------------------------------------------------------- the solver
 struct TraceRow {
   double v[10];
-};
-
-// Stream time per phase of a solve.  An event is recorded on the solve's
-// stream where a phase begins; the time between consecutive events goes to
-// the phase that began at the first of them, so it includes the stream's
-// idle time while the host works inside the phase (the small eigensolve
-// counts to Rayleigh-Ritz, a served solve's wait for its shared filter batch
-// to the filter).  Finished intervals are folded whenever a new phase
-// begins; the solve's host waits keep the list of pending events short.
-class PhaseClock {
- public:
-  enum { kLanczos = 0, kFilter, kOrtho, kRR, kOther, kCount };
-  explicit PhaseClock(hipStream_t st) : st_(st) {}
-  PhaseClock(const PhaseClock&) = delete;
-  PhaseClock& operator=(const PhaseClock&) = delete;
-  ~PhaseClock() {
-    for (const Mark& m : marks_) (void)hipEventDestroy(m.ev);
-    for (hipEvent_t e : pool_) (void)hipEventDestroy(e);
-  }
-  void mark(int phase) {
-    fold(false);
-    hipEvent_t e;
-    if (!pool_.empty()) {
-      e = pool_.back();
-      pool_.pop_back();
-    } else {
-      RCG_HIP(hipEventCreate(&e));
-    }
-    RCG_HIP(hipEventRecord(e, st_));
-    marks_.push_back({e, phase});
-  }
-  // closes the last phase and folds every interval (waits for the stream)
-  void finish() {
-    mark(kOther);
-    if (!marks_.empty()) wait_event(marks_.back().ev, true);
-    fold(true);
-  }
-  double seconds(int phase) const { return sec_[phase]; }
-
- private:
-  struct Mark {
-    hipEvent_t ev;
-    int phase;
-  };
-  void fold(bool done) {
-    while (marks_.size() >= 2) {
-      if (!done) {
-        const hipError_t r = hipEventQuery(marks_[1].ev);
-        if (r != hipSuccess) {
-          (void)hipGetLastError();
-          break;
-        }
-      }
-      float ms = 0.f;
-      RCG_HIP(hipEventElapsedTime(&ms, marks_[0].ev, marks_[1].ev));
-      sec_[marks_[0].phase] += 1.0e-3 * ms;
-      pool_.push_back(marks_[0].ev);
-      marks_.pop_front();
-    }
-  }
-  hipStream_t st_;
-  std::deque<Mark> marks_;
-  std::vector<hipEvent_t> pool_;
-  double sec_[kCount] = {};
 };
 
 class Solver {
@@ -2222,7 +2227,7 @@ class Solver {
          FilterBatcher* batcher = nullptr)
       : op_(op), p_(p), eng_(ctx ? ctx : op->ctx, op, op->n), clock_(eng_.stream()) {
     eng_.set_batcher(batcher);
-    eng_.time_steps();
+    eng_.set_clock(&clock_);
     for (DevBuf* b : {&Vb_, &Tb_, &Wb_, &Yb_, &Mb_}) b->use_stream(eng_.stream());
   }
   Solver(const Solver&) = delete;
@@ -2410,7 +2415,10 @@ class Solver {
           starDegree = starDegreeSave;
           starBound = starBoundSave;
         }
-        clock_.mark(PhaseClock::kFilter);
+        // after an iteration's residuals the stream is empty
+        const bool idle = innerLoopCount > 0 && residual_count_ > 0;
+        clock_.mark(PhaseClock::kFilter, idle);
+        if (idle) eng_.set_idle();
         if (!completedBasis) {
           if (mixed)
             eng_.filter_mixed(subspaceSize, starDegree, rep, starBound, shift, fTheta, fRitz);
@@ -2421,7 +2429,7 @@ class Solver {
         applyCount += 1;
         count_apply_ += starDegree * subspaceSize;
 
-        clock_.mark(PhaseClock::kOrtho);
+        if (foundSize > 0) clock_.mark(PhaseClock::kOrtho);
         eng_.deflate(subspaceSize, foundSize);
         count_ortho_ += 1;
 
@@ -2434,6 +2442,7 @@ class Solver {
         t_eig_ += wall() - te;
         const long residualCheckCount = (foundSize + subspaceSize < N) ? inc : subspaceSize;
         eng_.rotate_residuals(subspaceSize, Yh, theta, residualCheckCount, subspaceResiduals);
+        residual_count_ = residualCheckCount;
         fTheta.assign(theta.begin(), theta.end());
         fRitz.assign(subspaceSize, 1);
         count_apply_ += residualCheckCount;
@@ -2591,12 +2600,12 @@ class Solver {
     clock_.finish();
     R->t_total = wall() - t0;
     R->t_lanczos = clock_.seconds(PhaseClock::kLanczos);
-    R->t_filter = clock_.seconds(PhaseClock::kFilter);
+    R->t_filter = clock_.seconds(PhaseClock::kFilter) + clock_.seconds(PhaseClock::kSteps);
     R->t_ortho = clock_.seconds(PhaseClock::kOrtho);
     R->t_rr = clock_.seconds(PhaseClock::kRR);
     R->t_eig = t_eig_;
     R->filter_degree_sum = degree_sum_;
-    R->t_filter_device = eng_.step_seconds();
+    R->t_filter_device = clock_.seconds(PhaseClock::kSteps);
     R->filter_bytes = eng_.step_bytes();
     R->filter_launches = eng_.step_launches();
     R->filter_panel = eng_.last_panel();
@@ -2653,6 +2662,7 @@ class Solver {
   PhaseClock clock_;
   long count_ortho_ = 0, count_apply_ = 0, count_eig_ = 0, degree_sum_ = 0;
   double guard_ = 0.0, t_eig_ = 0.0;
+  long residual_count_ = 0;  // residuals of the last iteration (it waited for them)
 };
 
 // allow_cx: a complex operator with complex (C128) blocks is accepted too.

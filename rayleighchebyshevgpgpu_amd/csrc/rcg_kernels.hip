@@ -1377,35 +1377,33 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
   const bool a_vec = ((reinterpret_cast<uintptr_t>(A) & 15) == 0) && (lda % W == 0);
   const bool x_vec = ((reinterpret_cast<uintptr_t>(X) & 15) == 0) && (ld % W == 0) &&
                      (c0 + xc + XE <= ncols);
-  // every row of the tile and every column of its X slice exist and both
-  // operands are 16-byte aligned: whole chunks are then loaded with no per-lane
-  // guard (decided once per wave: loads that lanes take or skip on their own
-  // make the wave wait, where the paths join, for the loads still in flight,
-  // which would undo the prefetch)
-  const bool tile_ok = a_vec && i0 + BM <= n && ((reinterpret_cast<uintptr_t>(X) & 15) == 0) &&
-                       (ld % W == 0) && c0 + BN <= ncols;
+  // Whole chunks are loaded with no guard: a row past n reads row n - 1 and a
+  // column vector past the rows' padding the last one, whose products land in
+  // entries that are not stored.  A's rows may start at any multiple of an element.
+  const bool x_ok = ((reinterpret_cast<uintptr_t>(X) & 15) == 0) && (ld % W == 0);
+  const T* arow = A + min(ai, n - 1) * lda + ak;
+  int xcol[XE / W];
+#pragma unroll
+  for (int q = 0; q < XE / W; ++q) xcol[q] = min(c0 + xc + q * W, ld - W);
+  typedef T VecU __attribute__((ext_vector_type(W), aligned(sizeof(T))));
   T ra2[2][AE], rx2[2][XE];
+  auto fetch_full = [&](int64_t k0, T (&ra)[AE], T (&rx)[XE]) {
+#pragma unroll
+    for (int q = 0; q < AE / W; ++q) {
+      const VecU t = *reinterpret_cast<const VecU*>(arow + k0 + q * W);
+#pragma unroll
+      for (int w = 0; w < W; ++w) ra[q * W + w] = t[w];
+    }
+#pragma unroll
+    for (int q = 0; q < XE / W; ++q) {
+      T t[W];
+      VT::ld(X + (k0 + xk) * ld + xcol[q], t);
+#pragma unroll
+      for (int w = 0; w < W; ++w) rx[q * W + w] = t[w];
+    }
+  };
   auto fetch_to = [&](int64_t k0, T (&ra)[AE], T (&rx)[XE]) {
     const int64_t ka = k0 + ak;
-    if (__builtin_amdgcn_readfirstlane((int)(tile_ok && k0 + BK <= n)) != 0) {
-      const T* ap = A + ai * lda + ka;
-      const T* xp = X + (k0 + xk) * ld + c0 + xc;
-#pragma unroll
-      for (int q = 0; q < AE / W; ++q) {
-        T t[W];
-        VT::ld(ap + q * W, t);
-#pragma unroll
-        for (int w = 0; w < W; ++w) ra[q * W + w] = t[w];
-      }
-#pragma unroll
-      for (int q = 0; q < XE / W; ++q) {
-        T t[W];
-        VT::ld(xp + q * W, t);
-#pragma unroll
-        for (int w = 0; w < W; ++w) rx[q * W + w] = t[w];
-      }
-      return;
-    }
     if (a_vec && ai < n && ka + AE <= n) {
       const T* ap = A + ai * lda + ka;
 #pragma unroll
@@ -1463,11 +1461,52 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
 #pragma unroll
     for (int q = 0; q < XE; ++q) Xs[buf][xk][xc + q] = sx[q];
   };
-  fetch_to(0, ra2[0], rx2[0]);
-  put(0, ra2[0], rx2[0]);
-  if (BK < n) fetch_to(BK, ra2[1], rx2[1]);
-  __syncthreads();
-  for (int64_t k0 = 0; k0 < n; k0 += 2 * BK) {
+  // Chunks [0, done) without guards.  The loop has no branch between a set's loads
+  // and its LDS stores: with one (whole chunk or not, last chunk or not) the
+  // compiler cannot count the loads in flight and waits for all of them, the set
+  // just issued included, before every store -- the loads were then one chunk
+  // of MFMAs ahead, not two (FP64 step at n = 16384, b = 256: 2.41 -> DFP64 ms; FP32
+  // 1.22 -> DFP32).
+  int64_t done = 0;
+  if (__builtin_amdgcn_readfirstlane((int)(x_ok && n >= 4 * BK)) != 0) {
+    const int64_t nf = n / BK;
+    fetch_full(0, ra2[0], rx2[0]);
+    put(0, ra2[0], rx2[0]);
+    fetch_full(BK, ra2[1], rx2[1]);
+    __syncthreads();
+    int64_t c = 0;
+    for (; c + 3 < nf; c += 2) {
+      fetch_full((c + 2) * BK, ra2[0], rx2[0]);
+      chunk(0);
+      put(1, ra2[1], rx2[1]);
+      __syncthreads();
+      fetch_full((c + 3) * BK, ra2[1], rx2[1]);
+      chunk(1);
+      put(0, ra2[0], rx2[0]);
+      __syncthreads();
+    }
+    // the last two or three: c in buffer 0, c + 1 in set 1
+    const bool three = c + 2 < nf;
+    if (three) fetch_full((c + 2) * BK, ra2[0], rx2[0]);
+    chunk(0);
+    put(1, ra2[1], rx2[1]);
+    __syncthreads();
+    chunk(1);
+    if (three) {
+      put(0, ra2[0], rx2[0]);
+      __syncthreads();
+      chunk(0);
+    }
+    done = nf * BK;
+    __syncthreads();  // both buffers are free
+  }
+  if (done < n) {
+    fetch_to(done, ra2[0], rx2[0]);
+    put(0, ra2[0], rx2[0]);
+    if (done + BK < n) fetch_to(done + BK, ra2[1], rx2[1]);
+    __syncthreads();
+  }
+  for (int64_t k0 = done; k0 < n; k0 += 2 * BK) {
     // even chunk: buffer 0, its successor in set 1; fetch chunk + 2 into set 0
     if (k0 + 2 * BK < n) fetch_to(k0 + 2 * BK, ra2[0], rx2[0]);
     chunk(0);
@@ -1818,9 +1857,12 @@ __global__ void herm_embed_kernel(double* G, int f, int b) {
 }
 
 // ----------------------------------------------------------------- Lanczos
-// rows per partial block of the Lanczos kernels: 512 below 2^20 rows (more
-// blocks for small operators), 2048 from there (fewer partials to reduce)
-inline int64_t lz_rows(int64_t n) { return n >= (int64_t(1) << 20) ? 2048 : 512; }
+// rows per partial block of the Lanczos kernels: 256, a row per thread, below 2^17
+// rows (more blocks for small operators), then 512, and 2048 from 2^20 (fewer
+// partials to reduce)
+inline int64_t lz_rows(int64_t n) {
+  return n >= (int64_t(1) << 20) ? 2048 : (n >= (int64_t(1) << 17) ? 512 : kThreads);
+}
 
 __device__ __forceinline__ double block_sum(double v, double* red) {
   red[threadIdx.x] = v;
@@ -1980,6 +2022,34 @@ __device__ void last_block_total(double s, double* P, unsigned* cnt, double* out
   }
 }
 
+// (A (x scale))_i, the nonzeros in order.  Eight at a time: their columns and
+// values are loaded together, then the gathers, then the FMAs (one at a time, each
+// of a row's nonzeros is a trip to memory of its own: n = 17576, 7 nonzeros, with
+// a row per thread instead of two, 11.3 -> 8.2 us).
+template <bool SCALE>
+__device__ __forceinline__ double lz_row(const int* __restrict__ rowptr,
+                                         const int* __restrict__ col,
+                                         const double* __restrict__ val,
+                                         const double* __restrict__ x, int64_t i, double scale) {
+  const int p1 = rowptr[i + 1];
+  double a = 0.0;
+  for (int p = rowptr[i]; p < p1; p += 8) {
+    int j[8];
+    double v[8], u[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      j[e] = p + e < p1 ? col[p + e] : 0;
+      v[e] = p + e < p1 ? val[p + e] : 0.0;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) u[e] = p + e < p1 ? x[j[e]] : 0.0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (p + e < p1) a = fma(v[e], SCALE ? u[e] * scale : u[e], a);
+  }
+  return a;
+}
+
 // One Lanczos step on a ping-pong pair of vectors (LanczosMaxMinFinder.h:
 // 300-345), for real CSR operators.  The previous step's swap (when
 // |beta_{k-1}| > 1e-14: w' = v / beta, v' = -beta w) is folded into the
@@ -1999,12 +2069,8 @@ __global__ __launch_bounds__(kThreads) void lz_step_kernel(
   const int64_t i1 = min(n, i0 + rpb);
   double s = 0.0;
   for (int64_t i = i0 + threadIdx.x; i < i1; i += kThreads) {
-    double a = 0.0;
-    if (sw) {
-      for (int p = rowptr[i]; p < rowptr[i + 1]; ++p) a = fma(val[p], v[col[p]] * rb, a);
-    } else {
-      for (int p = rowptr[i]; p < rowptr[i + 1]; ++p) a = fma(val[p], w[col[p]], a);
-    }
+    const double a = sw ? lz_row<true>(rowptr, col, val, v, i, rb)
+                        : lz_row<false>(rowptr, col, val, w, i, 1.0);
     const double wi = sw ? v[i] * rb : w[i];
     const double vi = sw ? w[i] * (-b) : v[i];
     const double vnew = vi + a;

@@ -1337,11 +1337,13 @@ struct DenseCfg {
   static constexpr int PA = sizeof(T) == 8 ? 1 : 2;
   static constexpr int PX = sizeof(T) == 8 ? 1 : 16;
 };
+// The products of one K split, summed by dense_combine_kernel.
+constexpr int kDensePartial = 7;
 template <typename T, int MODE>
 __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
     int64_t n, const T* __restrict__ A, int64_t lda, const T* __restrict__ X, const T* Z, T* out,
     int ld, int ncols, T p0, T p1, T p2, const T* __restrict__ R, const T* __restrict__ kap,
-    int ntn) {
+    int ntn, int nsplit, T* __restrict__ P) {
   constexpr int BK = DenseCfg<T>::BK;
   constexpr int BM = DenseCfg<T>::BM, BN = DenseCfg<T>::BN;
   constexpr int AE = BM * BK / kThreads;  // A elements per thread per chunk
@@ -1353,9 +1355,13 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
   using Acc = typename MfmaAcc<T>::type;
   const int64_t L = xcd_remap(blockIdx.x, gridDim.x);
   const int64_t ntm = (n + BM - 1) / BM;
-  if (L >= ntm * ntn) return;
-  const int64_t i0 = (L / ntn) * BM;
-  const int c0 = (int)(L % ntn) * BN;
+  if (L >= ntm * ntn * nsplit) return;
+  // K range of this split, whole chunks but for the last one's end
+  const int64_t split = L / (ntm * ntn), T0 = L % (ntm * ntn);
+  const int64_t kper = (n + (int64_t)nsplit * BK - 1) / ((int64_t)nsplit * BK) * BK;
+  const int64_t kbeg = min(n, split * kper), kend = min(n, kbeg + kper);
+  const int64_t i0 = (T0 / ntn) * BM;
+  const int c0 = (int)(T0 % ntn) * BN;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   Acc acc[NA][NB];
@@ -1404,7 +1410,7 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
   };
   auto fetch_to = [&](int64_t k0, T (&ra)[AE], T (&rx)[XE]) {
     const int64_t ka = k0 + ak;
-    if (a_vec && ai < n && ka + AE <= n) {
+    if (a_vec && ai < n && ka + AE <= kend) {
       const T* ap = A + ai * lda + ka;
 #pragma unroll
       for (int q = 0; q < AE / W; ++q) {
@@ -1415,10 +1421,10 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
       }
     } else {
 #pragma unroll
-      for (int q = 0; q < AE; ++q) ra[q] = (ai < n && ka + q < n) ? A[ai * lda + ka + q] : T(0);
+      for (int q = 0; q < AE; ++q) ra[q] = (ai < n && ka + q < kend) ? A[ai * lda + ka + q] : T(0);
     }
     const int64_t kx = k0 + xk;
-    if (x_vec && kx < n) {
+    if (x_vec && kx < kend) {
       const T* xp = X + kx * ld + c0 + xc;
 #pragma unroll
       for (int q = 0; q < XE / W; ++q) {
@@ -1431,7 +1437,7 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
 #pragma unroll
       for (int q = 0; q < XE; ++q) {
         const int c = c0 + xc + q;
-        rx[q] = (kx < n && c < ncols) ? X[kx * ld + c] : T(0);
+        rx[q] = (kx < kend && c < ncols) ? X[kx * ld + c] : T(0);
       }
     }
   };
@@ -1465,29 +1471,30 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
   // and its LDS stores: with one (whole chunk or not, last chunk or not) the
   // compiler cannot count the loads in flight and waits for all of them, the set
   // just issued included, before every store -- the loads were then one chunk
-  // of MFMAs ahead, not two (FP64 step at n = 16384, b = 256: 2.41 -> DFP64 ms; FP32
-  // 1.22 -> DFP32).
-  int64_t done = 0;
-  if (__builtin_amdgcn_readfirstlane((int)(x_ok && n >= 4 * BK)) != 0) {
-    const int64_t nf = n / BK;
-    fetch_full(0, ra2[0], rx2[0]);
+  // of MFMAs ahead, not two (FP64 step at n = 16384, b = 256: 2.38 -> 2.05 ms, 67
+  // TFLOP/s; FP32 1.19 -> 1.13; n = 9001, b = 64, whose rows are not 16-byte
+  // aligned: 1.22 -> 0.70 and 0.54 -> 0.23).
+  int64_t done = kbeg;
+  if (__builtin_amdgcn_readfirstlane((int)(x_ok && kend - kbeg >= 4 * BK)) != 0) {
+    const int64_t nf = (kend - kbeg) / BK;
+    fetch_full(kbeg, ra2[0], rx2[0]);
     put(0, ra2[0], rx2[0]);
-    fetch_full(BK, ra2[1], rx2[1]);
+    fetch_full(kbeg + BK, ra2[1], rx2[1]);
     __syncthreads();
     int64_t c = 0;
     for (; c + 3 < nf; c += 2) {
-      fetch_full((c + 2) * BK, ra2[0], rx2[0]);
+      fetch_full(kbeg + (c + 2) * BK, ra2[0], rx2[0]);
       chunk(0);
       put(1, ra2[1], rx2[1]);
       __syncthreads();
-      fetch_full((c + 3) * BK, ra2[1], rx2[1]);
+      fetch_full(kbeg + (c + 3) * BK, ra2[1], rx2[1]);
       chunk(1);
       put(0, ra2[0], rx2[0]);
       __syncthreads();
     }
     // the last two or three: c in buffer 0, c + 1 in set 1
     const bool three = c + 2 < nf;
-    if (three) fetch_full((c + 2) * BK, ra2[0], rx2[0]);
+    if (three) fetch_full(kbeg + (c + 2) * BK, ra2[0], rx2[0]);
     chunk(0);
     put(1, ra2[1], rx2[1]);
     __syncthreads();
@@ -1497,26 +1504,26 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
       __syncthreads();
       chunk(0);
     }
-    done = nf * BK;
+    done = kbeg + nf * BK;
     __syncthreads();  // both buffers are free
   }
-  if (done < n) {
+  if (done < kend) {
     fetch_to(done, ra2[0], rx2[0]);
     put(0, ra2[0], rx2[0]);
-    if (done + BK < n) fetch_to(done + BK, ra2[1], rx2[1]);
+    if (done + BK < kend) fetch_to(done + BK, ra2[1], rx2[1]);
     __syncthreads();
   }
-  for (int64_t k0 = done; k0 < n; k0 += 2 * BK) {
+  for (int64_t k0 = done; k0 < kend; k0 += 2 * BK) {
     // even chunk: buffer 0, its successor in set 1; fetch chunk + 2 into set 0
-    if (k0 + 2 * BK < n) fetch_to(k0 + 2 * BK, ra2[0], rx2[0]);
+    if (k0 + 2 * BK < kend) fetch_to(k0 + 2 * BK, ra2[0], rx2[0]);
     chunk(0);
-    if (k0 + BK < n) put(1, ra2[1], rx2[1]);
+    if (k0 + BK < kend) put(1, ra2[1], rx2[1]);
     __syncthreads();
-    if (k0 + BK >= n) break;
+    if (k0 + BK >= kend) break;
     // odd chunk: buffer 1, its successor in set 0; fetch chunk + 2 into set 1
-    if (k0 + 3 * BK < n) fetch_to(k0 + 3 * BK, ra2[1], rx2[1]);
+    if (k0 + 3 * BK < kend) fetch_to(k0 + 3 * BK, ra2[1], rx2[1]);
     chunk(1);
-    if (k0 + 2 * BK < n) put(0, ra2[0], rx2[0]);
+    if (k0 + 2 * BK < kend) put(0, ra2[0], rx2[0]);
     __syncthreads();
   }
 #pragma unroll
@@ -1530,14 +1537,43 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
         if (i >= n || c >= ncols) continue;
         const int64_t off = i * ld + c;
         const T v = acc[a][b][j];
+        if constexpr (MODE == kDensePartial) {
+          P[(split * n + i) * ncols + c] = v;
+          continue;
+        }
         T o;
-        if constexpr (MODE == kApply) o = p0 * v;
+        if constexpr (MODE == kApply || MODE == kDensePartial) o = p0 * v;
         else if constexpr (MODE == kApplyBeta) o = fma(p0, v, p1 * out[off]);
         else if constexpr (MODE == kChebFirst) o = p2 * (p1 * fma(p0, v, X[off]));
         else if constexpr (MODE == kCheb) o = p2 * fma(p1, fma(p0, v, X[off]), -Z[off]);
         else o = p2 * fma(kap[c], R[off], fma(p1, fma(p0, v, X[off]), -Z[off]));
         out[off] = o;
       }
+}
+
+// The step from the K splits' partial products, summed in their order.
+template <int MODE>
+__global__ __launch_bounds__(kThreads) void dense_combine_kernel(
+    int64_t n, const double* __restrict__ P, int nsplit, const double* X, const double* Z,
+    double* out, int ld, int ncols, double p0, double p1, double p2) {
+  const int64_t e = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  const int64_t m = n * ncols;
+  if (e >= m) return;
+  double v = 0.0;
+  for (int s = 0; s < nsplit; s += 4) {
+    double x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = s + u < nsplit ? P[(s + u) * m + e] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v += x[u];
+  }
+  const int64_t off = (e / ncols) * ld + e % ncols;
+  double o;
+  if constexpr (MODE == kApply) o = p0 * v;
+  else if constexpr (MODE == kApplyBeta) o = fma(p0, v, p1 * out[off]);
+  else if constexpr (MODE == kChebFirst) o = p2 * (p1 * fma(p0, v, X[off]));
+  else o = p2 * fma(p1, fma(p0, v, X[off]), -Z[off]);
+  out[off] = o;
 }
 
 // One column of a dense operator (the dense Lanczos matrix-vector products):
@@ -2210,10 +2246,27 @@ void launch_to_f32(int64_t n, const double* x, float* y, hipStream_t st) {
   RCG_HIP(hipGetLastError());
 }
 
+// K splits of an FP64 dense step: with fewer tiles than the two workgroups that a
+// CU holds, the tiles' K ranges are cut (at least 8 chunks each) and summed by a
+// second kernel, as far as the workspace reaches.  n = 2048, b = 64 (16 tiles): 157
+// -> 21.5 us; n = 700, b = 48: 59 -> 17; n = 6547, b = 119 (104 tiles): 499 -> 256.
+inline int dense_splits(int64_t n, int ncols, int64_t tiles, size_t ws_elems) {
+  const int64_t fill = 512 / tiles;
+  const int64_t depth = n / (8 * DenseCfg<double>::BK);
+  const int64_t room = (int64_t)(ws_elems / ((size_t)n * (size_t)ncols));
+  return (int)std::max<int64_t>(1, std::min({fill, depth, room, (int64_t)32}));
+}
+size_t dense_ws_elems(int64_t n, int ncols) {
+  const int64_t tiles = ((n + DenseCfg<double>::BM - 1) / DenseCfg<double>::BM) *
+                        ((ncols + DenseCfg<double>::BN - 1) / DenseCfg<double>::BN);
+  const int s = dense_splits(n, ncols, tiles, SIZE_MAX / 2);
+  return s > 1 ? (size_t)s * n * ncols : 0;
+}
+
 template <typename T>
 void launch_dense_step(int64_t n, const T* A, int64_t lda, const T* X, const T* Z, T* out, int ld,
                        int ncols, T p0, T p1, T p2, int mode, const T* R, const T* kap,
-                       hipStream_t st) {
+                       hipStream_t st, T* ws, size_t ws_elems) {
   if (n <= 0 || ncols <= 0) return;
   if constexpr (std::is_same<T, double>::value) {
     if (ncols == 1 && ld == 1 && (mode == kApply || mode == kApplyBeta)) {
@@ -2230,10 +2283,33 @@ void launch_dense_step(int64_t n, const T* A, int64_t lda, const T* X, const T* 
   }
   const int ntn = (ncols + DenseCfg<T>::BN - 1) / DenseCfg<T>::BN;
   const int64_t tiles = ((n + DenseCfg<T>::BM - 1) / DenseCfg<T>::BM) * ntn;
+  if constexpr (std::is_same<T, double>::value) {
+    const int nsplit = dense_splits(n, ncols, tiles, ws_elems);
+    if (ws && nsplit > 1 && mode != kChebSrc) {
+      const dim3 g2((unsigned)round_up(tiles * nsplit, kXcds));
+      hipLaunchKernelGGL((dense_step_kernel<T, kDensePartial>), g2, dim3(kThreads), 0, st, n, A, lda,
+                         X, Z, out, ld, ncols, p0, p1, p2, R, kap, ntn, nsplit, ws);
+      RCG_HIP(hipGetLastError());
+      const dim3 g3((unsigned)((n * ncols + kThreads - 1) / kThreads));
+#define RCG_COMBINE(M)                                                                           \
+  hipLaunchKernelGGL(dense_combine_kernel<M>, g3, dim3(kThreads), 0, st, n, ws, nsplit, X, Z, out, \
+                     ld, ncols, p0, p1, p2)
+      switch (mode) {
+        case kApply: RCG_COMBINE(kApply); break;
+        case kApplyBeta: RCG_COMBINE(kApplyBeta); break;
+        case kChebFirst: RCG_COMBINE(kChebFirst); break;
+        case kCheb: RCG_COMBINE(kCheb); break;
+        default: throw Error(1, "unknown dense step mode");
+      }
+#undef RCG_COMBINE
+      RCG_HIP(hipGetLastError());
+      return;
+    }
+  }
   const dim3 grid((unsigned)round_up(tiles, kXcds));
 #define RCG_DENSE(M)                                                                           \
   hipLaunchKernelGGL((dense_step_kernel<T, M>), grid, dim3(kThreads), 0, st, n, A, lda, X, Z, out, \
-                     ld, ncols, p0, p1, p2, R, kap, ntn)
+                     ld, ncols, p0, p1, p2, R, kap, ntn, 1, (T*)nullptr)
   switch (mode) {
     case kApply: RCG_DENSE(kApply); break;
     case kApplyBeta: RCG_DENSE(kApplyBeta); break;
@@ -2991,7 +3067,7 @@ void launch_lz_dot_c(int64_t n, const double* w, const double* v, double* alpha_
                                          hipStream_t);                                            \
   template void launch_fill_cols<T>(int64_t, T*, int, int, int, T, hipStream_t);                 \
   template void launch_dense_step<T>(int64_t, const T*, int64_t, const T*, const T*, T*, int, int, \
-                                     T, T, T, int, const T*, const T*, hipStream_t);
+                                     T, T, T, int, const T*, const T*, hipStream_t, T*, size_t);
 
 RCG_INST(double)
 RCG_INST(float)

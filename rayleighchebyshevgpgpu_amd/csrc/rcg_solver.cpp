@@ -862,6 +862,7 @@ class Engine {
     e = std::max(e, 2 * rcg::gram_ws_elems<double>(n_, fold, fold));
     e = std::max(e, rcg::colred_ws_elems(n_, 2 * (int)bb_));
     e = std::max(e, rcg::lz_ws_elems(n_));
+    if (op_ && op_->is_dense()) e = std::max(e, rcg::dense_ws_elems(n_, (int)bmax));
     ctx_->ws.ensure(e * sizeof(double));
     ws_elems_ = ctx_->ws.bytes / sizeof(double);
     const size_t sm = sizeof(double) * (size_t)(2 * bb_ * bb_ + 4 * bb_ + 64);
@@ -1120,7 +1121,8 @@ class Engine {
     }
     if (op_->is_dense()) {
       rcg::launch_dense_step<double>(n_, op_->dense, op_->lda, X, nullptr, out, (int)ld_, (int)b,
-                                     1.0, 0.0, 0.0, rcg::kStepApply, nullptr, nullptr, st_);
+                                     1.0, 0.0, 0.0, rcg::kStepApply, nullptr, nullptr, st_, ws(),
+                                     ws_elems_);
       return;
     }
     rcg::launch_csr_apply<double>(n_, op_->rowptr, op_->col, op_->val, X, out, (int)ld_,
@@ -1277,11 +1279,13 @@ class Engine {
       double* X1 = T();
       const double s1 = (m == 1) ? 0.5 : 1.0;
       rcg::launch_dense_step<double>(n_, op_->dense, op_->lda, X0, nullptr, X1, (int)ld_, (int)b,
-                                     c.g1, c.g2, s1, rcg::kStepFirst, nullptr, nullptr, st_);
+                                     c.g1, c.g2, s1, rcg::kStepFirst, nullptr, nullptr, st_, ws(),
+                                     ws_elems_);
       for (long j = 2; j <= m; ++j) {
         const double s = (j == m) ? 1.0 / double(m + 1) : 1.0;
         rcg::launch_dense_step<double>(n_, op_->dense, op_->lda, X1, X0, X0, (int)ld_, (int)b,
-                                       c.g1, c.g2, s, rcg::kStepCheb, nullptr, nullptr, st_);
+                                       c.g1, c.g2, s, rcg::kStepCheb, nullptr, nullptr, st_, ws(),
+                                       ws_elems_);
         std::swap(X0, X1);
       }
       if (X1 != V()) swapVT();

@@ -641,9 +641,11 @@ __global__ __launch_bounds__(kThreads) void gram_mfma_kernel(
 // Gram partials for blocks wider than one tile (bx or by > 64), through LDS.
 // Each workgroup owns one 64x64 output tile (enumerated as in gram_mfma_kernel)
 // and one row block; 32-row chunks of X[:, a0:a0+64] and Y[:, b0:b0+64] are
-// loaded with 16-byte loads one chunk ahead and staged in double-buffered LDS
-// (one barrier per chunk; loads two chunks ahead, as in the dense step, were
-// 5% faster for X^T X and 3-5% slower for the other two forms at 1024^2 x 192).  Wave w owns the 32x32 quadrant (w & 1, w >> 1) of
+// loaded as pairs, two chunks ahead, without guards, and staged in double-buffered
+// LDS (one barrier per chunk).  FP64 MFMA issue bounds it; with guarded loads one
+// chunk ahead and rows padded to 65 entries the waves waited on memory and banks:
+// X^T Y at 2^20 x 192 1.75 -> 1.47 ms (44 -> 53 TFLOP/s), X^T X 1.15 -> 0.95; 20000 x
+// 256, X^T X, 69 -> 49 us.  Wave w owns the 32x32 quadrant (w & 1, w >> 1) of
 // the tile, so no cross-wave reduction is needed; in a diagonal tile of X^T X
 // the quadrant below the diagonal is the mirror of the one above and its wave
 // idles.  (Each wave multiplying a quarter of every chunk's rows into the
@@ -658,8 +660,8 @@ template <int MODE>
 __global__ __launch_bounds__(kThreads, 2) void gram_lds_kernel(
     int64_t n, const double* __restrict__ X, int ldx, int bx, const double* __restrict__ Y, int ldy,
     int by, double* __restrict__ P, int64_t rows_per_blk, int nta, int ntiles, int64_t nblk) {
-  __shared__ double xs[2][kGramKr][kTile + 1];
-  __shared__ double ys[2][kGramKr][kTile + 1];
+  __shared__ __align__(16) double xs[2][kGramKr][kTile];
+  __shared__ __align__(16) double ys[2][kGramKr][kTile];
   const int64_t L = xcd_remap(blockIdx.x, gridDim.x);
   if (L >= nblk * ntiles) return;
   const int tile = (int)(L % ntiles);
@@ -690,71 +692,123 @@ __global__ __launch_bounds__(kThreads, 2) void gram_lds_kernel(
   const bool idle = diag && qa == 1 && qb == 0;
   const int64_t i0 = rblk * rows_per_blk;
   const int64_t i1 = min(n, i0 + rows_per_blk);
-  const bool vx = ((reinterpret_cast<uintptr_t>(X) & 15) == 0) && (ldx % 2 == 0);
-  const bool vy = ((reinterpret_cast<uintptr_t>(Y) & 15) == 0) && (ldy % 2 == 0);
-  // thread t moves pairs e = t + 256 m, m < 4: chunk row e / 32, columns
-  // 2 (e % 32) and 2 (e % 32) + 1 of the tile's 64
-  auto ld2 = [&](const double* B, int ldb, int bw, bool vec, int64_t row, int col) -> dvec2 {
+  // thread t moves pairs of columns: chunk rows t / 32 + 8 m, m < 4, columns 2 (t % 32)
+  // and 2 (t % 32) + 1 of the tile's 64
+  const int er = threadIdx.x / 32, ec = 2 * (threadIdx.x % 32);
+  auto ld2 = [&](const double* B, int ldb, int bw, int64_t row, int col) -> dvec2 {
     if (row >= i1) return dvec2{0.0, 0.0};
     const double* ptr = B + row * ldb + col;
-    if (vec && col + 1 < bw) return *reinterpret_cast<const dvec2*>(ptr);
     return dvec2{col < bw ? ptr[0] : 0.0, col + 1 < bw ? ptr[1] : 0.0};
   };
-  dvec2 px[4], py[4];
-  auto fetch = [&](int64_t r0) {
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int e = threadIdx.x + kThreads * m;
-      const int64_t row = r0 + e / 32;
-      const int c = 2 * (e % 32);
-      px[m] = ld2(X, ldx, bx, vx, row, a0 + c);
-      if (!diag) py[m] = ld2(Y, ldy, by, vy, row, b0 + c);
-    }
-  };
-  auto stash = [&](int buf) {
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int e = threadIdx.x + kThreads * m;
-      const int rr = e / 32;
-      const int c = 2 * (e % 32);
-      xs[buf][rr][c] = px[m].x;
-      xs[buf][rr][c + 1] = px[m].y;
-      if (!diag) {
-        ys[buf][rr][c] = py[m].x;
-        ys[buf][rr][c + 1] = py[m].y;
-      }
-    }
-  };
+  // Without guards: columns past the block's last pair are loaded from that pair (their
+  // products reach no output), an odd block's last column as the pair's second.
+  const int cx = min(a0 + ec, bx - 2), cy = min(b0 + ec, by - 2);
+  const bool shx = a0 + ec == bx - 1, shy = b0 + ec == by - 1;
+  typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
   d4v acc[2][2];
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
     for (int q = 0; q < 2; ++q) acc[p][q] = d4v{0.0, 0.0, 0.0, 0.0};
   const bool dquad = diag && qa == qb;  // quadrant on the diagonal: subtiles p <= q
-  int buf = 0;
-  if (i0 < i1) fetch(i0);
-  for (int64_t r0 = i0; r0 < i1; r0 += kGramKr) {
-    stash(buf);
-    __syncthreads();
-    if (r0 + kGramKr < i1) fetch(r0 + kGramKr);
-    if (!idle) {
-      const double(*yb)[kTile + 1] = diag ? xs[buf] : ys[buf];
+  // column of a row in LDS: rows of 64 with the halves of each 32 columns exchanged
+  // in odd rows, so that a half-wave's fragment (2 rows x 16 columns) covers all
+  // banks and a pair is stored by one 16-byte write
+  const int swz = 16 * (kr & 1);
+  auto run = [&](auto dg) {
+    constexpr bool DG = decltype(dg)::value;
+    dvec2 sx[2][4], sy[2][4];
+    auto fetch_full = [&](int64_t r0, int s) {
+      const double* xp = X + (r0 + er) * ldx + cx;
+      const double* yp = Y + (r0 + er) * ldy + cy;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const pair v = *reinterpret_cast<const pair*>(xp + (int64_t)(8 * m) * ldx);
+        sx[s][m] = dvec2{v[0], v[1]};
+        if constexpr (!DG) {
+          const pair w = *reinterpret_cast<const pair*>(yp + (int64_t)(8 * m) * ldy);
+          sy[s][m] = dvec2{w[0], w[1]};
+        }
+      }
+    };
+    auto put = [&](int buf, int s, bool ox, bool oy) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int rr = er + 8 * m, c = ec ^ (16 * (rr & 1));
+        dvec2 v = sx[s][m];
+        if (ox) v.x = v.y;
+        *reinterpret_cast<dvec2*>(&xs[buf][rr][c]) = v;
+        if constexpr (!DG) {
+          dvec2 w = sy[s][m];
+          if (oy) w.x = w.y;
+          *reinterpret_cast<dvec2*>(&ys[buf][rr][c]) = w;
+        }
+      }
+    };
+    auto chunk = [&](int buf) {
+      if (DG && idle) return;
+      const double(*yb)[kTile] = DG ? xs[buf] : ys[buf];
 #pragma unroll
       for (int k4 = 0; k4 < kGramKr; k4 += 4) {
         const int kk = k4 + kr;
         double af[2], bf[2];
 #pragma unroll
-        for (int p = 0; p < 2; ++p) af[p] = xs[buf][kk][32 * qa + 16 * p + cc];
+        for (int p = 0; p < 2; ++p) af[p] = xs[buf][kk][32 * qa + ((16 * p + cc) ^ swz)];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) bf[q] = yb[kk][32 * qb + 16 * q + cc];
+        for (int q = 0; q < 2; ++q) bf[q] = yb[kk][32 * qb + ((16 * q + cc) ^ swz)];
         acc[0][0] = mfma16x16x4(af[0], bf[0], acc[0][0]);
         acc[0][1] = mfma16x16x4(af[0], bf[1], acc[0][1]);
-        if (!dquad) acc[1][0] = mfma16x16x4(af[1], bf[0], acc[1][0]);
+        if (!DG || !dquad) acc[1][0] = mfma16x16x4(af[1], bf[0], acc[1][0]);
         acc[1][1] = mfma16x16x4(af[1], bf[1], acc[1][1]);
       }
+    };
+    // whole chunks, loaded two ahead into register set c % 2 with no branch between
+    // a set's loads and its stores (with one the compiler waits for all loads in flight)
+    const int64_t nf = bx > 1 && by > 1 ? (i1 - i0) / kGramKr : 0;
+    int64_t done = i0;
+    if (nf >= 4) {
+      fetch_full(i0, 0);
+      put(0, 0, shx, shy);
+      fetch_full(i0 + kGramKr, 1);
+      __syncthreads();
+      int64_t c = 0;
+      for (; c + 3 < nf; c += 2) {
+        fetch_full(i0 + (c + 2) * kGramKr, 0);
+        chunk(0);
+        put(1, 1, shx, shy);
+        __syncthreads();
+        fetch_full(i0 + (c + 3) * kGramKr, 1);
+        chunk(1);
+        put(0, 0, shx, shy);
+        __syncthreads();
+      }
+      const bool three = c + 2 < nf;
+      if (three) fetch_full(i0 + (c + 2) * kGramKr, 0);
+      chunk(0);
+      put(1, 1, shx, shy);
+      __syncthreads();
+      chunk(1);
+      if (three) {
+        put(0, 0, shx, shy);
+        __syncthreads();
+        chunk(0);
+      }
+      done = i0 + nf * kGramKr;
     }
-    buf ^= 1;
-  }
+    for (int64_t r0 = done; r0 < i1; r0 += kGramKr) {
+      __syncthreads();  // buffer 0 is free
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        sx[0][m] = ld2(X, ldx, bx, r0 + er + 8 * m, a0 + ec);
+        if constexpr (!DG) sy[0][m] = ld2(Y, ldy, by, r0 + er + 8 * m, b0 + ec);
+      }
+      put(0, 0, false, false);
+      __syncthreads();
+      chunk(0);
+    }
+  };
+  if (diag) run(std::true_type{});
+  else run(std::false_type{});
   if (idle) return;
   double* Pb = P + rblk * (int64_t)bx * by;
 #pragma unroll

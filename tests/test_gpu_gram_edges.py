@@ -1,5 +1,6 @@
-"""Gram products wider than 64 columns (64x64 tiles through LDS) at the edges of their tiles, row
-chunks (32) and row blocks, through deflation (Y^T X) and orthonormalisation (X^T X).
+"""Gram products, in one tile (up to 64 columns, passes of 32 or 64 rows per wave) and in 64x64 tiles
+through LDS (chunks of 32 rows), at the edges of both, through deflation (Y^T X) and
+orthonormalisation (X^T X).
 
 Tolerances: with unit columns an entry of a Gram product is off by at most (n + 32) u.  Deflation
 twice leaves Y^T X off by f times that; CholQR twice leaves X^T X off by b times that (the second
@@ -21,7 +22,9 @@ def unit(g, n, cols):
 
 
 @pytest.mark.parametrize("n,b", [(300, 65), (383, 128), (512, 127), (1000, 97), (2053, 193),
-                                 (4128, 130), (40001, 66)])
+                                 (4128, 130), (40001, 66),
+                                 (1, 1), (63, 2), (300, 15), (259, 17), (4099, 33), (4101, 47),
+                                 (30011, 49), (9999, 63), (50000, 64)])
 def test_orthonormalize(n, b):
     from rayleighchebyshevgpgpu_amd import solver as rcg
     print(f"case: orthonormalize n={n} b={b}", flush=True)
@@ -37,7 +40,9 @@ def test_orthonormalize(n, b):
 
 
 @pytest.mark.parametrize("n,b,f", [(200, 1, 65), (257, 65, 1), (1000, 2, 129), (999, 129, 3),
-                                   (2047, 66, 65), (4100, 67, 127), (40003, 96, 33)])
+                                   (2047, 66, 65), (4100, 67, 127), (40003, 96, 33),
+                                   (70, 1, 1), (300, 1, 64), (4097, 17, 1), (5000, 33, 48),
+                                   (9999, 63, 64), (30001, 16, 31)])
 def test_deflate(n, b, f):
     from rayleighchebyshevgpgpu_amd import solver as rcg
     print(f"case: deflate n={n} b={b} f={f}", flush=True)

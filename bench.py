@@ -17,7 +17,7 @@ is timed the same way
 and reported under "mixed", with its speed-up and its largest eigenvalue
 difference from the FP64 solve.
 
-roofline: the fused Chebyshev step kernel (csr_block_kernel, mode kCheb),
+roofline: the fused Chebyshev step kernel (csr_tile_kernel, mode kCheb),
 timed with HIP events on the library's stream around every filter
 application inside the timed solves; its algorithmic bytes per launch are
 nnz*(8+4) + 4*(n+1) + 3*n*b*8 (CSR values+columns+row pointers, one read of
@@ -632,13 +632,13 @@ def main():
         alg_bytes = sum(x[2].filter_bytes for x in results)
         achieved = alg_bytes / t_dev / 1e9 if t_dev > 0 else 0.0
         if WL["complex"]:
-            kern = ("csr_block_kernel<float,...,kChebSrc,complex> (complex64 correction step)"
+            kern = ("complex64 correction step (csr_tile_kernel or csr_block_kernel, kChebSrc)"
                     if precision == "mixed" else
-                    "csr_block_kernel<double,...,kCheb,complex> (fused complex128 Chebyshev step)")
+                    "csr_tile_kernel<double,true,kCheb> (fused complex128 Chebyshev step)")
         else:
-            kern = ("csr_block_kernel<float,8,2,kChebSrc> (FP32 correction step)"
+            kern = ("csr_tile_kernel<float,false,kChebSrc> (FP32 correction step)"
                     if precision == "mixed" else
-                    "csr_block_kernel<double,16,2,kCheb> (fused FP64 Chebyshev step)")
+                    "csr_tile_kernel<double,false,kCheb> (fused FP64 Chebyshev step)")
         roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                     "traffic": traffic_from_profiles(precision), "kernel": kern,

@@ -19,7 +19,7 @@ ROOT = os.path.dirname(HERE)
 
 SOURCES = ["rcg_kernels.hip", "rcg_batch.hip", "rcg_small.hip", "rcg_tile.hip",
            "rcg_solver.cpp", "rcg_io.cpp"]
-HEADERS = ["rcg_internal.hpp", "rcg_csr_rows.hpp", "rcg_cpoly.hpp", "rcg_dense.hpp"]
+HEADERS = ["rcg_internal.hpp", "rcg_csr_rows.hpp", "rcg_lz_row.hpp", "rcg_cpoly.hpp", "rcg_dense.hpp"]
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 FLAGS = [

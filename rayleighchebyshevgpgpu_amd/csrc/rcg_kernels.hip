@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "rcg_csr_rows.hpp"
+#include "rcg_lz_row.hpp"
 
 namespace rcg {
 namespace {
@@ -2157,34 +2158,6 @@ __device__ void last_block_total(double s, double* P, unsigned* cnt, double* out
     *out = take_sqrt ? sqrt(fabs(a)) : a;
     *cnt = 0u;
   }
-}
-
-// (A (x scale))_i, the nonzeros in order.  Eight at a time: their columns and
-// values are loaded together, then the gathers, then the FMAs (one at a time, each
-// of a row's nonzeros is a trip to memory of its own: n = 17576, 7 nonzeros, with
-// a row per thread instead of two, 11.3 -> 8.2 us).
-template <bool SCALE>
-__device__ __forceinline__ double lz_row(const int* __restrict__ rowptr,
-                                         const int* __restrict__ col,
-                                         const double* __restrict__ val,
-                                         const double* __restrict__ x, int64_t i, double scale) {
-  const int p1 = rowptr[i + 1];
-  double a = 0.0;
-  for (int p = rowptr[i]; p < p1; p += 8) {
-    int j[8];
-    double v[8], u[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      j[e] = p + e < p1 ? col[p + e] : 0;
-      v[e] = p + e < p1 ? val[p + e] : 0.0;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) u[e] = p + e < p1 ? x[j[e]] : 0.0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      if (p + e < p1) a = fma(v[e], SCALE ? u[e] * scale : u[e], a);
-  }
-  return a;
 }
 
 // One Lanczos step on a ping-pong pair of vectors (LanczosMaxMinFinder.h:

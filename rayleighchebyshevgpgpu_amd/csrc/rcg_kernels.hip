@@ -512,7 +512,8 @@ __device__ __forceinline__ void gram_tile_accumulate(d4v (&acc)[NT][NT], const d
     }
   };
   // Without guards: lanes past the last column (pair) load that one, which
-  // reaches no output; an odd block's last column is the second of its pair.
+  // reaches no output; an odd block's last column is the second of its pair.  A
+  // block of one column is the first of a pair with the row's padding.
   typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
   auto row_full = [&](const double* __restrict__ B, int ldb, int bw, int c0, int64_t row,
                       double (&v)[NT]) {
@@ -520,7 +521,7 @@ __device__ __forceinline__ void gram_tile_accumulate(d4v (&acc)[NT][NT], const d
 #pragma unroll
       for (int h = 0; h < NT / 2; ++h) {
         const int c = c0 + gram_col<NT>(2 * h, cc);
-        const pair t = *reinterpret_cast<const pair*>(B + row * ldb + min(c, bw - 2));
+        const pair t = *reinterpret_cast<const pair*>(B + row * ldb + max(0, min(c, bw - 2)));
         v[2 * h] = t[0];
         v[2 * h + 1] = t[1];
       }
@@ -541,8 +542,8 @@ __device__ __forceinline__ void gram_tile_accumulate(d4v (&acc)[NT][NT], const d
   bool sx[NT], sy[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    sx[t] = NT % 2 == 0 && a0 + gram_col<NT>(t, cc) == bx - 1;
-    sy[t] = NT % 2 == 0 && b0 + gram_col<NT>(t, cc) == by - 1;
+    sx[t] = NT % 2 == 0 && bx > 1 && a0 + gram_col<NT>(t, cc) == bx - 1;
+    sy[t] = NT % 2 == 0 && by > 1 && b0 + gram_col<NT>(t, cc) == by - 1;
   }
   auto mul = [&](const double (&xv)[U][NT], const double (&yv)[U][NT], bool shift) {
 #pragma unroll
@@ -567,7 +568,7 @@ __device__ __forceinline__ void gram_tile_accumulate(d4v (&acc)[NT][NT], const d
   // 128^3 x 64 511 -> 384 us, 5.6 TB/s; X^T X 280 -> 245; the pair of them at
   // 17576 x 24 13.2 -> 10.0).
   const int64_t last = i1 - ib - 16 * (U - 1) - 4;
-  const bool any = last >= 0 && (NT % 2 != 0 || (bx > 1 && (DIAG || by > 1)));
+  const bool any = last >= 0 && (NT % 2 != 0 || (ldx > 1 && (DIAG || ldy > 1)));
   const int np = __builtin_amdgcn_readfirstlane(any ? (int)(last / (16 * U)) + 1 : 0);
   if (np > 0) {
     load_full(ib, xa, yb);
@@ -749,9 +750,10 @@ __global__ __launch_bounds__(kThreads, 2) void gram_lds_kernel(
     return dvec2{col < bw ? ptr[0] : 0.0, col + 1 < bw ? ptr[1] : 0.0};
   };
   // Without guards: columns past the block's last pair are loaded from that pair (their
-  // products reach no output), an odd block's last column as the pair's second.
-  const int cx = min(a0 + ec, bx - 2), cy = min(b0 + ec, by - 2);
-  const bool shx = a0 + ec == bx - 1, shy = b0 + ec == by - 1;
+  // products reach no output), an odd block's last column as the pair's second, a
+  // block's only column as the first of a pair with the row's padding.
+  const int cx = max(0, min(a0 + ec, bx - 2)), cy = max(0, min(b0 + ec, by - 2));
+  const bool shx = bx > 1 && a0 + ec == bx - 1, shy = by > 1 && b0 + ec == by - 1;
   typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
   d4v acc[2][2];
 #pragma unroll
@@ -812,7 +814,7 @@ __global__ __launch_bounds__(kThreads, 2) void gram_lds_kernel(
     };
     // whole chunks, loaded two ahead into register set c % 2 with no branch between
     // a set's loads and its stores (with one the compiler waits for all loads in flight)
-    const int64_t nf = bx > 1 && by > 1 ? (i1 - i0) / kGramKr : 0;
+    const int64_t nf = ldx > 1 && ldy > 1 ? (i1 - i0) / kGramKr : 0;
     int64_t done = i0;
     if (nf >= 4) {
       fetch_full(i0, 0);

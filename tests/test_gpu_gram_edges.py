@@ -56,3 +56,24 @@ def test_deflate(n, b, f):
     ref -= Y @ (Y.T @ ref)
     ref /= np.linalg.norm(ref, axis=0) / np.linalg.norm(D, axis=0)
     assert np.max(np.abs(D - ref)) <= 4 * f * (n + 32) * U * max(1.0, np.abs(D).max())
+
+
+@pytest.mark.parametrize("n,b,f", [(257, 65, 1), (4097, 17, 1), (4097, 1, 24), (4100, 1, 96),
+                                   (9999, 96, 1), (2050, 31, 45)])
+def test_deflate_beside_nan(n, b, f):
+    """Columns of either block past the ones in use hold NaN, which reaches no result."""
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    print(f"case: deflate beside NaN n={n} b={b} f={f}", flush=True)
+    g = np.random.default_rng(n)
+    Y, X = np.full((n, f + 3), np.nan), np.full((n, b + 3), np.nan)
+    Y[:, :f] = np.linalg.qr(unit(g, n, f))[0]
+    X[:, :b] = unit(g, n, b)
+    bx, by = rcg.Block.from_host(X), rcg.Block.from_host(Y)
+    capi.check(capi.lib().rcg_deflate(bx.h, b, by.h, f))
+    D = bx.download()
+    assert np.isnan(D[:, b:]).all() and np.isfinite(D[:, :b]).all()
+    D, Y, X = D[:, :b], Y[:, :f], X[:, :b]
+    ref = X - Y @ (Y.T @ X)
+    ref -= Y @ (Y.T @ ref)
+    ref /= np.linalg.norm(ref, axis=0) / np.linalg.norm(D, axis=0)
+    assert np.max(np.abs(D - ref)) <= 4 * f * (n + 32) * U * max(1.0, np.abs(D).max())

@@ -49,6 +49,22 @@ inline void upper_inverse(const std::vector<double>& R, long n, std::vector<doub
   }
 }
 
+// Whether one CholQR pass makes a block orthonormal as well as two: inv2 =
+// ||R^{-1}||_F^2 of the factor of its n x n Gram matrix G with a unit diagonal, which
+// is trace(G^{-1}) while trace(G) = n.  The eigenvalues other than the least have
+// inverses of at least (n - 1)^2 / n in sum, so inv2 <= n + 1 leaves 1/lmin <= 3, and
+// likewise lmax < 3: the block's condition is below 3, and a pass loses the square of
+// it, a factor of 9.  (A bound on the pivots is none on the condition: unit columns
+// with every pivot above 1/2 reach 10^8 at 64 columns.)  The filtered Ritz blocks of
+// seven solves, 8 to 64 columns, stay below n + 0.6 in every iteration.
+inline bool one_pass_enough(double inv2, long n) { return inv2 <= double(n) + 1.0; }
+template <class S>
+double frobenius2(const std::vector<S>& M) {
+  double s = 0.0;
+  for (const S& x : M) s += std::norm(x);
+  return s;
+}
+
 // Symmetric eigensystem by cyclic Jacobi with an RMS threshold, ascending
 // eigenvalues, eigenvectors in the columns of Z (column-major).  H holds the
 // full symmetric matrix (column-major); it is not modified.

@@ -253,10 +253,10 @@ void launch_gram(int64_t n, const T* X, int ldx, int bx, const T* Y, int ldy, in
 void launch_gram_pair(int64_t n, const double* X, int ldx, const double* Y, int ldy, int b,
                       double* G, double* ws, size_t ws_elems, hipStream_t st);
 // The CholQR factor C = D R^{-1} (b x b) of X's columns on the device (see
-// reduce_chol_kernel); *clean = the smallest pivot of the Gram matrix scaled to
-// unit diagonal, 0 where it is not positive definite.
+// reduce_chol_kernel); *inv2 = ||R^{-1}||_F^2 of the factor of the Gram matrix scaled
+// to unit diagonal, 0 where it is not positive definite.
 bool chol_fits(int64_t n, int b);
-void launch_gram_chol(int64_t n, const double* X, int ldx, int b, double* C, double* clean,
+void launch_gram_chol(int64_t n, const double* X, int ldx, int b, double* C, double* inv2,
                       double* ws, size_t ws_elems, hipStream_t st);
 template <typename T>
 size_t gram_ws_elems(int64_t n, int bx, int by);

@@ -255,8 +255,8 @@ __global__ __launch_bounds__(kThreads) void reduce_partials_kernel(const T* __re
 // The partial sums of a b x b Gram matrix (b <= B) and its Cholesky factor, in one
 // workgroup: G = R^T R of the matrix scaled to unit diagonal, C = D R^{-1} (b x b
 // column-major; V C is orthonormal), so that a CholQR pass needs no trip to the
-// host.  *clean = the smallest pivot, or 0 where one is not positive; C is then
-// the identity.
+// host.  *inv2 = ||R^{-1}||_F^2, which bounds the block's condition (one_pass_enough
+// in rcg_dense.hpp), or 0 where a pivot is not positive; C is then the identity.
 //
 // One wave factors, without a barrier: lane c < 32 holds column c of the trailing
 // matrix, lane 32 + c column c of M = R^{-T} (the same eliminations applied to the
@@ -283,7 +283,7 @@ template <int B>
 __global__ __launch_bounds__(kCholThreads) void reduce_chol_kernel(const double* __restrict__ P,
                                                                    int64_t nblk, int b,
                                                                    double* __restrict__ C,
-                                                                   double* clean) {
+                                                                   double* inv2) {
   constexpr int NO = (B * B + 255) / 256;  // outputs per thread
   constexpr int NU = B <= 24 ? 8 : 4;      // partials of each in flight
   __shared__ double part[4][NO * 256];
@@ -333,15 +333,15 @@ __global__ __launch_bounds__(kCholThreads) void reduce_chol_kernel(const double*
     if (!right && i < b && c < b) a[i] = g(i, c) * (di * dg);
   }
   bool ok = true;
-  double least = 1.0;
+  double sum = 0.0;  // |column c of M|^2
 #pragma unroll
   for (int j = 0; j < B; ++j) {
     const double d = lane_of(a[j], j);
     // unit diagonal before elimination: a pivot below 1e-200 is no pivot
     const bool fine = d > 1e-200 && isfinite(d);
     ok = ok && fine;
-    least = fmin(least, d);
     a[j] *= rsqrt_newton(fine ? d : 1.0);
+    sum = fma(a[j], a[j], sum);
 #pragma unroll
     for (int i = j + 1; i < B; ++i) a[i] = fma(-lane_of(a[j], i), a[j], a[i]);
   }
@@ -351,7 +351,10 @@ __global__ __launch_bounds__(kCholThreads) void reduce_chol_kernel(const double*
     for (int k = 0; k < B; ++k)
       if (k < b) C[c + k * b] = ok ? (c <= k ? a[k] * dg : 0.0) : (c == k ? 1.0 : 0.0);
   }
-  if (lane == 0) *clean = ok ? least : 0.0;
+  sum = right && c < b ? sum : 0.0;
+#pragma unroll
+  for (int h = 16; h > 0; h /= 2) sum += __shfl_xor(sum, h);
+  if (lane == 32) *inv2 = ok ? sum : 0.0;
 }
 
 inline unsigned reduce_grid(int64_t m) { return (unsigned)((m + 63) / 64); }
@@ -2497,7 +2500,7 @@ bool chol_fits(int64_t n, int b) {
   return n > 0 && b >= 1 && b <= kCholMax && gram_blocks<double>(n, b, b, &rpb) * b * b <= 65536;
 }
 
-void launch_gram_chol(int64_t n, const double* X, int ldx, int b, double* C, double* clean,
+void launch_gram_chol(int64_t n, const double* X, int ldx, int b, double* C, double* inv2,
                       double* ws, size_t ws_elems, hipStream_t st) {
   if (!chol_fits(n, b)) throw Error(1, "block too large for the device factor");
   int64_t rpb;
@@ -2508,7 +2511,7 @@ void launch_gram_chol(int64_t n, const double* X, int ldx, int b, double* C, dou
   RCG_HIP(hipGetLastError());
 #define RCG_CHOL(B)                                                                              \
   hipLaunchKernelGGL(reduce_chol_kernel<B>, dim3(1), dim3(kCholThreads), 0, st, ws, nblk, b, C, \
-                     clean)
+                     inv2)
   if (b <= 16) RCG_CHOL(16);
   else if (b <= 24) RCG_CHOL(24);
   else RCG_CHOL(32);

@@ -917,8 +917,8 @@ class Engine {
   double* hvecUp() { return ctx_->pinned.as<double>() + 2 * bb_ * bb_ + bb_; }
   double* hlz() { return ctx_->pinned.as<double>() + 2 * bb_ * bb_ + 3 * bb_; }
 
-  // where reduce_chol_kernel says whether its factor is sound (past the Grams)
-  size_t clean_at() const { return 2 * (size_t)(cw_ * bb_) * (size_t)(cw_ * bb_) + 4 * (size_t)(cw_ * bb_); }
+  // where reduce_chol_kernel says how good its factor is (past the Grams)
+  size_t inv2_at() const { return 2 * (size_t)(cw_ * bb_) * (size_t)(cw_ * bb_) + 4 * (size_t)(cw_ * bb_); }
 
   double* ws() { return ctx_->ws.as<double>(); }
 
@@ -1637,13 +1637,6 @@ class Engine {
     for (int64_t j = 0; j < b; ++j)
       for (int64_t i = 0; i < b; ++i) G[i + j * b] *= d[i] * d[j];
   }
-  // the smallest pivot of the factorisation that gave R
-  template <class S>
-  static double least_pivot(int64_t b, const std::vector<S>& R) {
-    double p = 1.0;
-    for (int64_t j = 0; j < b; ++j) p = std::min(p, std::norm(R[j + j * b]));
-    return p;
-  }
 
   // One CholQR pass on V[:, :b]: G = V^H V scaled to unit diagonal,
   // G = R^H R, V <- V D R^{-1}.  A failed factorisation retries with the
@@ -1657,7 +1650,6 @@ class Engine {
     unit_diagonal(b, G, d);
     std::vector<S> R, Ri;
     bool clean = rcg::dense::cholesky_upper(G.data(), b, R);
-    one_pass_ = clean && least_pivot(b, R) >= kOnePass;
     if (!clean) {
       if (!allow_shift) throw Error(RCG_ERR_NUMERIC, "CholQR breakdown after a shifted pass");
       double gn = 0.0;
@@ -1668,6 +1660,7 @@ class Engine {
         throw Error(RCG_ERR_NUMERIC, "shifted CholQR breakdown (block is numerically rank deficient)");
     }
     rcg::dense::upper_inverse(R, b, Ri);
+    one_pass_ = clean && rcg::dense::one_pass_enough(rcg::dense::frobenius2(Ri), b);
     for (int64_t j = 0; j < b; ++j)
       for (int64_t i = 0; i < b; ++i) Ri[i + j * b] *= d[i];
     right_multiply<S>(b, Ri.data(), gram);
@@ -1678,7 +1671,6 @@ class Engine {
   // pass when the first needed a shift.
   void orthonormalize(int64_t b) {
     fold_b_ = 0;
-
     if (b <= 0) return;
     if (cx_) orthonormalize_t<cplx>(b);
     else orthonormalize_t<double>(b);
@@ -1772,12 +1764,11 @@ class Engine {
   // plain passes.
   //
   // Once the filter acts on Ritz vectors its output is nearly orthogonal, and
-  // the first pass does nothing that the second cannot: where the last Gram
-  // matrix, scaled to unit diagonal, had no pivot below 1/2 (R's condition is then
-  // a small number and one pass loses a few ulps), the projection starts from
-  // the block as it is and the first pass is skipped.  The Gram matrix that comes
-  // with it must meet the same bound; if not, the first pass runs after all.
-  static constexpr double kOnePass = 0.5;
+  // the first pass does nothing that the second cannot: where the last block's
+  // condition was bounded by a small number (one_pass_enough), the projection
+  // starts from the block as it is and the first pass is skipped.  The Gram matrix
+  // that comes with it must meet the same bound; if not, the first pass runs after
+  // all.
   // W = A V, then
   // G = V^H V and H1 = V^H W right after it, so that one wait brings both
   // back.  Below 2^22 block entries both products go in one paired launch
@@ -1821,7 +1812,11 @@ class Engine {
       sync();
       combine_gram<S>(hres(), b, b, G.data());
       unit_diagonal(b, G, scale);
-      one_pass = rcg::dense::cholesky_upper(G.data(), b, R) && least_pivot(b, R) >= kOnePass;
+      one_pass = rcg::dense::cholesky_upper(G.data(), b, R);
+      if (one_pass) {
+        rcg::dense::upper_inverse(R, b, Ri);
+        one_pass = rcg::dense::one_pass_enough(rcg::dense::frobenius2(Ri), b);
+      }
       if (!one_pass) std::fill(scale.begin(), scale.end(), 1.0);
       one_pass_ = one_pass;
     }
@@ -1830,15 +1825,16 @@ class Engine {
     bool on_device = !one_pass && !cx_ && !large && rcg::chol_fits(n_, (int)b);
     if (on_device) {
       gram_ready_ = false;
-      rcg::launch_gram_chol(n_, V(), (int)ld_, (int)b, dmatA(), dres() + clean_at(), ws(),
+      rcg::launch_gram_chol(n_, V(), (int)ld_, (int)b, dmatA(), dres() + inv2_at(), ws(),
                             ws_elems_, st_);
       rcg::launch_tall_gemm<double>(n_, V(), (int)ld_, (int)b, dmatA(), (int)b, (int)b, 1.0, 0.0,
                                     nullptr, T(), (int)ld_, st_);
       swapVT();
       first_projection(b, rb, apart, large);
       sync();
-      one_pass_ = hres()[clean_at()] >= kOnePass;
-      if (hres()[clean_at()] == 0.0) {
+      const double inv2 = hres()[inv2_at()];
+      one_pass_ = inv2 != 0.0 && rcg::dense::one_pass_enough(inv2, b);
+      if (inv2 == 0.0) {
         swapVT();
         on_device = false;
       }
@@ -1861,7 +1857,7 @@ class Engine {
       project<S>(b, H);
       return;
     }
-    rcg::dense::upper_inverse(R, b, Ri);
+    if (!one_pass) rcg::dense::upper_inverse(R, b, Ri);
     for (int64_t j = 0; j < b; ++j)
       for (int64_t i = 0; i <= j; ++i) Ri[i + j * b] *= scale[i];
     for (int64_t i = 0; i < b; ++i) {
@@ -2212,7 +2208,7 @@ class Engine {
   HostBuf hcoef_;
   FilterBatcher* batcher_ = nullptr;
   hipEvent_t ev_done_ = nullptr;  // the batcher has run this engine's steps
-  bool one_pass_ = false;    // the last scaled Gram matrix had no pivot below kOnePass
+  bool one_pass_ = false;    // one pass was enough for the last block (one_pass_enough)
   bool gram_ready_ = false;  // dres() holds (or will) the real Gram matrix of V's columns
   PhaseClock* clock_ = nullptr;
   bool idle_ = false;

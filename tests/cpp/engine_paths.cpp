@@ -1,0 +1,106 @@
+// The solve's engine (csrc/rcg_solver.cpp, compiled into this library) driven
+// piece by piece, for tests of branches that a whole solve reaches only with
+// unusual blocks or little memory.  The C entry points are this library's own
+// copies; the kernels come from librcg.so.  Launches are counted, and device
+// allocations can be made to fail from a size on.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <chrono>
+#include <cmath>
+#include <complex>
+#include <condition_variable>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <deque>
+#include <map>
+#include <memory>
+#include <mutex>
+#include <string>
+#include <thread>
+#include <type_traits>
+#include <vector>
+
+#include "../../rayleighchebyshevgpgpu_amd/csrc/rcg_internal.hpp"
+
+namespace {
+size_t g_alloc_limit = ~size_t(0);  // allocations above fail
+int g_device_factors = 0, g_pairs = 0, g_grams = 0;
+
+hipError_t limited_malloc(void** p, size_t bytes) {
+  if (bytes > g_alloc_limit) return hipErrorOutOfMemory;
+  return hipMalloc(p, bytes);
+}
+}  // namespace
+namespace rcg {
+inline void counted_gram_chol(int64_t n, const double* X, int ldx, int b, double* C, double* inv2,
+                              double* ws, size_t ws_elems, hipStream_t st) {
+  ++g_device_factors;
+  launch_gram_chol(n, X, ldx, b, C, inv2, ws, ws_elems, st);
+}
+inline void counted_gram_pair(int64_t n, const double* X, int ldx, const double* Y, int ldy, int b,
+                              double* G, double* ws, size_t ws_elems, hipStream_t st) {
+  ++g_pairs;
+  launch_gram_pair(n, X, ldx, Y, ldy, b, G, ws, ws_elems, st);
+}
+template <typename T, typename... Args>
+void counted_gram(int64_t n, const T* X, Args... args) {
+  ++g_grams;
+  launch_gram<T>(n, X, args...);
+}
+}  // namespace rcg
+#define hipMalloc limited_malloc
+#define launch_gram counted_gram
+#define launch_gram_chol counted_gram_chol
+#define launch_gram_pair counted_gram_pair
+#include "../../rayleighchebyshevgpgpu_amd/csrc/rcg_solver.cpp"
+
+namespace {
+template <class S>
+void project_and_rotate(Engine& e, int64_t b, double* H_out, double* res) {
+  std::vector<S> H, I(b * b, S(0.0));
+  e.ortho_project<S>(b, H);
+  std::memcpy(H_out, H.data(), sizeof(S) * b * b);
+  std::vector<double> th(b), r;
+  for (int64_t j = 0; j < b; ++j) {
+    I[j + j * b] = S(1.0);
+    th[j] = std::real(H[j + j * b]);
+  }
+  e.rotate_residuals(b, I, th, b, r);
+  std::memcpy(res, r.data(), sizeof(double) * b);
+}
+}  // namespace
+
+extern "C" {
+void test_alloc_limit(int64_t bytes) { g_alloc_limit = bytes < 0 ? ~size_t(0) : (size_t)bytes; }
+
+// An iteration's orthonormalisation and projection of V (H, b x b), then its
+// rotation by the identity: V holds the orthonormal basis, res the residuals with
+// the diagonal of H.  prime (or null) goes first through the same engine, as the
+// iteration before.  counts: device factors, paired and single
+// Gram products for V.
+int test_ortho_project(rcg_operator op, rcg_block prime, rcg_block V, rcg_block T, rcg_block W,
+                       int64_t b, double* H, double* res, int32_t* counts) {
+  return guarded([&] {
+    Engine e(op->ctx, op, op->n);
+    e.reserve(real_ld(V), real_ld(V));
+    auto run = [&](rcg_block X) {
+      e.attach(static_cast<double*>(X->d()), static_cast<double*>(T->d()),
+               static_cast<double*>(W->d()), real_ld(X), nullptr, 0);
+      g_device_factors = g_pairs = g_grams = 0;
+      if (e.cx()) project_and_rotate<cplx>(e, b, H, res);
+      else project_and_rotate<double>(e, b, H, res);
+    };
+    if (prime) run(prime);
+    run(V);
+    counts[0] = g_device_factors;
+    counts[1] = g_pairs;
+    counts[2] = g_grams;
+    if (!e.v_is_first())
+      rcg::launch_copy_cols<double>(V->n, e.V(), (int)real_ld(V), 0, static_cast<double*>(V->d()),
+                                    (int)real_ld(V), 0, (int)(e.cw() * b), e.stream());
+    e.sync();
+  });
+}
+}

@@ -1,0 +1,136 @@
+"""Branches of the solve's engine that a whole solve reaches only with unusual
+blocks, driven piece by piece through tests/cpp/engine_paths.cpp.
+
+An iteration's orthonormalisation takes one CholQR pass where the block is known to
+be nearly orthonormal, else two, and three after a shift; the first factor is made
+on the device for real blocks of at most 32 columns.  Whatever the way, the basis
+must be orthonormal and span the block, H = Q^H A Q, and the residuals those of Q;
+the numbers of launches say which way was taken.
+
+Tolerance: an entry of a Gram product of unit columns is summed in chains of fewer
+than 256 terms (a lane's rows of a row block, then the partials), so it is off by at
+most 256 u, and a basis of b columns by b times that.
+"""
+import ctypes as C
+import gc
+import os
+
+import numpy as np
+import pytest
+
+from rayleighchebyshevgpgpu_amd import capi
+from rayleighchebyshevgpgpu_amd import operators as ops
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0**-53
+LIB = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "libengine_paths.so")
+
+
+@pytest.fixture(scope="module")
+def eng():
+    """The Python classes over the test library."""
+    from rayleighchebyshevgpgpu_amd import solver
+    old = capi._lib, capi.LIB_PATH, solver._default_ctx
+    capi._lib, capi.LIB_PATH, solver._default_ctx = None, LIB, None
+    L = capi.lib()
+    vp, i64 = C.c_void_p, C.c_int64
+    L.test_ortho_project.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, vp]
+    yield L
+    gc.collect()
+    if solver._default_ctx is not None:
+        solver._default_ctx.close()
+    capi._lib, capi.LIB_PATH, solver._default_ctx = old
+
+
+def operator(shape, cx):
+    if cx:
+        return ops.hofstadter_2d(shape[0], phi=1.0 / 8, W=1.0)
+    n = int(np.prod(shape))
+    return ops.laplacian_3d(*shape, "dirichlet", ops.anderson_potential(n, 3.0, n))
+
+
+def block(kind, n, b, cx, seed):
+    g = np.random.default_rng(seed)
+
+    def draw(r, c):
+        x = g.standard_normal((r, c))
+        return x + 1j * g.standard_normal((r, c)) if cx else x
+
+    Q = np.linalg.qr(draw(n, b))[0]
+    if kind == "near":  # as a filter leaves Ritz vectors
+        return Q + 1e-3 / np.sqrt(n) * draw(n, b)
+    if kind == "random":
+        return Q @ (np.diag(np.logspace(0, -4, b)) @ np.linalg.qr(draw(b, b))[0])
+    if kind == "pivots":  # every pivot above 1/2, and yet a condition of thousands
+        R = np.zeros((b, b))
+        for j in range(b):
+            k = min(4, j)
+            R[j, j] = np.sqrt(0.51) if k else 1.0
+            R[j - k:j, j] = -np.sqrt(0.49 / k) if k else 0.0
+        assert np.linalg.cond(R) > 1e3
+        return Q @ R
+    if kind == "rank":  # half of the directions below the Gram matrix's roundoff
+        return Q @ (np.diag(np.where(np.arange(b) % 2, 1e-9, 1.0)) @ np.linalg.qr(draw(b, b))[0])
+    assert kind == "zero"
+    Q[:, b // 2] = 0.0
+    return Q
+
+
+def ortho_project(L, A, V, prime):
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    n, b = V.shape
+    op = rcg.CsrOperator(A)
+    bp = None if prime is None else rcg.Block.from_host(prime)
+    bv = rcg.Block.from_host(V)
+    bt, bw = rcg.Block(n, b, dtype=V.dtype), rcg.Block(n, b, dtype=V.dtype)
+    H, res = np.zeros((b, b), dtype=V.dtype, order="F"), np.zeros(b)
+    counts = np.full(3, -1, dtype=np.int32)
+    capi.check(L.test_ortho_project(op.h, bp and bp.h, bv.h, bt.h, bw.h, b,
+                                    H.ctypes.data_as(C.c_void_p), res.ctypes.data_as(C.c_void_p),
+                                    counts.ctypes.data_as(C.c_void_p)))
+    return bv.download(), H, res, counts.tolist()
+
+
+# launches (device factors, paired, single Gram products) of the block by kind, and
+# of the same after a nearly orthonormal block, where one pass is tried first
+SMALL = {"near": ([1, 1, 0], [0, 1, 0]), "random": ([1, 1, 0], [1, 2, 0]),
+         "pivots": ([1, 1, 0], [1, 2, 0]), "rank": ([1, 1, 4], [1, 2, 4])}
+HOST = {"near": ([0, 1, 1], [0, 1, 0]), "random": ([0, 1, 1], [0, 2, 1]),
+        "pivots": ([0, 1, 1], [0, 2, 1]), "rank": ([0, 0, 4], [0, 1, 4])}
+LARGE = {"near": ([0, 0, 2], [0, 0, 2]), "random": ([0, 0, 2], [0, 0, 4]),
+         "pivots": ([0, 0, 2], [0, 0, 4]), "rank": ([0, 0, 3], [0, 0, 5])}
+
+
+@pytest.mark.parametrize("primed", [False, True])
+@pytest.mark.parametrize("kind", ["near", "random", "pivots", "rank"])
+@pytest.mark.parametrize("shape,b,cx,want", [
+    ((12, 12, 12), 24, False, SMALL), ((11, 12, 13), 32, False, SMALL), ((10, 9, 11), 40, False, HOST),
+    ((24, 24), 24, True, HOST), ((64, 64, 64), 24, False, LARGE)])
+def test_ortho_project(eng, shape, b, cx, want, kind, primed):
+    print(f"case: {shape} b={b} cx={cx} {kind} primed={primed}", flush=True)
+    A = operator(shape, cx)
+    V = block(kind, A.n, b, cx, 1)
+    prime = block("near", A.n, b, cx, 2) if primed else None
+    Q, H, res, counts = ortho_project(eng, A, V, prime)
+    tol = 256 * b * U
+    S = A.to_scipy()
+    AQ = S @ Q
+    norm = np.abs(S).sum(axis=1).max()
+    assert np.max(np.abs(Q.conj().T @ Q - np.eye(b))) <= tol
+    assert np.max(np.abs(Q @ (Q.conj().T @ V) - V)) <= 2 * tol
+    assert np.max(np.abs(Q.conj().T @ AQ - H)) <= 2 * norm * tol
+    ref = np.linalg.norm(Q * np.real(np.diag(H)) - AQ, axis=0)
+    assert np.max(np.abs(res - ref)) <= 2 * norm * tol
+    assert counts == want[kind][primed]
+
+
+@pytest.mark.parametrize("primed", [False, True])
+@pytest.mark.parametrize("shape,b,cx", [((12, 12, 12), 24, False), ((24, 24), 24, True)])
+def test_zero_column_is_refused(eng, shape, b, cx, primed):
+    """A block with a zero column has no orthonormal basis: the shifted passes end with
+    an error whichever way they are reached."""
+    A = operator(shape, cx)
+    with pytest.raises(capi.RcgError, match="CholQR breakdown after a shifted pass"):
+        ortho_project(eng, A, block("zero", A.n, b, cx, 1),
+                      block("near", A.n, b, cx, 2) if primed else None)

@@ -2325,21 +2325,29 @@ void launch_to_f32(int64_t n, const double* x, float* y, hipStream_t st) {
   RCG_HIP(hipGetLastError());
 }
 
+inline int64_t dense_tiles(int64_t n, int64_t ncols, int bm, int bn) {
+  return ((n + bm - 1) / bm) * ((ncols + bn - 1) / bn);
+}
 // K splits of an FP64 dense step: with fewer tiles than the two workgroups that a
 // CU holds, the tiles' K ranges are cut (at least 8 chunks each) and summed by a
-// second kernel, as far as the workspace reaches.  n = 2048, b = 64 (16 tiles): 157
-// -> 21.5 us; n = 700, b = 48: 59 -> 17; n = 6547, b = 119 (104 tiles): 499 -> 256.
-inline int dense_splits(int64_t n, int ncols, int64_t tiles, size_t ws_elems) {
-  const int64_t fill = 512 / tiles;
+// second kernel.  n = 2048, b = 64 (16 tiles): 157 -> 21.5 us; n = 700, b = 48: 59 ->
+// 17; n = 6547, b = 119 (104 tiles): 499 -> 256.  The sizes alone decide, so that
+// the order of the sums, and with it the bits, never depends on what a workspace
+// happens to hold.
+inline int dense_splits(int64_t n, int64_t ncols) {
+  const int64_t fill = 512 / dense_tiles(n, ncols, DenseCfg<double>::BM, DenseCfg<double>::BN);
   const int64_t depth = n / (8 * DenseCfg<double>::BK);
-  const int64_t room = (int64_t)(ws_elems / ((size_t)n * (size_t)ncols));
-  return (int)std::max<int64_t>(1, std::min({fill, depth, room, (int64_t)32}));
+  return (int)std::max<int64_t>(1, std::min({fill, depth, (int64_t)32}));
 }
 size_t dense_ws_elems(int64_t n, int ncols) {
-  const int64_t tiles = ((n + DenseCfg<double>::BM - 1) / DenseCfg<double>::BM) *
-                        ((ncols + DenseCfg<double>::BN - 1) / DenseCfg<double>::BN);
-  const int s = dense_splits(n, ncols, tiles, SIZE_MAX / 2);
-  return s > 1 ? (size_t)s * n * ncols : 0;
+  // fewer columns can take more splits: the most columns of every number of tiles
+  size_t most = 0;
+  for (int64_t c = 0; c < ncols;) {
+    c = std::min<int64_t>(ncols, c + DenseCfg<double>::BN);
+    const int s = dense_splits(n, c);
+    if (s > 1) most = std::max(most, (size_t)s * (size_t)n * (size_t)c);
+  }
+  return most;
 }
 
 template <typename T>
@@ -2361,10 +2369,12 @@ void launch_dense_step(int64_t n, const T* A, int64_t lda, const T* X, const T* 
     }
   }
   const int ntn = (ncols + DenseCfg<T>::BN - 1) / DenseCfg<T>::BN;
-  const int64_t tiles = ((n + DenseCfg<T>::BM - 1) / DenseCfg<T>::BM) * ntn;
+  const int64_t tiles = dense_tiles(n, ncols, DenseCfg<T>::BM, DenseCfg<T>::BN);
   if constexpr (std::is_same<T, double>::value) {
-    const int nsplit = dense_splits(n, ncols, tiles, ws_elems);
+    const int nsplit = dense_splits(n, ncols);
     if (ws && nsplit > 1 && mode != kChebSrc) {
+      if ((size_t)nsplit * (size_t)n * (size_t)ncols > ws_elems)
+        throw Error(3, "dense step workspace too small");
       const dim3 g2((unsigned)round_up(tiles * nsplit, kXcds));
       hipLaunchKernelGGL((dense_step_kernel<T, kDensePartial>), g2, dim3(kThreads), 0, st, n, A, lda,
                          X, Z, out, ld, ncols, p0, p1, p2, R, kap, ntn, nsplit, ws);

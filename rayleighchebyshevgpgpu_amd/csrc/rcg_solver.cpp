@@ -862,7 +862,7 @@ class Engine {
     e = std::max(e, 2 * rcg::gram_ws_elems<double>(n_, fold, fold));
     e = std::max(e, rcg::colred_ws_elems(n_, 2 * (int)bb_));
     e = std::max(e, rcg::lz_ws_elems(n_));
-    if (op_ && op_->is_dense()) e = std::max(e, rcg::dense_ws_elems(n_, (int)bmax));
+    if (op_ && op_->is_dense()) e = std::max(e, rcg::dense_ws_elems(n_, (int)bb_));
     ctx_->ws.ensure(e * sizeof(double));
     ws_elems_ = ctx_->ws.bytes / sizeof(double);
     const size_t sm = sizeof(double) * (size_t)(2 * bb_ * bb_ + 4 * bb_ + 64);

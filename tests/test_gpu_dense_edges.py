@@ -68,3 +68,28 @@ def test_padded_rows(n, lda, cols):
     capi.check(capi.lib().rcg_cheb_filter(h, bx.h, bt.h, cols, 1, 1, 4.0 * n, 0.0))
     assert np.isfinite(bx.download()).all()
     capi.check(capi.lib().rcg_operator_destroy(h))
+
+
+@pytest.mark.parametrize("n,cols,pad", [(3000, 64, 4), (2049, 64, 4)])
+def test_products_do_not_depend_on_earlier_calls(n, cols, pad):
+    """The same call before and after one that needs more workspace: the same bits."""
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    print(f"case: dense history n={n} cols={cols}", flush=True)
+    g = np.random.default_rng(n)
+    A = g.uniform(-1, 1, (n, n))
+    A = np.asfortranarray((A + A.T) / n)
+    X = np.zeros((n, cols + pad))
+    X[:, :cols] = g.uniform(-1, 1, (n, cols))
+    ctx = rcg.Context(0)
+    op = rcg.DenseOperator(A, ctx=ctx)
+
+    def filtered():
+        bx, bt = rcg.Block.from_host(X, ctx), rcg.Block(n, cols + pad, ctx=ctx)
+        capi.check(capi.lib().rcg_cheb_filter(op.h, bx.h, bt.h, cols, 3, 1, 2.0, 1.0))
+        return bx.download(cols)
+
+    first = filtered()
+    wide, tmp = rcg.Block(100000, 200, ctx=ctx), rcg.Block(100000, 200, ctx=ctx)
+    wide.randomize(0, 200, 1, 0)
+    capi.check(capi.lib().rcg_orthonormalize(wide.h, tmp.h, 200))
+    assert np.array_equal(filtered(), first)

@@ -239,7 +239,8 @@ int rcg_residuals(rcg_operator op, rcg_block V, rcg_block W, int64_t count, cons
  * values and sums live in a library-owned device array of 16 MiB per device
  * (2^21 doubles), held until the process ends: 3 doubles per real column
  * (2 per complex column) plus one per real column and 512 rows must fit, else
- * RCG_ERR_INVALID.  The operator's CSR rows are visited in the default order
+ * RCG_ERR_INVALID.  The partial sums of a dense operator's product pass through
+ * the same array.  The operator's CSR rows are visited in the default order
  * (no autotuning).  All calls on one device share that array: calls that
  * overlap on one device race.  Waits for its stream before returning. */
 int rcg_residuals_noalloc(rcg_operator op, rcg_block V, rcg_block W, int64_t count,

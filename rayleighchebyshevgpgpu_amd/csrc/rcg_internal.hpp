@@ -237,7 +237,8 @@ void launch_dense_step(int64_t n, const T* A, int64_t lda, const T* X, const T* 
                        int ncols, T p0, T p1, T p2, int mode, const T* R, const T* kap,
                        hipStream_t st, T* ws = nullptr, size_t ws_elems = 0);
 // Workspace (FP64) of steps of up to ncols columns, with which a step of too few
-// tiles to fill the chip is split along K; without it the step is not split.
+// tiles to fill the chip is split along K.  With less the step runs on fewer columns
+// at a time (the same bits), with none it is not split.
 size_t dense_ws_elems(int64_t n, int ncols);
 
 // G (bx x by, column-major, ldg = bx) = X^H Y over n rows; ws holds partials.

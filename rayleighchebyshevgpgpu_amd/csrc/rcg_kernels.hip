@@ -1426,7 +1426,8 @@ struct MfmaAcc<float> {
 // the free LDS buffer after the MFMAs of the chunk before it, one barrier per
 // chunk.  The column tiles of a row
 // tile are consecutive logical workgroups, kept on one XCD, so the A rows
-// they share come from the same L2.
+// they share come from the same L2.  The step is made on columns [cfirst, ncols),
+// cfirst a multiple of 4.
 template <typename T>
 struct DenseCfg {
   // FP32 runs 64-row tiles (16 rows per wave): at n = 16384, b = 256 that is
@@ -1450,7 +1451,7 @@ template <typename T, int MODE>
 __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
     int64_t n, const T* __restrict__ A, int64_t lda, const T* __restrict__ X, const T* Z, T* out,
     int ld, int ncols, T p0, T p1, T p2, const T* __restrict__ R, const T* __restrict__ kap,
-    int ntn, int nsplit, T* __restrict__ P) {
+    int cfirst, int ntn, int nsplit, T* __restrict__ P) {
   constexpr int BK = DenseCfg<T>::BK;
   constexpr int BM = DenseCfg<T>::BM, BN = DenseCfg<T>::BN;
   constexpr int AE = BM * BK / kThreads;  // A elements per thread per chunk
@@ -1468,7 +1469,7 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
   const int64_t kper = (n + (int64_t)nsplit * BK - 1) / ((int64_t)nsplit * BK) * BK;
   const int64_t kbeg = min(n, split * kper), kend = min(n, kbeg + kper);
   const int64_t i0 = (T0 / ntn) * BM;
-  const int c0 = (int)(T0 % ntn) * BN;
+  const int c0 = cfirst + (int)(T0 % ntn) * BN;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   Acc acc[NA][NB];
@@ -1645,7 +1646,7 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
         const int64_t off = i * ld + c;
         const T v = acc[a][b][j];
         if constexpr (MODE == kDensePartial) {
-          P[(split * n + i) * ncols + c] = v;
+          P[(split * n + i) * (ncols - cfirst) + c - cfirst] = v;
           continue;
         }
         T o;
@@ -1662,9 +1663,10 @@ __global__ __launch_bounds__(kThreads, 2) void dense_step_kernel(
 template <int MODE>
 __global__ __launch_bounds__(kThreads) void dense_combine_kernel(
     int64_t n, const double* __restrict__ P, int nsplit, const double* X, const double* Z,
-    double* out, int ld, int ncols, double p0, double p1, double p2) {
+    double* out, int ld, int cfirst, int ncols, double p0, double p1, double p2) {
   const int64_t e = blockIdx.x * (int64_t)kThreads + threadIdx.x;
-  const int64_t m = n * ncols;
+  const int nc = ncols - cfirst;
+  const int64_t m = n * nc;
   if (e >= m) return;
   double v = 0.0;
   for (int s = 0; s < nsplit; s += 4) {
@@ -1674,7 +1676,7 @@ __global__ __launch_bounds__(kThreads) void dense_combine_kernel(
 #pragma unroll
     for (int u = 0; u < 4; ++u) v += x[u];
   }
-  const int64_t off = (e / ncols) * ld + e % ncols;
+  const int64_t off = (e / nc) * ld + cfirst + e % nc;
   double o;
   if constexpr (MODE == kApply) o = p0 * v;
   else if constexpr (MODE == kApplyBeta) o = fma(p0, v, p1 * out[off]);
@@ -2372,33 +2374,40 @@ void launch_dense_step(int64_t n, const T* A, int64_t lda, const T* X, const T* 
   const int64_t tiles = dense_tiles(n, ncols, DenseCfg<T>::BM, DenseCfg<T>::BN);
   if constexpr (std::is_same<T, double>::value) {
     const int nsplit = dense_splits(n, ncols);
-    if (ws && nsplit > 1 && mode != kChebSrc) {
-      if ((size_t)nsplit * (size_t)n * (size_t)ncols > ws_elems)
-        throw Error(3, "dense step workspace too small");
-      const dim3 g2((unsigned)round_up(tiles * nsplit, kXcds));
-      hipLaunchKernelGGL((dense_step_kernel<T, kDensePartial>), g2, dim3(kThreads), 0, st, n, A, lda,
-                         X, Z, out, ld, ncols, p0, p1, p2, R, kap, ntn, nsplit, ws);
-      RCG_HIP(hipGetLastError());
-      const dim3 g3((unsigned)((n * ncols + kThreads - 1) / kThreads));
+    // as many columns at a time as the workspace holds the partial products of: all
+    // of them where dense_ws_elems was reserved; fewer change no bits
+    const int64_t room = (int64_t)(ws_elems / ((size_t)nsplit * (size_t)n));
+    const int cper = room >= ncols ? ncols : (int)(room / 4 * 4);
+    if (ws && nsplit > 1 && cper > 0 && mode != kChebSrc) {
+      for (int c0 = 0; c0 < ncols; c0 += cper) {
+        const int c1 = std::min(ncols, c0 + cper);
+        const int tn = (c1 - c0 + DenseCfg<T>::BN - 1) / DenseCfg<T>::BN;
+        const int64_t wgs = dense_tiles(n, c1 - c0, DenseCfg<T>::BM, DenseCfg<T>::BN) * nsplit;
+        hipLaunchKernelGGL((dense_step_kernel<T, kDensePartial>),
+                           dim3((unsigned)round_up(wgs, kXcds)), dim3(kThreads), 0, st, n, A, lda,
+                           X, Z, out, ld, c1, p0, p1, p2, R, kap, c0, tn, nsplit, ws);
+        RCG_HIP(hipGetLastError());
+        const dim3 g3((unsigned)((n * (c1 - c0) + kThreads - 1) / kThreads));
 #define RCG_COMBINE(M)                                                                           \
   hipLaunchKernelGGL(dense_combine_kernel<M>, g3, dim3(kThreads), 0, st, n, ws, nsplit, X, Z, out, \
-                     ld, ncols, p0, p1, p2)
-      switch (mode) {
-        case kApply: RCG_COMBINE(kApply); break;
-        case kApplyBeta: RCG_COMBINE(kApplyBeta); break;
-        case kChebFirst: RCG_COMBINE(kChebFirst); break;
-        case kCheb: RCG_COMBINE(kCheb); break;
-        default: throw Error(1, "unknown dense step mode");
-      }
+                     ld, c0, c1, p0, p1, p2)
+        switch (mode) {
+          case kApply: RCG_COMBINE(kApply); break;
+          case kApplyBeta: RCG_COMBINE(kApplyBeta); break;
+          case kChebFirst: RCG_COMBINE(kChebFirst); break;
+          case kCheb: RCG_COMBINE(kCheb); break;
+          default: throw Error(1, "unknown dense step mode");
+        }
 #undef RCG_COMBINE
-      RCG_HIP(hipGetLastError());
+        RCG_HIP(hipGetLastError());
+      }
       return;
     }
   }
   const dim3 grid((unsigned)round_up(tiles, kXcds));
 #define RCG_DENSE(M)                                                                           \
   hipLaunchKernelGGL((dense_step_kernel<T, M>), grid, dim3(kThreads), 0, st, n, A, lda, X, Z, out, \
-                     ld, ncols, p0, p1, p2, R, kap, ntn, 1, (T*)nullptr)
+                     ld, ncols, p0, p1, p2, R, kap, 0, ntn, 1, (T*)nullptr)
   switch (mode) {
     case kApply: RCG_DENSE(kApply); break;
     case kApplyBeta: RCG_DENSE(kApplyBeta); break;

@@ -3302,13 +3302,23 @@ int rcg_operator_apply(rcg_operator op, rcg_block in, rcg_block out, double alph
       e.attach(nullptr, nullptr, nullptr, real_ld(in), nullptr, 0);
       e.cb_apply_ab(static_cast<const double*>(in->d()), static_cast<double*>(out->d()), cols,
                     alpha, beta);
-    } else if (op->is_dense())
+    } else if (op->is_dense()) {
+      // workspace for the product's K splits, so that it has the bits of every other
+      // product with the operator; where there is no room for it, unsplit
+      DevBuf ws(op->ctx->stream);
+      size_t elems = rcg::dense_ws_elems(op->n, (int)cols);
+      try {
+        ws.ensure(sizeof(double) * elems);
+      } catch (const Error& e) {
+        if (e.code != RCG_ERR_ALLOC) throw;
+        elems = 0;
+      }
       rcg::launch_dense_step<double>(op->n, op->dense, op->lda, static_cast<const double*>(in->d()),
                                      nullptr, static_cast<double*>(out->d()), (int)in->ld,
                                      (int)cols, alpha, beta, 0.0,
                                      beta == 0.0 ? rcg::kStepApply : rcg::kStepApplyBeta, nullptr,
-                                     nullptr, op->ctx->stream);
-    else {
+                                     nullptr, op->ctx->stream, ws.as<double>(), elems);
+    } else {
       Engine e(op->ctx, op, op->n);
       e.attach(nullptr, nullptr, nullptr, real_ld(in), nullptr, 0);
       rcg::launch_csr_apply<double>(op->n, op->rowptr, op->col, op->val,
@@ -3583,9 +3593,10 @@ int rcg_residuals_noalloc(rcg_operator op, rcg_block V, rcg_block W, int64_t cou
     }
     const double* v = static_cast<const double*>(V->d());
     double* w = static_cast<double*>(W->d());
-    if (op->is_dense())
+    if (op->is_dense())  // the region of the residuals' partials, and what follows it
       rcg::launch_dense_step<double>(op->n, op->dense, op->lda, v, nullptr, w, (int)ld, (int)count,
-                                     1.0, 0.0, 0.0, rcg::kStepApply, nullptr, nullptr, st);
+                                     1.0, 0.0, 0.0, rcg::kStepApply, nullptr, nullptr, st, ws,
+                                     kNoAllocDoubles - (size_t)(3 * rc));
     else
       rcg::launch_csr_apply<double>(op->n, op->rowptr, op->col, op->val, v, w, (int)ld, (int)rc,
                                     1.0, 0.0, st, nullptr, cw == 2);

@@ -70,6 +70,46 @@ def test_padded_rows(n, lda, cols):
     capi.check(capi.lib().rcg_operator_destroy(h))
 
 
+def dense_products(rcg, A, X):
+    """A X by every entry point that forms it, as their W or out block."""
+    n, cols = X.shape
+    op = rcg.DenseOperator(A)
+    bv = rcg.Block.from_host(X)
+    th, res = np.zeros(cols), np.zeros(cols)
+    H = np.zeros((cols, cols), order="F")
+    out = {}
+    for name in ("residuals", "noalloc", "project", "apply"):
+        bw = rcg.Block(n, cols)
+        p = [a.ctypes.data_as(C.c_void_p) for a in (th, res, H)]
+        L = capi.lib()
+        capi.check({"residuals": lambda: L.rcg_residuals(op.h, bv.h, bw.h, cols, p[0], p[1]),
+                    "noalloc": lambda: L.rcg_residuals_noalloc(op.h, bv.h, bw.h, cols, p[0], p[1]),
+                    "project": lambda: L.rcg_project(op.h, bv.h, bw.h, cols, p[2]),
+                    "apply": lambda: L.rcg_operator_apply(op.h, bv.h, bw.h, 1.0, 0.0, cols)}[name]())
+        out[name] = (bw.download(), res.copy() if name in ("residuals", "noalloc") else None)
+    return out
+
+
+@pytest.mark.parametrize("n,cols", [(255, 5), (700, 48), (1500, 130), (2900, 64), (4099, 130)])
+def test_one_product_everywhere(n, cols):
+    """A dense FP64 product has the same bits from every entry point, also where the fixed
+    workspace of the no-allocation residuals holds the partial sums of some columns only,
+    and the no-allocation residuals are those of the others."""
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    print(f"case: dense products n={n} cols={cols}", flush=True)
+    g = np.random.default_rng(n)
+    A = g.uniform(-1, 1, (n, n))
+    A = np.asfortranarray((A + A.T) / n)
+    X = g.uniform(-1, 1, (n, cols))
+    got = dense_products(rcg, A, X)
+    W, res = got["residuals"]
+    scale = np.max(np.abs(A).sum(axis=1))
+    assert np.max(np.abs(W - A @ X)) <= 2 * (n + 32) * 2.0**-53 * scale
+    for name, (w, r) in got.items():
+        assert np.array_equal(w, W), name
+        assert r is None or np.max(np.abs(r - res) / res) <= 1e-14
+
+
 @pytest.mark.parametrize("n,cols,pad", [(3000, 64, 4), (2049, 64, 4)])
 def test_products_do_not_depend_on_earlier_calls(n, cols, pad):
     """The same call before and after one that needs more workspace: the same bits."""

@@ -59,6 +59,8 @@ struct TilePlan {
   int64_t ntile = 0;
 };
 struct TileShape {
+  int64_t gx = 0, gy = 0, gz = 0;
+  int rows = 0;  // of a full tile
   int ex = 0, ey = 0, ez = 0;  // rows of a tile along x, y, z
   int sy = 0, sz = 0;          // tiles of a bundle along y, z
   int smax = 0;
@@ -67,9 +69,8 @@ struct TileShape {
 };
 TileShape tile_shape(int64_t gx, int64_t gy, int64_t gz);
 // *bad (zero before) is set if the operator does not fit the tiles.
-void launch_tile_plan(const TileShape& t, int64_t n, const int* rowptr, const int* col, int64_t gx,
-                      int64_t gy, int64_t gz, int* srow, int* pstart, unsigned char* lidx, int* bad,
-                      hipStream_t st);
+void launch_tile_plan(const TileShape& t, int64_t n, const int* rowptr, const int* col, int* srow,
+                      int* pstart, unsigned char* lidx, int* bad, hipStream_t st);
 // Order in which the CSR kernels visit row blocks.  The rows computed and
 // their arithmetic do not depend on it; it only changes which rows are in
 // flight together (cache locality).  order == nullptr: contiguous blocks.

@@ -980,15 +980,34 @@ class Engine {
   // 220 / 117; 128^3 x 32 534 / 349, x 64 825 / 676; 1024^2 x 64 377 / 317; equal
   // at 12 columns.  Below, the blocks stay in L2 and there are too few tiles to
   // fill the chip: 32^3 x 64 15.4 / 17.4, 44^3 x 32 17.1 / 18.0, x 45 31.6 / 26.5.
-  bool tiles_fp64(int64_t b) const { return n_ * b >= (int64_t)3 << 20 && b >= 16; }
-
-  // The tile plan of an operator on a grid, as a schedule of its own.
-  void build_tiles() {
+  bool tiles_fp64(int64_t b) const {
+    return n_ * b >= (int64_t)3 << 20 && b >= 16 && tiles_filled(b);
+  }
+  // Whether the grid fills its tiles by two thirds: a tile costs the same however
+  // many rows it holds.  FP64 us per step, row blocks / tiles: 512 x 512 x 2 x 16 (a
+  // half) 68 / 97; 5 x 5 x 4000 x 64 (0.39) 39 / 56; 9 x 12000 x 48 (0.56) 36 / 39; 5 x
+  // 200 x 200 x 32 (0.62) 40.7 / 42.0; 10 x 10 x 1000 x 48 (0.69) 36.7 / 36.5; 300 x 300
+  // x 3 x 32 (0.75) 68 / 51; 12 x 10000 x 64 (0.75) 44 / 41; 33^3 x 96 (0.77) 31 / 29.
+  // And the tile kernel's launch must stay below 2^32 threads.
+  bool tiles_filled(int64_t b) const {
+    rcg::TileShape sh;
+    return tile_shape_of(&sh) && 3 * n_ >= 2 * sh.rows * sh.ntile &&
+           sh.ntile * ((b + 63) / 64) < (int64_t)1 << 23;
+  }
+  // The tiles of the operator's grid (the hint, else the one its rows show).
+  bool tile_shape_of(rcg::TileShape* sh) const {
     const bool hint = op_->gx > 0;
     const int64_t gx = hint ? op_->gx : op_->dx, gy = hint ? op_->gy : op_->dy,
                   gz = hint ? op_->gz : op_->dz;
-    if (!op_->own_pattern || gx < 4 || gy < 4 || gx * gy * gz != n_) return;
-    const rcg::TileShape sh = rcg::tile_shape(gx, gy, gz);
+    if (!op_->own_pattern || gx < 4 || gy < 4 || gx * gy * gz != n_) return false;
+    *sh = rcg::tile_shape(gx, gy, gz);
+    return true;
+  }
+
+  // The tile plan of an operator on a grid, as a schedule of its own.
+  void build_tiles() {
+    rcg::TileShape sh;
+    if (!tile_shape_of(&sh)) return;
     auto c = std::make_unique<SchedCand>();
     c->name = "lds-tiles";
     try {
@@ -1003,8 +1022,8 @@ class Engine {
     bad.ensure(sizeof(int));
     int hbad = 0;
     RCG_HIP(hipMemcpyAsync(bad.p, &hbad, sizeof(int), hipMemcpyHostToDevice, st_));
-    rcg::launch_tile_plan(sh, n_, op_->rowptr, op_->col, gx, gy, gz, c->srow.as<int>(),
-                          c->pstart.as<int>(), c->lidx.as<unsigned char>(), bad.as<int>(), st_);
+    rcg::launch_tile_plan(sh, n_, op_->rowptr, op_->col, c->srow.as<int>(), c->pstart.as<int>(),
+                          c->lidx.as<unsigned char>(), bad.as<int>(), st_);
     RCG_HIP(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st_));
     sync();
     if (hbad) return;
@@ -1055,7 +1074,7 @@ class Engine {
       // 48 81 / 48 us, x 64 83 / 56; 128^3 x 64 488 / 445, x 24 268 / 294; 1024^2 x
       // 96 345 / 387), where the best order of row blocks is seldom far from
       // "rows" and "tile16x16": those three are timed, else every order
-      const bool tiles = fp32 && b >= 24 && have_tiles();
+      const bool tiles = fp32 && b >= 24 && tiles_filled(b) && have_tiles();
       std::vector<int> cands;
       for (int k = 0; k < (int)op_->scheds.size(); ++k)
         if (!tiles || op_->scheds[k]->name == "rows" || op_->scheds[k]->name == "tile16x16")

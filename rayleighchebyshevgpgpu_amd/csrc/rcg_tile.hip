@@ -408,6 +408,10 @@ void tile_launch(const TilePlan& t, const T* val, const T* X, const T* Z, T* out
 
 TileShape tile_shape(int64_t gx, int64_t gy, int64_t gz) {
   TileShape t;
+  t.gx = gx;
+  t.gy = gy;
+  t.gz = gz;
+  t.rows = kTileRows;
   if (gz > 1) {
     t.ex = t.ey = t.ez = 4;
     t.sy = 32;
@@ -427,12 +431,11 @@ TileShape tile_shape(int64_t gx, int64_t gy, int64_t gz) {
   return t;
 }
 
-void launch_tile_plan(const TileShape& t, int64_t n, const int* rowptr, const int* col, int64_t gx,
-                      int64_t gy, int64_t gz, int* srow, int* pstart, unsigned char* lidx, int* bad,
-                      hipStream_t st) {
-  if (gx * gy * gz != n || t.ntile > INT32_MAX) throw Error(1, "tile plan: grid does not match");
+void launch_tile_plan(const TileShape& t, int64_t n, const int* rowptr, const int* col, int* srow,
+                      int* pstart, unsigned char* lidx, int* bad, hipStream_t st) {
+  if (t.gx * t.gy * t.gz != n || t.ntile > INT32_MAX) throw Error(1, "tile plan: grid does not match");
   hipLaunchKernelGGL(tile_plan_kernel, dim3((unsigned)t.ntile), dim3(256), 0, st, n, rowptr, col,
-                     (int)gx, (int)gy, (int)gz, t.ex, t.ey, t.ez, t.sy, t.sz, t.smax, srow, pstart,
+                     (int)t.gx, (int)t.gy, (int)t.gz, t.ex, t.ey, t.ez, t.sy, t.sz, t.smax, srow, pstart,
                      lidx, bad);
   RCG_HIP(hipGetLastError());
 }

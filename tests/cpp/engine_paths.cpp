@@ -103,4 +103,17 @@ int test_ortho_project(rcg_operator op, rcg_block prime, rcg_block V, rcg_block 
     e.sync();
   });
 }
+
+// An FP64 filter of degree m: the schedule it took, its column panel and launches.
+int test_filter_route(rcg_operator op, rcg_block X, rcg_block T, int64_t cols, int64_t m,
+                      char* sched, int64_t cap, int64_t* panel, int64_t* launches) {
+  return guarded([&] {
+    Piece pc(X, T, op);
+    pc.eng.filter(cols, (long)m, 1, 14.0, 1.0);
+    std::snprintf(sched, (size_t)cap, "%s", pc.eng.last_sched().c_str());
+    *panel = pc.eng.last_panel();
+    *launches = pc.eng.step_launches();
+    pc.settle(X, cols);
+  });
+}
 }

@@ -36,6 +36,7 @@ def eng():
     L = capi.lib()
     vp, i64 = C.c_void_p, C.c_int64
     L.test_ortho_project.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, vp]
+    L.test_filter_route.argtypes = [vp, vp, vp, i64, i64, vp, i64, vp, vp]
     yield L
     gc.collect()
     if solver._default_ctx is not None:
@@ -134,3 +135,29 @@ def test_zero_column_is_refused(eng, shape, b, cx, primed):
     with pytest.raises(capi.RcgError, match="CholQR breakdown after a shifted pass"):
         ortho_project(eng, A, block("zero", A.n, b, cx, 1),
                       block("near", A.n, b, cx, 2) if primed else None)
+
+
+def filter_route(L, A, grid, cols, m):
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    op = rcg.CsrOperator(A, grid=grid)
+    bx, bt = rcg.Block(A.n, cols), rcg.Block(A.n, cols)
+    bx.randomize(0, cols, 1, 0)
+    name, panel, launches = C.create_string_buffer(64), C.c_int64(), C.c_int64()
+    capi.check(L.test_filter_route(op.h, bx.h, bt.h, cols, m, name, 64, C.byref(panel),
+                                   C.byref(launches)))
+    return name.value.decode(), panel.value, launches.value
+
+
+@pytest.mark.parametrize("grid,cols,tiles", [
+    ((300, 300, 3), 32, True), ((45, 45, 45), 48, True), ((12, 10000, 1), 32, True),
+    ((256, 256, 2), 32, False), ((5, 5, 8000), 32, False), ((5, 40000, 1), 32, False),
+    ((9, 9, 1500), 32, False)])
+def test_thin_grids_keep_row_blocks(eng, grid, cols, tiles):
+    """FP64 steps go over LDS tiles where the grid fills them by two thirds."""
+    print(f"case: route on {grid} x {cols}", flush=True)
+    n = int(np.prod(grid))
+    pot = ops.anderson_potential(n, 3.0, n)
+    A = ops.laplacian_2d(*grid[:2], "dirichlet", pot) if grid[2] == 1 else \
+        ops.laplacian_3d(*grid, "dirichlet", pot)
+    name, _, _ = filter_route(eng, A, grid, cols, 3)
+    assert (name == "lds-tiles") == tiles, name

@@ -159,6 +159,9 @@ template <typename T>
 bool launch_tile_step(const TilePlan& t, int mode, const T* val, const T* X, const T* Z, T* out,
                       int ld, int ncols, T p0, T p1, T p2, const T* R, const T* kap, bool cx,
                       const MixedArgs& ms, hipStream_t st);
+// Its kernel launches.
+template <typename T>
+int tile_step_launches(int ncols);
 
 // Mixed-precision filter.  The FP64 filter output s*X_m of X_0 = v is split
 // per column as X_j = u_j(theta_c) v + E_j, u_j the scalar recurrence of the

@@ -1046,13 +1046,17 @@ class Engine {
   rcg_operator_s::Tuned tuned_for(int64_t b, int kind, Launch&& launch) {
     std::lock_guard<std::mutex> lk(op_->lazy_mu);
     build_schedules();
-    const int64_t key = (int64_t)kind * 1000000000000LL + ld_ * 100000 + b;
+    // a forced column panel is one of the row orders: tiles have none
+    const char* env_panel = std::getenv("RCG_FILTER_PANEL");
+    const int panel = env_panel ? std::atoi(env_panel) : 0;
+    const int64_t key =
+        (int64_t)(kind + (panel > 0 ? 4 : 0)) * 1000000000000LL + ld_ * 100000 + b;
     auto it = op_->tuned.find(key);
     rcg_operator_s::Tuned t{(int)b, 0};
     const bool fp32 = kind == 1 || kind == 3;
     if (it != op_->tuned.end()) {
       t = it->second;
-    } else if (!fp32 && tiles_fp64(b) && have_tiles()) {
+    } else if (!fp32 && panel <= 0 && tiles_fp64(b) && have_tiles()) {
       t.sched = kTileSched;
     } else if (n_ * b >= (int64_t)1 << 22) {  // only large blocks are worth timing
       hipEvent_t e0, e1;
@@ -1074,7 +1078,7 @@ class Engine {
       // 48 81 / 48 us, x 64 83 / 56; 128^3 x 64 488 / 445, x 24 268 / 294; 1024^2 x
       // 96 345 / 387), where the best order of row blocks is seldom far from
       // "rows" and "tile16x16": those three are timed, else every order
-      const bool tiles = fp32 && b >= 24 && tiles_filled(b) && have_tiles();
+      const bool tiles = fp32 && panel <= 0 && b >= 24 && tiles_filled(b) && have_tiles();
       std::vector<int> cands;
       for (int k = 0; k < (int)op_->scheds.size(); ++k)
         if (!tiles || op_->scheds[k]->name == "rows" || op_->scheds[k]->name == "tile16x16")
@@ -1099,10 +1103,7 @@ class Engine {
       (void)hipEventDestroy(e1);
       op_->tuned[key] = t;
     }
-    if (const char* env = std::getenv("RCG_FILTER_PANEL")) {
-      const int v = std::atoi(env);
-      if (v > 0) t.panel = v;
-    }
+    if (panel > 0) t.panel = panel;
     if (const char* env = std::getenv("RCG_FILTER_SCHED")) {
       int pick = -1;
       for (int sidx = 0; sidx < (int)op_->scheds.size(); ++sidx)
@@ -1113,7 +1114,14 @@ class Engine {
                                                  "operator: ") + env);
       t.sched = pick;
     }
+    if (t.sched == kTileSched) t.panel = (int)b;
     return t;
+  }
+  // Kernel launches of one step on rb real columns.
+  template <typename T>
+  static long launches_per_step(const rcg_operator_s::Tuned& t, int64_t rb) {
+    if (t.sched == kTileSched) return rcg::tile_step_launches<T>((int)rb);
+    return t.panel > 0 ? (rb + t.panel - 1) / t.panel : 0;
   }
   // b counts real columns here.  Timing writes Chebyshev steps into T, so an
   // engine without a T block (the piecewise residual / apply entry points)
@@ -1210,7 +1218,7 @@ class Engine {
     const rcg::CsrSched* sc = &sched_at(tn.sched).sc;
     last_panel_ = tn.panel;
     last_sched_ = sched_at(tn.sched).name;
-    step_begin(rep * m * ((rb + tn.panel - 1) / tn.panel),
+    step_begin(rep * m * launches_per_step<double>(tn, rb),
                double(rep) * (csr + 2.0 * blk + double(m - 1) * (csr + 3.0 * blk)));
     for (long r = 0; r < rep; ++r) {
       double* X0 = V();
@@ -1506,7 +1514,7 @@ class Engine {
       }
       float* X0 = E_[0];
       float* X1 = E_[1];
-      step_begin((m - 1) * ((rb + tn.panel - 1) / tn.panel), double(m - 1) * (csr + 4.0 * blk));
+      step_begin((m - 1) * launches_per_step<float>(tn, rb), double(m - 1) * (csr + 4.0 * blk));
       for (long j = 2; j <= m; ++j) {
         if (dn) {
           rcg::launch_dense_step<float>(n_, val32, op_->lda, X1, X0, X0, (int)ld_, (int)rb, g1f,

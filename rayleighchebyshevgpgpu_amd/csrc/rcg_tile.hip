@@ -386,12 +386,13 @@ void tile_launch_nv(const TilePlan& t, const T* val, const T* X, const T* Z, T* 
 // Panels of 64 elements: FP64 rows of 512 bytes (two workgroups of 80 KB per
 // CU), FP32 rows of 256.  FP64 columns left over, up to 32, take a launch with
 // half the lanes' work and half the LDS.
+inline int fp64_full_panels(int ncols) { return ncols / 64 + (ncols % 64 > 32 ? 1 : 0); }
 template <typename T, bool CX, int MODE>
 void tile_launch(const TilePlan& t, const T* val, const T* X, const T* Z, T* out, int ld, int ncols,
                  T p0, T p1, T p2, const T* R, const T* kap, const MixedArgs& ms, hipStream_t st) {
   if constexpr (std::is_same<T, double>::value) {
     const int rest = ncols % 64;
-    const int full = ncols / 64 + (rest > 32 ? 1 : 0);
+    const int full = fp64_full_panels(ncols);
     if (full > 0)
       tile_launch_nv<T, CX, MODE, 2>(t, val, X, Z, out, ld, ncols, 0, full, p0, p1, p2, R, kap, ms,
                                      st);
@@ -468,6 +469,15 @@ bool launch_tile_step(const TilePlan& t, int mode, const T* val, const T* X, con
   }
 #undef RCG_TILE_MODE
 }
+template <typename T>
+int tile_step_launches(int ncols) {
+  if constexpr (std::is_same<T, float>::value) return ncols > 0 ? 1 : 0;
+  const int full = fp64_full_panels(ncols);
+  return (full > 0 ? 1 : 0) + (ncols > 64 * full ? 1 : 0);
+}
+template int tile_step_launches<double>(int);
+template int tile_step_launches<float>(int);
+
 template bool launch_tile_step<double>(const TilePlan&, int, const double*, const double*,
                                        const double*, double*, int, int, double, double, double,
                                        const double*, const double*, bool, const MixedArgs&,

@@ -161,3 +161,25 @@ def test_thin_grids_keep_row_blocks(eng, grid, cols, tiles):
         ops.laplacian_3d(*grid, "dirichlet", pot)
     name, _, _ = filter_route(eng, A, grid, cols, 3)
     assert (name == "lds-tiles") == tiles, name
+
+
+@pytest.mark.parametrize("env,want", [
+    ({}, ("lds-tiles", 96, 6)),  # 64 columns and 32 more, a launch each
+    ({"RCG_FILTER_PANEL": "32"}, (None, 32, 9)),
+    ({"RCG_FILTER_PANEL": "96"}, (None, 96, 3)),
+    ({"RCG_FILTER_PANEL": "0"}, ("lds-tiles", 96, 6)),
+    ({"RCG_FILTER_SCHED": "lds-tiles", "RCG_FILTER_PANEL": "32"}, ("lds-tiles", 96, 6)),
+    ({"RCG_FILTER_SCHED": "rows", "RCG_FILTER_PANEL": "16"}, ("rows", 16, 18))])
+def test_forced_panel(eng, monkeypatch, env, want):
+    """RCG_FILTER_PANEL forces the column panel of the row orders, also where tiles (which
+    have no panels) would be taken, and the launches are counted as they are made."""
+    for k in ("RCG_FILTER_SCHED", "RCG_FILTER_PANEL"):
+        monkeypatch.delenv(k, raising=False)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    grid = (40, 40, 44)
+    n = int(np.prod(grid))
+    A = ops.laplacian_3d(*grid, "periodic", ops.anderson_potential(n, 3.0, n))
+    name, panel, launches = filter_route(eng, A, grid, 96, 3)
+    assert name == want[0] if want[0] else name != "lds-tiles"
+    assert (panel, launches) == want[1:]

@@ -188,7 +188,9 @@ struct DevBuf {
     if (b == 0) return;
     if (pooled) {
       RCG_HIP(hipGetDevice(&dev));
-      p = MemPool::get().alloc(dev, b, &bytes);
+      size_t cap = 0;
+      p = MemPool::get().alloc(dev, b, &cap);
+      bytes = cap;  // only now: a failed allocation leaves an empty buffer
       return;
     }
     hipError_t e = hipMalloc(&p, b);
@@ -234,7 +236,9 @@ struct HostBuf {
     if (b <= bytes) return;
     release();
     if (pooled) {
-      p = MemPool::get().alloc(-1, b, &bytes);
+      size_t cap = 0;
+      p = MemPool::get().alloc(-1, b, &cap);
+      bytes = cap;
       return;
     }
     RCG_HIP(hipHostMalloc(&p, b, hipHostMallocDefault));

@@ -36,6 +36,7 @@ def eng():
     L = capi.lib()
     vp, i64 = C.c_void_p, C.c_int64
     L.test_ortho_project.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, vp]
+    L.test_alloc_limit.argtypes = [i64]
     L.test_filter_route.argtypes = [vp, vp, vp, i64, i64, vp, i64, vp, vp]
     yield L
     gc.collect()
@@ -183,3 +184,32 @@ def test_forced_panel(eng, monkeypatch, env, want):
     name, panel, launches = filter_route(eng, A, grid, 96, 3)
     assert name == want[0] if want[0] else name != "lds-tiles"
     assert (panel, launches) == want[1:]
+
+
+@pytest.fixture
+def scarce(eng):
+    """limit(bytes): device allocations above that fail until the test ends."""
+    def limit(nbytes):
+        capi.check(eng.rcg_memory_trim())
+        eng.test_alloc_limit(nbytes)
+    yield limit
+    eng.test_alloc_limit(-1)
+
+
+def test_calls_after_a_failed_allocation(eng, scarce):
+    """A context whose workspace could not be had is as good as new once there is memory."""
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    ctx = rcg.Context(0)
+    g = np.random.default_rng(3)
+    X = g.standard_normal((5000, 24))
+    bx, bt = rcg.Block.from_host(X, ctx), rcg.Block(5000, 24, ctx=ctx)
+    scarce(0)
+    for _ in range(2):
+        with pytest.raises(capi.RcgError) as e:
+            capi.check(eng.rcg_orthonormalize(bx.h, bt.h, 24))
+        assert e.value.code == 3
+    eng.test_alloc_limit(-1)
+    capi.check(eng.rcg_orthonormalize(bx.h, bt.h, 24))
+    Q = bx.download()
+    assert np.max(np.abs(Q.T @ Q - np.eye(24))) <= 256 * 24 * U
+    assert np.max(np.abs(Q @ (Q.T @ X) - X)) <= 2 * 256 * 24 * U * np.linalg.norm(X, axis=0).max()

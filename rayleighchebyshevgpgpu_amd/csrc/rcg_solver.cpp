@@ -2988,10 +2988,36 @@ class HostPipe {
   int k_ = 0;
 };
 
+// Host column-major <-> device row-interleaved through the host, which changes the
+// layout of some rows at a time: needs no device memory.
+void transfer_rows(rcg_block b, char* host, size_t stride, int64_t cols, bool up) {
+  const size_t es = rcg::dtype_size(b->dtype), row = es * (size_t)b->ld;
+  const int64_t per = std::min<int64_t>(b->n, (int64_t)((size_t(4) << 20) / row) + 1);
+  std::vector<char> buf(row * (size_t)per);
+  hipStream_t st = b->ctx->stream;
+  for (int64_t r0 = 0; r0 < b->n; r0 += per) {
+    const int64_t nr = std::min(per, b->n - r0);
+    char* dev = static_cast<char*>(b->d()) + row * (size_t)r0;
+    RCG_HIP(hipMemcpyAsync(buf.data(), dev, row * (size_t)nr, hipMemcpyDeviceToHost, st));
+    RCG_HIP(hipStreamSynchronize(st));
+    for (int64_t c = 0; c < cols; ++c)
+      for (int64_t i = 0; i < nr; ++i) {
+        char* x = host + stride * (size_t)c + es * (size_t)(r0 + i);
+        char* y = &buf[row * (size_t)i + es * (size_t)c];
+        std::memcpy(up ? y : x, up ? x : y, es);
+      }
+    if (!up) continue;
+    RCG_HIP(hipMemcpyAsync(dev, buf.data(), row * (size_t)nr, hipMemcpyHostToDevice, st));
+    RCG_HIP(hipStreamSynchronize(st));
+  }
+}
+
 // Host column-major <-> device row-interleaved, the layout changed on the
 // device (65280 x 32 FP64, up and down: 12.5 ms with the change on the host).  At
-// most kTransferBytes of columns are in the device's column-major buffer at once.
-constexpr size_t kTransferBytes = size_t(256) << 20;
+// most kTransferBytes are in the device's column-major buffer at once: whole
+// columns, or some rows of one.  With less device memory the buffer is smaller, and
+// with none the rows go through the host.
+constexpr size_t kTransferBytes = size_t(256) << 20, kTransferLeast = size_t(512) << 10;
 void transfer(rcg_block b, void* host, int64_t ld_host, int64_t cols, bool up) {
   need(b && host, "NULL argument");
   need(cols >= 0 && cols <= b->cols, "column count exceeds the block");
@@ -3003,23 +3029,29 @@ void transfer(rcg_block b, void* host, int64_t ld_host, int64_t cols, bool up) {
   hipStream_t st = b->ctx->stream;
   const size_t col = es * (size_t)b->n, stride = es * (size_t)ld_host;
   DevBuf tmp(st);
-  int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(cols, (int64_t)(kTransferBytes / col)));
-  try {
-    tmp.ensure(col * (size_t)chunk);
-  } catch (const Error& e) {
-    if (e.code != RCG_ERR_ALLOC || chunk == 1) throw;
-    chunk = 1;  // no room for many columns: one at a time
-    tmp.ensure(col);
+  std::unique_ptr<HostPipe> pipe;
+  size_t room = std::min(kTransferBytes, col * (size_t)cols);
+  while (!pipe) {
+    try {
+      tmp.ensure(room);
+      pipe = std::make_unique<HostPipe>(st, room);
+    } catch (const Error& e) {
+      if (e.code != RCG_ERR_ALLOC) throw;
+      if (room <= kTransferLeast || tmp.p) return transfer_rows(b, h, stride, cols, up);
+      room /= 2;
+    }
   }
-  HostPipe pipe(st, col * (size_t)chunk);
-  for (int64_t c0 = 0; c0 < cols; c0 += chunk) {
-    const int64_t nc = std::min(chunk, cols - c0);
-    char* hc = h + stride * (size_t)c0;
-    if (up) pipe.up(tmp.as<char>(), hc, col, stride, nc);
-    rcg::launch_block_layout(b->n, (int)nc, (int)es, static_cast<char*>(b->d()) + es * (size_t)c0,
-                             b->ld, tmp.p, b->n, !up, st);
-    if (!up) pipe.down(tmp.as<char>(), hc, col, stride, nc);
-  }
+  const int64_t cper = std::max<int64_t>(1, std::min<int64_t>(cols, (int64_t)(room / col)));
+  const int64_t rper = std::min<int64_t>(b->n, (int64_t)(room / es));
+  for (int64_t c0 = 0; c0 < cols; c0 += cper)
+    for (int64_t r0 = 0; r0 < b->n; r0 += rper) {
+      const int64_t nc = std::min(cper, cols - c0), nr = std::min(rper, b->n - r0);
+      char* hc = h + stride * (size_t)c0 + es * (size_t)r0;
+      char* dev = static_cast<char*>(b->d()) + es * ((size_t)r0 * (size_t)b->ld + (size_t)c0);
+      if (up) pipe->up(tmp.as<char>(), hc, es * (size_t)nr, stride, nc);
+      rcg::launch_block_layout(nr, (int)nc, (int)es, dev, b->ld, tmp.p, nr, !up, st);
+      if (!up) pipe->down(tmp.as<char>(), hc, es * (size_t)nr, stride, nc);
+    }
   RCG_HIP(hipStreamSynchronize(st));
 }
 }  // namespace

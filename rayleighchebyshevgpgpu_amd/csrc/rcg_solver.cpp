@@ -932,6 +932,7 @@ class Engine {
   // together.
   void build_schedules() {
     if (!op_->scheds.empty()) return;
+    std::vector<std::unique_ptr<SchedCand>> made;  // all of them or, without memory, none
     auto add = [&](const std::string& name, std::vector<int> order, int64_t rows, int remap) {
       auto c = std::make_unique<SchedCand>();
       c->name = name;
@@ -943,7 +944,7 @@ class Engine {
         c->sc.rows_per_blk = rows;
         c->sc.nblk = (int64_t)order.size();
       }
-      op_->scheds.push_back(std::move(c));
+      made.push_back(std::move(c));
     };
     add("rows", {}, 0, 1);
     add("rows-noremap", {}, 0, 0);
@@ -963,6 +964,7 @@ class Engine {
               order, gx, remap);
       }
     }
+    op_->scheds = std::move(made);
   }
 
   // Index of the tile schedule beside those of `scheds`.
@@ -972,10 +974,7 @@ class Engine {
   }
   // Whether the operator has tiles; made on the first call (lazy_mu held).
   bool have_tiles() {
-    if (!op_->tiles_tried) {
-      build_tiles();
-      op_->tiles_tried = true;
-    }
+    if (!op_->tiles_tried) op_->tiles_tried = build_tiles();
     return op_->tiles != nullptr;
   }
   // FP64 steps of b real columns go over LDS tiles from 3 * 2^20 block entries
@@ -1008,29 +1007,30 @@ class Engine {
     return true;
   }
 
-  // The tile plan of an operator on a grid, as a schedule of its own.
-  void build_tiles() {
+  // The tile plan of an operator on a grid, as a schedule of its own.  False: not
+  // settled, for want of memory (the row orders need none).
+  bool build_tiles() {
     rcg::TileShape sh;
-    if (!tile_shape_of(&sh)) return;
+    if (!tile_shape_of(&sh)) return true;
     auto c = std::make_unique<SchedCand>();
     c->name = "lds-tiles";
+    DevBuf bad(st_);
     try {
       c->srow.ensure(sizeof(int) * sh.srow);
       c->pstart.ensure(sizeof(int) * sh.pstart);
       c->lidx.ensure(sh.lidx);
+      bad.ensure(sizeof(int));
     } catch (const Error& e) {
       if (e.code != RCG_ERR_ALLOC) throw;
-      return;  // no memory for a plan: the general step needs none
+      return false;
     }
-    DevBuf bad(st_);
-    bad.ensure(sizeof(int));
     int hbad = 0;
     RCG_HIP(hipMemcpyAsync(bad.p, &hbad, sizeof(int), hipMemcpyHostToDevice, st_));
     rcg::launch_tile_plan(sh, n_, op_->rowptr, op_->col, c->srow.as<int>(), c->pstart.as<int>(),
                           c->lidx.as<unsigned char>(), bad.as<int>(), st_);
     RCG_HIP(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st_));
     sync();
-    if (hbad) return;
+    if (hbad) return true;
     c->plan.srow = c->srow.as<int>();
     c->plan.pstart = c->pstart.as<int>();
     c->plan.lidx = c->lidx.as<unsigned char>();
@@ -1038,6 +1038,7 @@ class Engine {
     c->plan.ntile = sh.ntile;
     c->sc.tile = &c->plan;
     op_->tiles = std::move(c);
+    return true;
   }
 
   // Filter shape for b columns: LDS tiles where they are known to win, else the
@@ -1127,17 +1128,8 @@ class Engine {
     if (t.sched == kTileSched) return rcg::tile_step_launches<T>((int)rb);
     return t.panel > 0 ? (rb + t.panel - 1) / t.panel : 0;
   }
-  // b counts real columns here.  Timing writes Chebyshev steps into T, so an
-  // engine without a T block (the piecewise residual / apply entry points)
-  // never tunes: it uses the cached choice or the contiguous default.
+  // b counts real columns here.
   rcg_operator_s::Tuned tuned_for(int64_t b) {
-    if (!T() || !V()) {
-      std::lock_guard<std::mutex> lk(op_->lazy_mu);
-      build_schedules();
-      if (tiles_fp64(b) && have_tiles()) return rcg_operator_s::Tuned{(int)b, kTileSched};
-      auto it = op_->tuned.find((int64_t)(cx_ ? 2 : 0) * 1000000000000LL + ld_ * 100000 + b);
-      return it != op_->tuned.end() ? it->second : rcg_operator_s::Tuned{(int)b, 0};
-    }
     return tuned_for(b, cx_ ? 2 : 0, [&](int panel, const rcg::CsrSched* sc) {
       rcg::launch_cheb_step<double>(n_, op_->rowptr, op_->col, op_->val, V(), T(), T(), (int)ld_,
                                     (int)b, 0.0, 1.0, 0.0, false, st_, panel, sc, cx_);
@@ -1164,9 +1156,21 @@ class Engine {
     rcg::launch_copy_cols<double>(n_, src, (int)lds, (int)(cw_ * s0), dst, (int)ldd,
                                   (int)(cw_ * d0), (int)(cw_ * cnt), st_);
   }
+  // The order of a product of b real columns (null: the default).  Timing writes
+  // Chebyshev steps into T, so an engine without a T block (the piecewise residual /
+  // apply entry points) never tunes: it takes tiles or the cached choice.
   const rcg::CsrSched* sched_for(int64_t b) {
     if (!op_ || batcher_ || n_ * b < (int64_t)3 << 20) return nullptr;
-    return &sched_at(tuned_for(b).sched).sc;
+    try {
+      if (T() && V()) return &sched_at(tuned_for(b).sched).sc;
+      std::lock_guard<std::mutex> lk(op_->lazy_mu);
+      if (tiles_fp64(b) && have_tiles()) return &op_->tiles->sc;
+      auto it = op_->tuned.find((int64_t)(cx_ ? 2 : 0) * 1000000000000LL + ld_ * 100000 + b);
+      return it != op_->tuned.end() ? &sched_at(it->second.sched).sc : nullptr;
+    } catch (const Error& e) {
+      if (e.code != RCG_ERR_ALLOC) throw;
+      return nullptr;  // no memory for an order: the default one needs none
+    }
   }
 
   // Whether the filter of b columns runs in one launch (rcg_small.hip).  The

@@ -237,3 +237,28 @@ def test_transfers_with_little_memory(scarce, n, cols, part, pad, limit, dtype):
     back = np.full((n + pad, cols), 7, dtype=dtype, order="F")
     capi.check(capi.lib().rcg_block_download(b.h, back.ctypes.data_as(C.c_void_p), n + pad, cols))
     assert np.array_equal(back[:n], want) and np.all(back[n:] == 7)
+
+
+@pytest.mark.parametrize("kind", ["grid", "dense"])
+def test_products_with_little_memory(eng, scarce, kind):
+    """rcg_operator_apply needs no device memory of its own: with none left it takes the
+    default row order, or the unsplit dense product."""
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    print(f"case: apply with no memory, {kind}", flush=True)
+    g = np.random.default_rng(5)
+    if kind == "grid":
+        grid = (64, 64, 64)
+        A = ops.laplacian_3d(*grid, "periodic", ops.anderson_potential(64**3, 3.0, 1))
+        op, S, cols, n = rcg.CsrOperator(A, grid=grid), A.to_scipy(), 20, 64**3
+    else:
+        n, cols = 900, 24
+        S = g.uniform(-1, 1, (n, n))
+        S = (S + S.T) / n
+        op = rcg.DenseOperator(S)
+    X = g.uniform(-1, 1, (n, cols))
+    bx, by = rcg.Block.from_host(X), rcg.Block(n, cols)
+    scarce(0)
+    capi.check(eng.rcg_operator_apply(op.h, bx.h, by.h, 1.0, 0.0, cols))
+    eng.test_alloc_limit(-1)
+    scale = np.max(np.abs(S).sum(axis=1))
+    assert np.max(np.abs(by.download() - S @ X)) <= 2 * (min(n, 1000) + 32) * U * scale

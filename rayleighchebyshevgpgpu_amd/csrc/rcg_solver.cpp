@@ -316,6 +316,14 @@ struct SchedCand {
   rcg::TilePlan plan;
 };
 
+// The step over LDS tiles of one pattern on one grid, shared by the operators of
+// the pattern (22 bytes a row).  Made when first wanted; only read from then on.
+struct TileSet {
+  std::mutex mu;
+  bool tried = false;
+  std::unique_ptr<SchedCand> cand;  // null: not made, or the rows do not fit tiles
+};
+
 struct rcg_operator_s {
   rcg_context_s* ctx = nullptr;
   int64_t n = 0, nnz = 0;
@@ -331,8 +339,7 @@ struct rcg_operator_s {
   // plan made from them stays true.  Arrays in the caller's memory may change.
   bool own_pattern = false;
   std::vector<std::unique_ptr<SchedCand>> scheds;
-  std::unique_ptr<SchedCand> tiles;  // the step over LDS tiles (made when first wanted)
-  bool tiles_tried = false;
+  std::shared_ptr<TileSet> tiles = std::make_shared<TileSet>();
   struct Tuned {
     int panel;
     int sched;
@@ -970,12 +977,14 @@ class Engine {
   // Index of the tile schedule beside those of `scheds`.
   static constexpr int kTileSched = -2;
   const SchedCand& sched_at(int k) const {
-    return k == kTileSched ? *op_->tiles : *op_->scheds[k];
+    return k == kTileSched ? *op_->tiles->cand : *op_->scheds[k];
   }
   // Whether the operator has tiles; made on the first call (lazy_mu held).
   bool have_tiles() {
-    if (!op_->tiles_tried) op_->tiles_tried = build_tiles();
-    return op_->tiles != nullptr;
+    TileSet& t = *op_->tiles;
+    std::lock_guard<std::mutex> lk(t.mu);
+    if (!t.tried) t.tried = build_tiles(t);
+    return t.cand != nullptr;
   }
   // FP64 steps of b real columns go over LDS tiles from 3 * 2^20 block entries
   // (24 MB: past L2) and 16 columns.  Measured on periodic 3-D and 2-D grids (us
@@ -1009,7 +1018,7 @@ class Engine {
 
   // The tile plan of an operator on a grid, as a schedule of its own.  False: not
   // settled, for want of memory (the row orders need none).
-  bool build_tiles() {
+  bool build_tiles(TileSet& t) {
     rcg::TileShape sh;
     if (!tile_shape_of(&sh)) return true;
     auto c = std::make_unique<SchedCand>();
@@ -1037,7 +1046,7 @@ class Engine {
     c->plan.smax = sh.smax;
     c->plan.ntile = sh.ntile;
     c->sc.tile = &c->plan;
-    op_->tiles = std::move(c);
+    t.cand = std::move(c);
     return true;
   }
 
@@ -1164,7 +1173,7 @@ class Engine {
     try {
       if (T() && V()) return &sched_at(tuned_for(b).sched).sc;
       std::lock_guard<std::mutex> lk(op_->lazy_mu);
-      if (tiles_fp64(b) && have_tiles()) return &op_->tiles->sc;
+      if (tiles_fp64(b) && have_tiles()) return &op_->tiles->cand->sc;
       auto it = op_->tuned.find((int64_t)(cx_ ? 2 : 0) * 1000000000000LL + ld_ * 100000 + b);
       return it != op_->tuned.end() ? &sched_at(it->second.sched).sc : nullptr;
     } catch (const Error& e) {
@@ -3274,6 +3283,7 @@ int rcg_operator_csr_share(rcg_operator base, const void* val, int mem, rcg_oper
     o->dy = base->dy;
     o->dz = base->dz;
     o->own_pattern = base->own_pattern;
+    o->tiles = base->tiles;
     if (mem == RCG_MEM_DEVICE) {
       o->val = static_cast<const double*>(val);
     } else {
@@ -3342,8 +3352,7 @@ int rcg_operator_set_grid(rcg_operator op, int64_t nx, int64_t ny, int64_t nz) {
     op->gy = ny;
     op->gz = nz;
     op->scheds.clear();
-    op->tiles.reset();
-    op->tiles_tried = false;
+    op->tiles = std::make_shared<TileSet>();
     op->tuned.clear();
   });
 }

@@ -138,9 +138,9 @@ def test_zero_column_is_refused(eng, shape, b, cx, primed):
                       block("near", A.n, b, cx, 2) if primed else None)
 
 
-def filter_route(L, A, grid, cols, m):
+def filter_route(L, A, grid, cols, m, op=None):
     from rayleighchebyshevgpgpu_amd import solver as rcg
-    op = rcg.CsrOperator(A, grid=grid)
+    op = op or rcg.CsrOperator(A, grid=grid)
     bx, bt = rcg.Block(A.n, cols), rcg.Block(A.n, cols)
     bx.randomize(0, cols, 1, 0)
     name, panel, launches = C.create_string_buffer(64), C.c_int64(), C.c_int64()
@@ -262,3 +262,38 @@ def test_products_with_little_memory(eng, scarce, kind):
     eng.test_alloc_limit(-1)
     scale = np.max(np.abs(S).sum(axis=1))
     assert np.max(np.abs(by.download() - S @ X)) <= 2 * (min(n, 1000) + 32) * U * scale
+
+
+def test_operators_of_one_pattern_share_their_tiles(eng, scarce):
+    """The tile plan holds the pattern only: operators that share a pattern and a grid share
+    it, whichever of them made it."""
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    grid = (40, 40, 44)
+    n = int(np.prod(grid))
+    A = ops.laplacian_3d(*grid, "periodic", ops.anderson_potential(n, 3.0, n))
+    base = rcg.CsrOperator(A, grid=grid)
+    first, second = base.share(2.0 * A.val), base.share(A.val)
+    assert filter_route(eng, A, None, 96, 3, first)[0] == "lds-tiles"
+    bx, bt = rcg.Block(n, 96), rcg.Block(n, 96)
+    bx.randomize(0, 96, 1, 0)
+    X = bx.download()
+    scarce(0)
+    name = C.create_string_buffer(64)
+    k, m = C.c_int64(), C.c_int64()
+    for op in (second, base):
+        capi.check(eng.test_filter_route(op.h, bx.h, bt.h, 96, 2, name, 64, C.byref(k), C.byref(m)))
+        assert name.value == b"lds-tiles"
+    eng.test_alloc_limit(-1)
+    # a grid of its own ends it
+    capi.check(eng.rcg_operator_set_grid(second.h, n, 1, 1))
+    assert filter_route(eng, A, None, 96, 2, second)[0] != "lds-tiles"
+    assert filter_route(eng, A, None, 96, 2, first)[0] == "lds-tiles"
+    # the filter is the operator's own: the second and the base have one value array's content
+    os.environ["RCG_FILTER_SCHED"] = "rows"
+    try:
+        by = rcg.Block.from_host(X)
+        for op in (second, base):
+            capi.check(eng.test_filter_route(op.h, by.h, bt.h, 96, 2, name, 64, C.byref(k), C.byref(m)))
+    finally:
+        del os.environ["RCG_FILTER_SCHED"]
+    assert np.array_equal(bx.download(), by.download())

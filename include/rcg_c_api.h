@@ -288,7 +288,8 @@ typedef struct rcg_solve_result {
   int64_t lanczos_iters;     /* getSpectralBoundsIterCount */
   double min_est, max_est;   /* getMinEigValueEst / getMaxEigValueEst */
   double guard;              /* getGuardEigenvalue */
-  int64_t count_ortho, count_apply, count_eig; /* getCountData */
+  int64_t count_ortho, count_apply, count_eig; /* getCountData: as the reference counts
+                                its steps, whether or not one is fused with another here */
   double final_maxres, final_maxdiff, final_maxgap; /* getFinalData */
   int64_t trace_len;
   uint64_t rng_counter;
@@ -302,8 +303,11 @@ typedef struct rcg_solve_result {
                                 deflation; t_rr: the projection with its CholQR passes,
                                 the small eigensolve, rotation, residuals and the final
                                 refinement */
-  double t_filter_device;    /* seconds between such marks around the Chebyshev step
-                                launches (FP64 steps, or the FP32 correction steps) */
+  double t_filter_device;    /* seconds around the Chebyshev step launches (FP64 steps, or
+                                the FP32 correction steps): between events, but for
+                                FP64 steps of blocks below 2^20 entries from the
+                                host's clock where the stream is empty, their launch
+                                included */
   double filter_bytes;       /* algorithmic bytes of those steps: CSR + 3 block passes
                                 (FP64) or CSR(FP32 values) + 4 FP32 block passes */
   int64_t filter_panel;      /* autotuned column-panel width of the filter step */

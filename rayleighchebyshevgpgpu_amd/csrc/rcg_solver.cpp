@@ -2462,7 +2462,9 @@ class Solver {
         // after an iteration's residuals the stream is empty
         const bool idle = innerLoopCount > 0 && residual_count_ > 0;
         clock_.mark(PhaseClock::kFilter, idle);
-        if (idle) eng_.set_idle();
+        // steps of large blocks are timed from an event all the same, without the
+        // host's work before their launch; it would cost a small solve 3-5 us a time
+        if (idle && op_->n * eng_.cw() * subspaceSize < (int64_t)1 << 20) eng_.set_idle();
         if (!completedBasis) {
           if (mixed)
             eng_.filter_mixed(subspaceSize, starDegree, rep, starBound, shift, fTheta, fRitz);

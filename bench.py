@@ -17,9 +17,10 @@ is timed the same way
 and reported under "mixed", with its speed-up and its largest eigenvalue
 difference from the FP64 solve.
 
-roofline: the fused Chebyshev step kernel (csr_tile_kernel, mode kCheb),
-timed with HIP events on the library's stream around every filter
-application inside the timed solves; its algorithmic bytes per launch are
+roofline: the fused Chebyshev step kernel (csr_tile_kernel on grids that fill
+its tiles, else csr_block_kernel; mode kCheb), timed with HIP events on the
+library's stream around the steps of every filter application inside the timed
+solves (t_filter_device of the C interface); its algorithmic bytes per launch are
 nnz*(8+4) + 4*(n+1) + 3*n*b*8 (CSR values+columns+row pointers, one read of
 X_{j-1}, one read of X_{j-2}, one write of X_j).
 
@@ -631,14 +632,12 @@ def main():
         t_dev = sum(x[2].t_filter_device for x in results)
         alg_bytes = sum(x[2].filter_bytes for x in results)
         achieved = alg_bytes / t_dev / 1e9 if t_dev > 0 else 0.0
-        if WL["complex"]:
-            kern = ("complex64 correction step (csr_tile_kernel or csr_block_kernel, kChebSrc)"
-                    if precision == "mixed" else
-                    "csr_tile_kernel<double,true,kCheb> (fused complex128 Chebyshev step)")
-        else:
-            kern = ("csr_tile_kernel<float,false,kChebSrc> (FP32 correction step)"
-                    if precision == "mixed" else
-                    "csr_tile_kernel<double,false,kCheb> (fused FP64 Chebyshev step)")
+        # the schedule follows the operator and the columns; either kernel does the step
+        step = {(False, False): "fused FP64 Chebyshev step", (False, True): "FP32 correction step",
+                (True, False): "fused complex128 Chebyshev step",
+                (True, True): "complex64 correction step"}[bool(WL["complex"]), precision == "mixed"]
+        kern = step + (" (csr_tile_kernel over LDS tiles or csr_block_kernel by rows, "
+                       + ("kChebSrc)" if precision == "mixed" else "kCheb)"))
         roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                     "traffic": traffic_from_profiles(precision), "kernel": kern,

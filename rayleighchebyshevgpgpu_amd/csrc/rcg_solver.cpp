@@ -1847,6 +1847,9 @@ class Engine {
     const char* unp = std::getenv("RCG_GRAM_UNPAIRED");
     const bool apart = unp && unp[0] == '1';
     const bool large = n_ * rb >= (int64_t(1) << 22);
+    // a caller's apply may call the library on this context: nothing stays in the
+    // results over it
+    const bool keeps = !op_->is_callback();
     std::vector<S> G(b * b), H1(b * b), R, Ri;
     std::vector<double> scale(b, 1.0);
     bool one_pass = one_pass_;
@@ -1866,7 +1869,7 @@ class Engine {
     }
     // the first pass's factor on the device, without a trip to the host; taken
     // back (the old block is in T) if the Gram matrix turns out not to factor
-    bool on_device = !one_pass && !cx_ && !large && rcg::chol_fits(n_, (int)b);
+    bool on_device = keeps && !one_pass && !cx_ && !large && rcg::chol_fits(n_, (int)b);
     if (on_device) {
       gram_ready_ = false;
       rcg::launch_gram_chol(n_, V(), (int)ld_, (int)b, dmatA(), dres() + inv2_at(), ws(),
@@ -1884,7 +1887,7 @@ class Engine {
       }
     }
     if (!one_pass && !on_device) {
-      if (!cholqr_pass<S>(b, true, large && !apart)) {
+      if (!cholqr_pass<S>(b, true, large && !apart && keeps)) {
         cholqr_pass<S>(b, true);
         cholqr_pass<S>(b, false);
         project<S>(b, H);

@@ -129,7 +129,7 @@ void csr_launch_cx(int64_t n, const int* rp, const int* ci, const T* va, const T
   RCG_CSR_CASE(128, 32, 4)
   RCG_CSR_CASE(256, 32, 8)
 #undef RCG_CSR_CASE
-  throw Error(6, "CSR block kernels support at most 256 16-byte column vectors per row");
+  throw Error(1, "CSR launch without a width class");
 }
 
 // ncols counts real columns (2 per complex column when cx).
@@ -138,6 +138,9 @@ void csr_launch(int64_t n, const int* rp, const int* ci, const T* va, const T* X
                 T* out, int ld, int ncols, T p0, T p1, T p2, hipStream_t st, const CsrSched* sc,
                 const T* R = nullptr, const T* kap = nullptr, bool cx = false,
                 const MixedArgs& ms = MixedArgs{}) {
+  // the limit of the row kernels' width classes, whichever kernel runs
+  if ((ncols + V16<T>::W - 1) / V16<T>::W > 256)
+    throw Error(6, "CSR block kernels support at most 256 16-byte column vectors per row");
   if (sc && sc->tile &&
       launch_tile_step<T>(*sc->tile, MODE, va, X, Z, out, ld, ncols, p0, p1, p2, R, kap, cx, ms,
                           st))

@@ -1187,6 +1187,7 @@ class Engine {
   // looked up once; it steers the choice only, any row length is computed.
   bool small_filter(int64_t b, long m, bool fp64) {
     if (batcher_ || !op_->is_csr() || n_ > rcg::kSmallFilterRows) return false;
+    if (cw_ * b > 512) return false;  // the general kernel refuses them
     // a forced panel or order asks for the general kernel
     if (std::getenv("RCG_FILTER_PANEL") || std::getenv("RCG_FILTER_SCHED")) return false;
     std::lock_guard<std::mutex> lk(op_->lazy_mu);

@@ -297,3 +297,28 @@ def test_operators_of_one_pattern_share_their_tiles(eng, scarce):
     finally:
         del os.environ["RCG_FILTER_SCHED"]
     assert np.array_equal(bx.download(), by.download())
+
+
+@pytest.mark.parametrize("kind,cols", [("tiles", 520), ("small", 520), ("small complex", 260)])
+def test_width_limit_on_every_route(eng, kind, cols):
+    """CSR operators take at most 256 16-byte column vectors (512 FP64 columns) whichever
+    kernel would run, and refuse more without touching the block."""
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    print(f"case: width limit, {kind}", flush=True)
+    grid = (20, 20, 20) if kind == "tiles" else (10, 10, 10)
+    A = ops.hofstadter_2d(32, phi=1.0 / 8, W=1.0) if "complex" in kind else \
+        ops.laplacian_3d(*grid, "dirichlet", ops.anderson_potential(int(np.prod(grid)), 3.0, 1))
+    op = rcg.CsrOperator(A)
+    dt = np.complex128 if A.is_complex else np.float64
+    bx, bt = rcg.Block(A.n, cols, dtype=dt), rcg.Block(A.n, cols, dtype=dt)
+    bx.randomize(0, cols, 1, 0)
+    X = bx.download()
+    th, rz = np.zeros(cols), np.ones(cols, dtype=np.int32)
+    assert eng.rcg_cheb_filter(op.h, bx.h, bt.h, cols, 8, 1, 14.0, 1.0) == 6
+    assert eng.rcg_cheb_filter_mixed(op.h, bx.h, bt.h, cols, 8, 1, 14.0, 1.0,
+                                     th.ctypes.data_as(C.c_void_p), rz.ctypes.data_as(C.c_void_p)) == 6
+    assert eng.rcg_operator_apply(op.h, bx.h, bt.h, 1.0, 0.0, cols) == 6
+    assert np.array_equal(bx.download(), X)
+    most = 256 if A.is_complex else 512
+    capi.check(eng.rcg_cheb_filter(op.h, bx.h, bt.h, most, 8, 1, 14.0, 1.0))
+    assert np.array_equal(bx.download()[:, most:], X[:, most:])

@@ -222,10 +222,10 @@ struct SmallFilter {
   T g1 = T(0), g2 = T(0), s_end = T(0);
 };
 // Whether the one-launch filter takes an operator of this size, with cols
-// columns (complex ones count once; c128: the FP64 filter of a complex one)
-// and degree m.
-bool small_filter_fits(int64_t n, int64_t nnz, int64_t max_row, int64_t cols, int64_t m,
-                       bool c128);
+// columns (complex ones count once) and degree m.  fp32: the mixed filter's
+// correction steps.
+bool small_filter_fits(int64_t n, int64_t nnz, int64_t max_row, int64_t cols, int64_t m, bool cx,
+                       bool fp32);
 template <typename T>
 void launch_small_filter(const SmallFilter<T>& a, int cols, int64_t max_row, bool cx,
                          hipStream_t st);

@@ -224,9 +224,26 @@ void small_launch(const SmallFilter<T>& a, int cols, hipStream_t st) {
 // kernel's and time per step, 12-48 columns, FP64 (us, one launch against
 // general): n = 1056 +7 and 0.5 against 5; n = 3904 +15 and 1.2 against 5; 16^3
 // +18 and 1.6 against 5.
-bool small_filter_fits(int64_t n, int64_t nnz, int64_t max_row, int64_t cols, int64_t m,
-                       bool c128) {
-  return n <= (c128 ? kSmallFilterRows / 2 : kSmallFilterRows) && m >= 2 + n / 1024 &&
+//
+// The mixed filter's correction steps begin one step later, after a launch that the
+// FP64 filter does not have, and the general kernel's FP32 steps are the shorter, so
+// they need more steps, most of all where two workgroups share a compute unit.  The
+// whole call, one launch over general, 96-256 and 272-512 columns: n = 1000 m = 2
+// 1.00-1.11 and 1.10-1.17, m = 4 0.70-0.79 and 0.86-0.91; n = 2025 m = 3 1.00 and
+// 1.21-1.23, m = 6 0.77-0.80 and 0.92-0.96; n = 3904 m = 5 1.03-1.08 and 1.29-1.35,
+// m = 6 0.96-1.00 and 1.22-1.27, m = 17 0.57-0.62 and 0.79-0.83; 4096 rows of 1 to 12
+// nonzeros m = 6 0.95-0.98 and 1.24-1.31, m = 17 0.65-0.70 and 0.95-1.03; complex, 64-256
+// columns, n = 1600 m = 3 0.95-1.08, m = 5 0.81-0.94; n = 3136 m = 5 1.05-1.13, m = 8
+// 0.85-0.93.
+bool small_filter_fits(int64_t n, int64_t nnz, int64_t max_row, int64_t cols, int64_t m, bool cx,
+                       bool fp32) {
+  int64_t least = 2 + n / 1024;
+  if (fp32) {
+    if (cx) least = 3 + n / 700;
+    else if (cols <= 256) least = 3 + n / 1200;
+    else least = n <= 2048 ? 3 + n / 650 : 4 + n / 250;
+  }
+  return n <= (cx && !fp32 ? kSmallFilterRows / 2 : kSmallFilterRows) && m >= least &&
          nnz <= 7 * n && max_row <= 12 && cols <= 512;
 }
 

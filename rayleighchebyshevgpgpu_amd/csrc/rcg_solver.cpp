@@ -1199,7 +1199,7 @@ class Engine {
       for (int64_t i = 0; i < n_; ++i)
         op_->max_row = std::max<int64_t>(op_->max_row, rp[i + 1] - rp[i]);
     }
-    return rcg::small_filter_fits(n_, op_->nnz, op_->max_row, b, m, cx_ && fp64);
+    return rcg::small_filter_fits(n_, op_->nnz, op_->max_row, b, m, cx_, !fp64);
   }
 
   // V <- P_m(A')^rep V over b columns (LanczosCpolyOperatorLM.h:192-304):

@@ -116,4 +116,9 @@ int test_filter_route(rcg_operator op, rcg_block X, rcg_block T, int64_t cols, i
     pc.settle(X, cols);
   });
 }
+
+int test_small_filter_fits(int64_t n, int64_t nnz, int64_t max_row, int64_t cols, int64_t m,
+                           int cx, int fp32) {
+  return rcg::small_filter_fits(n, nnz, max_row, cols, m, cx != 0, fp32 != 0) ? 1 : 0;
+}
 }

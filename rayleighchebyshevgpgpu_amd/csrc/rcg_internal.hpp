@@ -288,6 +288,11 @@ void launch_tall_gemm_cross(int64_t n, const double* X, int ldx, int bx, const d
                             int by, double alpha, const double* Z, double* out, int ldo, double* G,
                             double* ws, size_t ws_elems, hipStream_t st);
 
+// Whether the forms with a Gram matrix are faster than the product and a Gram
+// launch of its own.
+bool tall_gram_pays(int64_t n, int by);
+bool tall_cross_pays(int64_t n, int bx, int by);
+
 // sums[c] = sum_i |X[i,c]|^2, c < nc.
 template <typename T>
 void launch_col_sumsq(int64_t n, const T* X, int ld, int nc, double* sums, double* ws,

@@ -2722,6 +2722,31 @@ void launch_tall_resid(int64_t n, const double* V, const double* W, int ld, int 
   reduce_to(ws, nblk, 2 * nc, sums, st);
 }
 
+// A partial per workgroup of 64-row tiles costs the fused forms more than a partial per
+// 256 rows costs the Gram launch, until there are more tiles than workgroups; from
+// 2^19 rows the Gram launch streams faster than the narrow product's two workgroups
+// per CU.  us, fused / apart, out^T out of 8, 32 and 64 columns: n = 4000 9.6 / 11.1,
+// 15.1 / 15.9, 23.3 / 27.2; 14000 11.1 / 11.8, 17.4 / 17.6, 27.4 / 29.7; 17576 12.2 / 12.5,
+// 21.1 / 18.9, 38.2 / 31.8; 50000 15.8 / 15.0, 30.5 / 24.7, 52.1 / 42.0; 70000 17.1 /
+// 17.9, 34.9 / 34.5, 57.5 / 62.2; 200000 24.8 / 32.8, 54.6 / 58.5, 85.9 / 114; 2^20 70 / 62,
+// 194 / 193, 292 / 363.
+bool tall_gram_pays(int64_t n, int by) {
+  return n <= 14336 || (n >= 70000 && (n < (int64_t(1) << 19) || by > 40));
+}
+// X^T out reads X again, but the Gram launch it replaces reads X and out, and
+// multiplies max(bx, by)^2 tiles.  us, fused / apart, 24 x 24, 64 x 16, 20 x 64 and 64 x
+// 64 (bx x by): n = 4000 15.7 / 18.3, 14.3 / 31.1, 20.9 / 35.5, 29.3 / 35.9; 20000 23.7 /
+// 21.3, 21.7 / 33.5, 34.3 / 39.9, 56.6 / 41.0; 50000 30.6 / 26.7, 27.7 / 38.8, 46.5 / 51.0,
+// 75.8 / 54.2; 65536 30.7 / 34.8, 28.0 / 44.2, 48.1 / 60.4, 76.6 / 65.4; 75000 37.7 / 40.5,
+// 31.4 / 66.5, 54.3 / 84.3, 87.8 / 88.3; 2^20 x (16 x 24) 209 / 237, (64 x 64) 492 / 575.
+// With bx above 32 and 33-48 columns it spills: 48 x 48 at 75000 82.8 / 62.5.
+bool tall_cross_pays(int64_t n, int bx, int by) {
+  if (n <= 14336) return true;
+  if (bx > 32 && by > 32 && by <= 48) return false;
+  if (n >= 65536) return !(bx > 32 && by > 48) || n >= 70000;
+  return std::max(bx, by) > 48 && std::min(bx, by) <= 32;
+}
+
 void launch_tall_gemm_gram(int64_t n, const double* X, int ldx, int bx, const double* C, int ldc,
                            int by, double* out, int ldo, double* G, double* ws, size_t ws_elems,
                            hipStream_t st) {

@@ -1723,8 +1723,9 @@ class Engine {
   }
   template <class S>
   void orthonormalize_t(int64_t b) {
-    const bool clean = cholqr_pass<S>(b, true, true);
-    cholqr_pass<S>(b, true, !clean);
+    const bool gram = rcg::tall_gram_pays(n_, (int)(cw_ * b));
+    const bool clean = cholqr_pass<S>(b, true, gram);
+    cholqr_pass<S>(b, true, gram && !clean);
     if (!clean) cholqr_pass<S>(b, false);
   }
 
@@ -1733,13 +1734,13 @@ class Engine {
   // V -= Y (Y^H V), twice.  The normalisation of the reference is implied by
   // the CholQR that follows in the solve.
   // Up to 64 real columns each, the second pass's Y^H V is formed by the product
-  // of the first (no read of Y and V of its own); with `norms` the second
+  // of the first where that is faster (no read of Y and V of its own); with `norms` the second
   // product also leaves the columns' squared norms in dsums().
   void deflate(int64_t b, int64_t found, bool norms = false) {
     if (found <= 0 || b <= 0) return;
     gram_ready_ = false;
     const int64_t rf = cw_ * found, rb = cw_ * b;
-    const bool cross = rf <= 64 && rb <= 64;
+    const bool cross = rf <= 64 && rb <= 64 && rcg::tall_cross_pays(n_, (int)rf, (int)rb);
     for (int pass = 0; pass < 2; ++pass) {
       if (pass == 0 || !cross)
         rcg::launch_gram<double>(n_, Y_, (int)ldy_, (int)rf, V(), (int)ld_, (int)rb, dmatA(), ws(),
@@ -1851,6 +1852,8 @@ class Engine {
     // a caller's apply may call the library on this context: nothing stays in the
     // results over it
     const bool keeps = !op_->is_callback();
+    // the next Gram matrix comes with the product that writes the block
+    const bool fused = large && !apart && keeps && rcg::tall_gram_pays(n_, (int)rb);
     std::vector<S> G(b * b), H1(b * b), R, Ri;
     std::vector<double> scale(b, 1.0);
     bool one_pass = one_pass_;
@@ -1888,7 +1891,7 @@ class Engine {
       }
     }
     if (!one_pass && !on_device) {
-      if (!cholqr_pass<S>(b, true, large && !apart && keeps)) {
+      if (!cholqr_pass<S>(b, true, fused)) {
         cholqr_pass<S>(b, true);
         cholqr_pass<S>(b, false);
         project<S>(b, H);

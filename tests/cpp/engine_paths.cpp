@@ -117,6 +117,10 @@ int test_filter_route(rcg_operator op, rcg_block X, rcg_block T, int64_t cols, i
   });
 }
 
+int test_tall_gram_pays(int64_t n, int by) { return rcg::tall_gram_pays(n, by) ? 1 : 0; }
+int test_tall_cross_pays(int64_t n, int bx, int by) {
+  return rcg::tall_cross_pays(n, bx, by) ? 1 : 0;
+}
 int test_small_filter_fits(int64_t n, int64_t nnz, int64_t max_row, int64_t cols, int64_t m,
                            int cx, int fp32) {
   return rcg::small_filter_fits(n, nnz, max_row, cols, m, cx != 0, fp32 != 0) ? 1 : 0;

@@ -1,5 +1,6 @@
-"""The rule that sends a small CSR operator's filter to the one-launch kernel, at sizes
-where both kernels were timed (host code only)."""
+"""The rules that choose between two kernels by size, at sizes where both were timed
+(host code only): the filter of a small CSR operator in one launch, and the tall
+products that also form a Gram matrix."""
 import ctypes as C
 import os
 
@@ -22,6 +23,19 @@ LIB = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "libengine
     # never
     (4097, 5, 24, 40, False, False, False), (1000, 13, 24, 40, False, False, False),
     (1000, 7, 513, 40, False, True, False)])
-def test_rule(n, row, cols, m, cx, fp32, want):
+def test_small_filter(n, row, cols, m, cx, fp32, want):
     assert bool(C.CDLL(LIB).test_small_filter_fits(
         *(C.c_int64(v) for v in (n, min(row, 7) * n, row, cols, m)), int(cx), int(fp32))) == want
+
+
+@pytest.mark.parametrize("n,bx,by,gram,cross", [
+    (1000, 64, 64, True, True), (14000, 48, 48, True, True), (17576, 32, 32, False, False),
+    (20000, 64, 16, None, True), (20000, 20, 64, None, True), (50000, 24, 24, False, False),
+    (50000, 64, 64, False, False), (65536, 24, 24, False, True), (65536, 64, 64, False, False),
+    (75000, 64, 64, True, True), (75000, 48, 48, True, False), (200000, 8, 8, True, True),
+    (1 << 20, 24, 24, False, True), (1 << 20, 64, 64, True, True)])
+def test_tall_products(n, bx, by, gram, cross):
+    L = C.CDLL(LIB)
+    if gram is not None:
+        assert bool(L.test_tall_gram_pays(C.c_int64(n), by)) == gram
+    assert bool(L.test_tall_cross_pays(C.c_int64(n), bx, by)) == cross

@@ -995,6 +995,24 @@ class Engine {
   bool tiles_fp64(int64_t b) const {
     return n_ * b >= (int64_t)3 << 20 && b >= 16 && tiles_filled(b);
   }
+  // A product alone does without the step's streams from memory, so the tiles' LDS
+  // reads bind it sooner.  us of rcg_operator_apply, tiles / row blocks, real columns:
+  // 512^2 x 24 41 / 35, x 64 68 / 59, x 80 96 / 108; 1024^2 x 24 122 / 117, x 32 146 / 135, x
+  // 40 197 / 224, x 64 244 / 307, x 96 420 / 666; 1448^2 x 24 238 / 278; 64^3 x 40 68 / 64,
+  // 100^3 x 24 131 / 145, x 36 253 / 231, x 48 264 / 312; 128^3 x 32 305 / 390, x 36 528 /
+  // 475, x 64 605 / 748.  Complex rows do more per LDS read: 512^2 x 48 columns 117 / 86,
+  // x 80 190 / 204; 768^2 x 48 249 / 252; 1024^2 x 36 412 / 375, x 96 790 / 851.
+  bool tiles_apply(int64_t b) const {
+    rcg::TileShape sh;
+    if (!tiles_fp64(b) || !tile_shape_of(&sh)) return false;
+    if (cx_) return b >= 128 && n_ >= (int64_t)1 << 18 && n_ * b >= (int64_t)36 << 20;
+    if (b > 64) return true;
+    if (n_ * b <= (int64_t)1 << 24) return false;
+    if (b > 43) return true;
+    const bool flat = sh.gz == 1;
+    if (b > 32) return flat;  // 3-D: a second panel for few columns
+    return flat ? b >= 20 && n_ >= (int64_t)15 << 17 : n_ >= (int64_t)7 << 16;
+  }
   // Whether the grid fills its tiles by two thirds: a tile costs the same however
   // many rows it holds.  FP64 us per step, row blocks / tiles: 512 x 512 x 2 x 16 (a
   // half) 68 / 97; 5 x 5 x 4000 x 64 (0.39) 39 / 56; 9 x 12000 x 48 (0.56) 36 / 39; 5 x
@@ -1171,9 +1189,13 @@ class Engine {
   const rcg::CsrSched* sched_for(int64_t b) {
     if (!op_ || batcher_ || n_ * b < (int64_t)3 << 20) return nullptr;
     try {
+      if (!std::getenv("RCG_FILTER_SCHED") && !std::getenv("RCG_FILTER_PANEL")) {
+        std::lock_guard<std::mutex> lk(op_->lazy_mu);
+        if (tiles_fp64(b) && have_tiles()) return tiles_apply(b) ? &op_->tiles->cand->sc : nullptr;
+      }
       if (T() && V()) return &sched_at(tuned_for(b).sched).sc;
       std::lock_guard<std::mutex> lk(op_->lazy_mu);
-      if (tiles_fp64(b) && have_tiles()) return &op_->tiles->cand->sc;
+      if (tiles_apply(b) && have_tiles()) return &op_->tiles->cand->sc;
       auto it = op_->tuned.find((int64_t)(cx_ ? 2 : 0) * 1000000000000LL + ld_ * 100000 + b);
       return it != op_->tuned.end() ? &sched_at(it->second.sched).sc : nullptr;
     } catch (const Error& e) {

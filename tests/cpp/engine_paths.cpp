@@ -104,6 +104,16 @@ int test_ortho_project(rcg_operator op, rcg_block prime, rcg_block V, rcg_block 
   });
 }
 
+// Whether a product of cols columns goes over LDS tiles.
+int test_apply_tiles(rcg_operator op, int64_t cols, int32_t* tiles) {
+  return guarded([&] {
+    Engine e(op->ctx, op, op->n);
+    e.attach(nullptr, nullptr, nullptr, e.cw() * block_ld(cols), nullptr, 0);
+    const rcg::CsrSched* sc = e.sched_for(e.cw() * cols);
+    *tiles = sc && sc->tile;
+  });
+}
+
 // An FP64 filter of degree m: the schedule it took, its column panel and launches.
 int test_filter_route(rcg_operator op, rcg_block X, rcg_block T, int64_t cols, int64_t m,
                       char* sched, int64_t cap, int64_t* panel, int64_t* launches) {

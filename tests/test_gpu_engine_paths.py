@@ -37,6 +37,7 @@ def eng():
     vp, i64 = C.c_void_p, C.c_int64
     L.test_ortho_project.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, vp]
     L.test_alloc_limit.argtypes = [i64]
+    L.test_apply_tiles.argtypes = [vp, i64, vp]
     L.test_filter_route.argtypes = [vp, vp, vp, i64, i64, vp, i64, vp, vp]
     yield L
     gc.collect()
@@ -322,3 +323,28 @@ def test_width_limit_on_every_route(eng, kind, cols):
     most = 256 if A.is_complex else 512
     capi.check(eng.rcg_cheb_filter(op.h, bx.h, bt.h, most, 8, 1, 14.0, 1.0))
     assert np.array_equal(bx.download()[:, most:], X[:, most:])
+
+
+@pytest.mark.parametrize("grid,cx,cases", [
+    ((512, 512, 1), False, {24: 0, 64: 0, 72: 1}), ((1024, 1024, 1), False, {24: 0, 36: 1, 64: 1}),
+    ((64, 64, 64), False, {24: 0, 64: 0, 72: 1}), ((100, 100, 100), False, {24: 1, 36: 0, 48: 1}),
+    ((512, 512, 1), True, {48: 0, 64: 0, 80: 1})])
+def test_products_over_tiles_where_faster(eng, grid, cx, cases):
+    """A product takes tiles at fewer sizes than the filter's steps do, and has the same
+    bits either way."""
+    from rayleighchebyshevgpgpu_amd import solver as rcg
+    print(f"case: products on {grid}", flush=True)
+    n = int(np.prod(grid))
+    A = operator(grid, True) if cx else ops.laplacian_2d(*grid[:2]) if grid[2] == 1 else \
+        ops.laplacian_3d(*grid)
+    op, rows = rcg.CsrOperator(A, grid=grid), rcg.CsrOperator(A, grid=(n, 1, 1))
+    for cols, want in cases.items():
+        got = C.c_int32(-1)
+        capi.check(eng.test_apply_tiles(op.h, C.c_int64(cols), C.byref(got)))
+        assert got.value == want, cols
+    dt = np.complex128 if cx else np.float64
+    bx, by, bz = (rcg.Block(n, cols, dtype=dt) for _ in range(3))
+    bx.randomize(0, cols, 1, 0)
+    op.apply(bx, by)
+    rows.apply(bx, bz)
+    assert np.array_equal(by.download(), bz.download())

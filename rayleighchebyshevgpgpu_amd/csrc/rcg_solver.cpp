@@ -1186,12 +1186,16 @@ class Engine {
   // The order of a product of b real columns (null: the default).  Timing writes
   // Chebyshev steps into T, so an engine without a T block (the piecewise residual /
   // apply entry points) never tunes: it takes tiles or the cached choice.
-  const rcg::CsrSched* sched_for(int64_t b) {
+  // start: the product that becomes the mixed filter's start, whose three FP32 blocks
+  // make it a step's kind of kernel (1024^2 x 32, start and two steps: 535 us over
+  // tiles, 615 by rows).
+  const rcg::CsrSched* sched_for(int64_t b, bool start = false) {
     if (!op_ || batcher_ || n_ * b < (int64_t)3 << 20) return nullptr;
     try {
       if (!std::getenv("RCG_FILTER_SCHED") && !std::getenv("RCG_FILTER_PANEL")) {
         std::lock_guard<std::mutex> lk(op_->lazy_mu);
-        if (tiles_fp64(b) && have_tiles()) return tiles_apply(b) ? &op_->tiles->cand->sc : nullptr;
+        if (tiles_fp64(b) && have_tiles())
+          return start || tiles_apply(b) ? &op_->tiles->cand->sc : nullptr;
       }
       if (T() && V()) return &sched_at(tuned_for(b).sched).sc;
       std::lock_guard<std::mutex> lk(op_->lazy_mu);
@@ -1505,7 +1509,7 @@ class Engine {
         ms.g2 = c.g2;
         ms.nc = (int)rb;
         rcg::launch_csr_apply_start(n_, op_->rowptr, op_->col, op_->val, V(), (int)ld_, (int)rb,
-                                    ms, st_, sched_for(rb), cx_);
+                                    ms, st_, sched_for(rb, true), cx_);
       } else {
         apply(V(), W_, b);
         rcg::launch_mixed_start(n_, V(), W_, (int)ld_, (int)rb, dcp, g12, c.g1, c.g2, E_[0],

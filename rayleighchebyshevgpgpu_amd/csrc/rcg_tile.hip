@@ -244,6 +244,10 @@ __global__ __launch_bounds__(kTileThreads) void csr_tile_kernel(
   T av[IT], ai[CX ? IT : 1];
   unsigned long long there[IT];
   T zs[IT][NV][W], rs[kSrc ? IT : 1][NV][W], kv[kSrc ? NV : 1][W];
+  // kChebSrcEnd: V and its columns' factors, in whole 16-byte vectors and ahead of the
+  // gathers, as Z and R
+  constexpr bool kEnd = MODE == kChebSrcEnd;
+  double vs[kEnd ? IT : 1][kEnd ? NV : 1][W], uv[kEnd ? NV : 1][W];
 #pragma unroll
   for (int q = 0; q < IT; ++q) {
     const int k = wave * kWaveRows + q * 4 + (lane >> 4);
@@ -280,12 +284,24 @@ __global__ __launch_bounds__(kTileThreads) void csr_tile_kernel(
 #pragma unroll
       for (int w = 0; w < W; ++w) kv[k][w] = c < ld ? kap[c + w] : T(0);
     }
+    if constexpr (kEnd) {
+#pragma unroll
+      for (int w = 0; w < W; ++w) uv[k][w] = c + w < ncols ? ms.um[c + w] : 0.0;
+    }
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
       const int64_t o = (int64_t)row[q] * ld + c;
       if (row[q] >= 0 && c < ncols) {
         if constexpr (MODE == kCheb || kSrc) VT::ld_stream(Z + o, zs[q][k]);
         if constexpr (kSrc) VT::ld_stream(R + o, rs[q][k]);
+        if constexpr (kEnd) {
+#pragma unroll
+          for (int h = 0; h < W / 2; ++h) {
+            const dvec2 v = reinterpret_cast<const dvec2*>(ms.v_end + o)[h];
+            vs[q][k][2 * h] = v.x;
+            vs[q][k][2 * h + 1] = v.y;
+          }
+        }
       }
     }
   }
@@ -351,9 +367,18 @@ __global__ __launch_bounds__(kTileThreads) void csr_tile_kernel(
       if constexpr (MODE == kChebSrcEnd) {
         // V <- s_end (um V + x), V FP64; x itself is not stored
         double* v = ms.v_end + (int64_t)row[q] * ld + c;
+        double e[W];
 #pragma unroll
-        for (int w = 0; w < W; ++w)
-          if (c + w < ncols) v[w] = ms.s_end * fma(ms.um[c + w], v[w], double(o[w]));
+        for (int w = 0; w < W; ++w) e[w] = ms.s_end * fma(uv[k][w], vs[q][k][w], double(o[w]));
+        if (c + W <= ncols) {
+#pragma unroll
+          for (int h = 0; h < W / 2; ++h)
+            reinterpret_cast<dvec2*>(v)[h] = dvec2{e[2 * h], e[2 * h + 1]};
+        } else {
+#pragma unroll
+          for (int w = 0; w < W; ++w)
+            if (c + w < ncols) v[w] = e[w];
+        }
         continue;
       }
       T* y = out + (int64_t)row[q] * ld + c;

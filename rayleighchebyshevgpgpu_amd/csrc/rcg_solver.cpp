@@ -1733,7 +1733,7 @@ class Engine {
         throw Error(RCG_ERR_NUMERIC, "shifted CholQR breakdown (block is numerically rank deficient)");
     }
     rcg::dense::upper_inverse(R, b, Ri);
-    one_pass_ = clean && rcg::dense::one_pass_enough(rcg::dense::frobenius2(Ri), b);
+    one_pass_ = clean && rcg::dense::one_pass_enough(rcg::dense::upper_frobenius2(Ri, b), b);
     for (int64_t j = 0; j < b; ++j)
       for (int64_t i = 0; i < b; ++i) Ri[i + j * b] *= d[i];
     right_multiply<S>(b, Ri.data(), gram);
@@ -1894,7 +1894,7 @@ class Engine {
       one_pass = rcg::dense::cholesky_upper(G.data(), b, R);
       if (one_pass) {
         rcg::dense::upper_inverse(R, b, Ri);
-        one_pass = rcg::dense::one_pass_enough(rcg::dense::frobenius2(Ri), b);
+        one_pass = rcg::dense::one_pass_enough(rcg::dense::upper_frobenius2(Ri, b), b);
       }
       if (!one_pass) std::fill(scale.begin(), scale.end(), 1.0);
       one_pass_ = one_pass;

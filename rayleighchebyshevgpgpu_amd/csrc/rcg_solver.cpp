@@ -1847,8 +1847,8 @@ class Engine {
   // G = V^H V and H1 = V^H W right after it, so that one wait brings both
   // back.  Below 2^22 block entries both products go in one paired launch
   // (the same values; plain solves of served-size requests 568 -> 586
-  // eigenpairs/s); above, G comes with the product that wrote V (128^3 x 64: no
-  // pass of 0.27 ms of its own).  RCG_GRAM_UNPAIRED=1 runs the two products
+  // eigenpairs/s); above, G comes with the product that wrote V where that pays
+  // (128^3 x 64: no pass of 0.27 ms of its own).  RCG_GRAM_UNPAIRED=1 runs the two products
   // separately, with the paired launch's values.
   void first_projection(int64_t b, int64_t rb, bool apart, bool large) {
     apply(V(), W_, b);

@@ -909,6 +909,7 @@ class Engine {
       RCG_HIP(hipStreamSynchronize(st_));
     }
     coef_busy_ = false;
+    factor_busy_ = false;
   }
 
   // Scratch layout (device `small` and host `pinned` alike):
@@ -1417,6 +1418,9 @@ class Engine {
     rcg::launch_layout(n_, (int)b, cw_, out, ld_, cb_out_.as<double>(), n_, false, st_);
   }
   void call_user(const void* in, void* out, int64_t cols, int64_t ld, double alpha, double beta) {
+    // a factor still on its way from the context's pinned memory, which a library call
+    // inside the caller's apply would write
+    if (factor_busy_) sync();
     const int rc = op_->apply_fn(op_->user, in, out, n_, cols, ld, alpha, beta, (void*)st_);
     if (rc != 0)
       throw Error(RCG_ERR_INVALID, "the operator's apply callback returned " + std::to_string(rc));
@@ -1671,6 +1675,7 @@ class Engine {
     }
     const int64_t rb = cw_ * b;
     RCG_HIP(hipMemcpyAsync(dmatA(), hmatB(), sizeof(double) * rb * rb, hipMemcpyHostToDevice, st_));
+    factor_busy_ = true;
   }
   // V <- V C; the result lands in T, then swaps.  gram: the real Gram matrix of
   // the new V's (real) columns goes to dres() as well (at most 64 columns).
@@ -2284,6 +2289,7 @@ class Engine {
   DevBuf coef_;                       // mixed filter coefficient table
   DevBuf cb_in_, cb_out_;             // column-major blocks of a caller's operator
   bool coef_busy_ = false;            // its upload from hcoef_ may be in flight
+  bool factor_busy_ = false;          // so may a factor's from the context's pinned memory
   HostBuf hcoef_;
   FilterBatcher* batcher_ = nullptr;
   hipEvent_t ev_done_ = nullptr;  // the batcher has run this engine's steps

@@ -25,12 +25,15 @@ def test_library_calls_inside_apply(rcg, stencils, L, k, inc, buf):  # noqa: F81
     assert user
     mine, tmp = rcg.Block(4096, inc + buf), rcg.Block(4096, inc + buf)
     calls = [0]
+    mat = np.asfortranarray(np.full((inc + buf, inc + buf), 0.5) + np.eye(inc + buf))
+    turn = mat.ctypes.data_as(C.c_void_p)
 
     def solve(inner):
         def apply(pin, pout, n, cols, ld, alpha, beta, stream):
             if inner:
                 calls[0] += 1
                 mine.randomize(0, inc + buf, calls[0], 0)
+                capi.check(capi.lib().rcg_rotate(mine.h, tmp.h, inc + buf, turn))
                 capi.check(capi.lib().rcg_orthonormalize(mine.h, tmp.h, inc + buf))
             if stencils.anderson3d_apply(user, pin, pout, n, cols, ld, alpha, beta, stream) != 0:
                 raise RuntimeError("stencil apply failed")
